@@ -1,4 +1,4 @@
-// pk_adjoint.hip -- reverse mode of the fused RK2 hydro sweep (gfx950).
+// pk_adjoint.hip -- reverse mode of the fused RK2 sweep, hydro and MHD (gfx950).
 //
 // For one directional sweep of a periodic block with hydro fluids
 //   U* = floors(U + c1 R(U)),  U' = floors(U + c2 R(U*)),
@@ -15,10 +15,16 @@
 // output cells are lanes 8 .. TS-9: eight cells of halo on each side.
 // Reads wrap periodically along the sweep, so ghost cells are not used.
 #include <hip/hip_runtime.h>
+// the arithmetic of pk_math.hpp and pk_adjoint.hpp without range scaling in
+// divisions and square roots, in a namespace of its own
+#define PK_KNS pk_adj
+#define PK_NORMAL_RANGE 1
 #include "pk_adjoint.hpp"
 #include "pk_adjoint_kernels.hpp"
 
 namespace pk {
+
+using namespace pk_adj;
 
 template <int DIR>
 __device__ __forceinline__ int plane_of_adj(int k)
@@ -54,27 +60,26 @@ __device__ __forceinline__ void faces(const AdjArgs &a, const double (&qm)[P::NV
     }
 }
 
+// One lane's NV values of an LDS array, lane by lane (NV is odd: consecutive
+// lanes fall on different banks): one address per array and lane, the
+// variables at immediate offsets.  With the variables nt apart, nt a run-time
+// value, the MHD kernel held an address register per variable and array and
+// spilled them (395 scratch accesses in its code).
 template <int NV>
-__device__ __forceinline__ void lds_get(const double *A, int nt, int t, double (&x)[NV])
+__device__ __forceinline__ void lds_get(const double *A, int t, double (&x)[NV])
 {
 #pragma unroll
-    for (int v = 0; v < NV; v++) x[v] = A[v * nt + t];
+    for (int v = 0; v < NV; v++) x[v] = A[t * NV + v];
 }
 template <int NV>
-__device__ __forceinline__ void lds_put(double *A, int nt, int t, const double (&x)[NV])
+__device__ __forceinline__ void lds_put(double *A, int t, const double (&x)[NV])
 {
 #pragma unroll
-    for (int v = 0; v < NV; v++) A[v * nt + t] = x[v];
+    for (int v = 0; v < NV; v++) A[t * NV + v] = x[v];
 }
 
-// LDS arrays of NV doubles per lane: five shared neighbour buffers, and for
-// MHD three lane-private ones that hold values live across both flux VJPs
-// (registers for hydro, whose occupancy the larger LDS would halve).
-template <class P>
-constexpr int adj_lds_arrays()
-{
-    return P::MAG ? 8 : 5;
-}
+// LDS arrays of NV doubles per lane of the adjoint tile.
+constexpr int kAdjArrays = 4;
 
 // q_bar of cell k from its face-state adjoints (fpb: left state of k+1/2,
 // fmb: right state of k-1/2) through the limiter: the own-cell part and the
@@ -108,9 +113,9 @@ __device__ __forceinline__ double flux_vjp(const AdjArgs &a, const double *l, co
                                            double *lb, double *rb)
 {
     if constexpr (P::MAG) {
-        return hlld_vjp(l, r, a.gam, a.ch, fb, lb, rb);
+        return hlld_vjp_r(l, r, a.gam, a.rg, a.rg1, a.ch, a.rch, fb, lb, rb);
     } else {
-        hllc_vjp(l, r, a.gam, fb, lb, rb);
+        hllc_vjp_r(l, r, a.gam, a.rg1, fb, lb, rb);
         return 0.0;
     }
 }
@@ -136,21 +141,34 @@ __device__ __forceinline__ void prim_vjp(const AdjArgs &a, const double (&u)[P::
 
 // One tile (bid) of the adjoint sweep; lanes t >= TP*TS of a larger
 // workgroup take part in the barriers only.
+//
+// The tile keeps four LDS arrays of NV doubles per lane (73.7 KB for MHD, so
+// that two workgroups, two waves per SIMD, share a CU):
+//   Q  primitives of the stage in hand, and once those are used an exchange
+//   S  right-face states, then lam' (from the reverse of stage 2 on, own cell)
+//   T  fluxes and other neighbour exchanges
+//   K  R1 of the own cell until the reverse of stage 1, then exchanges
+// An array is rewritten only after a barrier that follows its last read by
+// another lane.  U and the stage-1 primitives are formed again where they are
+// needed instead of being held across the flux VJPs.
+//
+// Bound by FP64 VALU issue (hydro: four waves per SIMD, each issuing 23-24 %
+// of its cycles; MHD: two waves at 31 %, the rest LDS and scratch waits).
+// Against both-sided flux VJPs with IEEE divisions, eight (hydro five) arrays
+// and tiles in launch order: VALU instructions per wave 3143 -> 2136 (hydro)
+// and 9508 -> 5000 (MHD), waves per SIMD 2 -> 4 and 1 -> 2; the list sweeps of
+// 20 Orszag-Tang instances (64^2 .. 256^2) 527 and 633 us -> 297 and 325 us
+// (x, y), a 96^3 hydro rollout with its gradient 7.18 -> 5.3-5.8 ms.  The
+// XCD-aware order is worth 1.4x of that rollout: in launch order the tiles of
+// one cache line of a y or z sweep ran on eight L2s (110e6 busy CU cycles per
+// y sweep against 49e6 along x; in XCD order 50e6).
 template <int DIR, class P, int LIM>
 __device__ __forceinline__ void adjoint_tile(const AdjArgs &a, int bid, double *lds)
 {
     constexpr int NV = P::NV;
     const int nt = blockDim.x;
     const int t = threadIdx.x;
-    double *Q1 = lds, *Q2 = lds + NV * nt, *S1 = lds + 2 * NV * nt, *S2 = lds + 3 * NV * nt, *S3 = lds + 4 * NV * nt;
-    double *K1 = lds + 5 * NV * nt, *K2 = lds + 6 * NV * nt, *K3 = lds + 7 * NV * nt;  // MHD: lane-private
-    // park x in a lane-private LDS array (MHD) until fetch() reloads it
-    auto park = [&](double *K, const double (&x)[NV]) {
-        if constexpr (P::MAG) lds_put<NV>(K, nt, t, x);
-    };
-    auto fetch = [&](double *K, double (&x)[NV]) {
-        if constexpr (P::MAG) lds_get<NV>(K, nt, t, x);
-    };
+    double *Q = lds, *S = lds + NV * nt, *T = lds + 2 * NV * nt, *K = lds + 3 * NV * nt;
 
     constexpr int d1 = (DIR == 0) ? 1 : 0;
     constexpr int d2 = (DIR == 2) ? 1 : 2;
@@ -184,200 +202,197 @@ __device__ __forceinline__ void adjoint_tile(const AdjArgs &a, int bid, double *
     xyz[d2] = c2i;
     const long long idx = (long long)xyz[0] + (long long)a.sy * xyz[1] + (long long)a.sz * xyz[2];
 
-    double U[NV];
+    auto load_u = [&](double (&U)[NV]) {
 #pragma unroll
-    for (int k = 0; k < NV; k++) U[k] = a.u[(long long)plane_of_adj<DIR>(k) * a.sv + idx];
-
-    // ---- forward: stage 1 ----
-    double q[NV];
-    prim<P>(U, a.gam_1, q);
-    lds_put<NV>(Q1, nt, t, q);
-    __syncthreads();
-    double qm[NV], qp[NV], fp[NV], fm[NV], F[NV], R1[NV], Us_pre[NV], Us[NV];
-    lds_get<NV>(Q1, nt, tm, qm);
-    lds_get<NV>(Q1, nt, tp, qp);
-    faces<P, LIM>(a, qm, q, qp, fp, fm);
-    lds_put<NV>(S1, nt, t, fm);
-    __syncthreads();
-    {
-        double r[NV];
-        lds_get<NV>(S1, nt, tp, r);
-        flux<P>(a, fp, r, F);
-        lds_put<NV>(S2, nt, t, F);
-    }
-    __syncthreads();
-    {
-        double Fm[NV];
-        lds_get<NV>(S2, nt, tm, Fm);
+        for (int k = 0; k < NV; k++) U[k] = a.u[(long long)plane_of_adj<DIR>(k) * a.sv + idx];
+    };
+    // the stage-1 state before the floors, from U and R1
+    auto stage1 = [&](const double (&U)[NV], const double (&R1)[NV], double (&W)[NV]) {
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-            R1[v] = Fm[v] - F[v];
             const double un = U[v] + a.c1 * R1[v];
-            Us_pre[v] = (v < 5) ? un + 0.0 : un;
-            Us[v] = Us_pre[v];
+            W[v] = (v < 5) ? un + 0.0 : un;
         }
+    };
+    auto floored = [&](double (&W)[NV]) {
         unsigned fl = 0u;
         double dm = 0.0;
-        floors<P>(Us, a.smalld, a.smallei, a.use_smalld, a.use_smallei, false, fl, dm);
-    }
-    park(K1, R1);
-    park(K2, Us_pre);
-    // ---- forward: stage 2 ----
-    double qs[NV];
-    prim<P>(Us, a.gam_1, qs);
-    lds_put<NV>(Q2, nt, t, qs);
-    __syncthreads();
-    lds_get<NV>(Q2, nt, tm, qm);
-    lds_get<NV>(Q2, nt, tp, qp);
-    faces<P, LIM>(a, qm, qs, qp, fp, fm);
-    lds_put<NV>(S1, nt, t, fm);
-    __syncthreads();
+        floors<P>(W, a.smalld, a.smallei, a.use_smalld, a.use_smallei, false, fl, dm);
+    };
+
+    double fp[NV], r[NV], F[NV];
+    // ---- forward: stage 1 ----
     {
-        double r[NV];
-        lds_get<NV>(S1, nt, tp, r);
-        flux<P>(a, fp, r, F);
-        lds_put<NV>(S2, nt, t, F);
-    }
-    __syncthreads();
-    double lp[NV];  // lam' through the psi damping and the floors of stage 2
-    double dtb = 0.0, chb = 0.0;
-    {
-        double Fm[NV], R2[NV], Up[NV];
-        lds_get<NV>(S2, nt, tm, Fm);
-#pragma unroll
-        for (int v = 0; v < NV; v++) {
-            R2[v] = Fm[v] - F[v];
-            const double un = U[v] + a.c2 * R2[v];
-            Up[v] = (v < 5) ? un + 0.0 : un;
-        }
-        // ---- reverse: stage 2 ----
-#pragma unroll
-        for (int k = 0; k < NV; k++) lp[k] = a.lam_out[(long long)plane_of_adj<DIR>(k) * a.sv + idx];
-        if constexpr (P::MAG) lp[8] = lp[8] * a.psi_fac;
-        floors_vjp<P>(a, Up, lp);
-        if (outl) {
-            double acc = 0.0;
-#pragma unroll
-            for (int v = 0; v < NV; v++) acc += lp[v] * R2[v];
-            dtb += acc / a.dl;  // c2 = dt/dl
-        }
-    }
-    lds_put<NV>(S3, nt, t, lp);  // S1 still holds every cell's stage-2 right-face state fm
-    park(K3, lp);
-    __syncthreads();
-    double fpb[NV];
-    {
-        // interface k+1/2 of stage 2: l = left state of cell k (recomputed),
-        // r = right state of cell k+1 (the value the forward flux took)
-        double lpn[NV], fb[NV], q2[NV], l[NV], r[NV], junk[NV], rb[NV];
-        lds_get<NV>(S3, nt, tp, lpn);
-#pragma unroll
-        for (int v = 0; v < NV; v++) fb[v] = a.c2 * (lpn[v] - lp[v]);
-        double qc[NV];
-        lds_get<NV>(Q2, nt, t, qc);
-        lds_get<NV>(Q2, nt, tm, qm);
-        lds_get<NV>(Q2, nt, tp, q2);
-        faces<P, LIM>(a, qm, qc, q2, l, junk);
-        lds_get<NV>(S1, nt, tp, r);
-#pragma unroll
-        for (int v = 0; v < NV; v++) fpb[v] = rb[v] = 0.0;
-        const double cb = flux_vjp<P>(a, l, r, fb, fpb, rb);
-        if (outl) chb += cb;
-        lds_put<NV>(S2, nt, t, rb);  // belongs to cell k+1
-    }
-    __syncthreads();
-    double lsp[NV];  // lam* through the floors of stage 1
-    double l1[NV];   // stage-1 left state of interface k+1/2
-    {
-        double fmb[NV], qb[NV], dlb[NV], drb[NV];
-        double qc[NV];
-        lds_get<NV>(S2, nt, tm, fmb);
-        lds_get<NV>(Q2, nt, t, qc);
-        lds_get<NV>(Q2, nt, tm, qm);
-        lds_get<NV>(Q2, nt, tp, qp);
-        faces_vjp<P, LIM>(a, qm, qc, qp, fpb, fmb, qb, dlb, drb);
-        lds_put<NV>(S1, nt, t, dlb);
-        lds_put<NV>(S3, nt, t, drb);
+        double U[NV], q[NV], qm[NV], qp[NV], fm[NV];
+        load_u(U);
+        prim<P>(U, a.gam_1, q);
+        lds_put<NV>(Q, t, q);
         __syncthreads();
-        double dln[NV], drp[NV];
-        lds_get<NV>(S1, nt, tp, dln);
-        lds_get<NV>(S3, nt, tm, drp);
+        lds_get<NV>(Q, tm, qm);
+        lds_get<NV>(Q, tp, qp);
+        faces<P, LIM>(a, qm, q, qp, fp, fm);
+        lds_put<NV>(S, t, fm);
+        __syncthreads();
+        lds_get<NV>(S, tp, r);
+        flux<P>(a, fp, r, F);
+        lds_put<NV>(T, t, F);
+        __syncthreads();
+        double Fm[NV], R1[NV], Us[NV];
+        lds_get<NV>(T, tm, Fm);
+#pragma unroll
+        for (int v = 0; v < NV; v++) R1[v] = Fm[v] - F[v];
+        stage1(U, R1, Us);
+        floored(Us);
+        lds_put<NV>(K, t, R1);
+        // ---- forward: stage 2 ----
+        prim<P>(Us, a.gam_1, q);
+        lds_put<NV>(Q, t, q);
+        __syncthreads();
+        lds_get<NV>(Q, tm, qm);
+        lds_get<NV>(Q, tp, qp);
+        faces<P, LIM>(a, qm, q, qp, fp, fm);
+        lds_put<NV>(S, t, fm);
+        __syncthreads();
+        lds_get<NV>(S, tp, r);
+        flux<P>(a, fp, r, F);
+        lds_put<NV>(T, t, F);
+        __syncthreads();
+    }
+    double dtb = 0.0, chb = 0.0;
+    double fpb[NV];
+    // ---- reverse: stage 2 ----
+    {
+        double lp[NV];  // lam' through the psi damping and the floors of stage 2
+        {
+            double U[NV], Fm[NV], R2[NV], Up[NV];
+            load_u(U);
+            lds_get<NV>(T, tm, Fm);
+#pragma unroll
+            for (int v = 0; v < NV; v++) {
+                R2[v] = Fm[v] - F[v];
+                const double un = U[v] + a.c2 * R2[v];
+                Up[v] = (v < 5) ? un + 0.0 : un;
+            }
+#pragma unroll
+            for (int k = 0; k < NV; k++) lp[k] = a.lam_out[(long long)plane_of_adj<DIR>(k) * a.sv + idx];
+            if constexpr (P::MAG) lp[8] = lp[8] * a.psi_fac;
+            floors_vjp<P>(a, Up, lp);
+            if (outl) {
+                double acc = 0.0;
+#pragma unroll
+                for (int v = 0; v < NV; v++) acc += lp[v] * R2[v];
+                dtb += acc / a.dl;  // c2 = dt/dl
+            }
+        }
+        lds_put<NV>(S, t, lp);
+        __syncthreads();
+        // interface k+1/2: fp is cell k's left state, r cell k+1's right state
+        double lpn[NV], fb[NV], rb[NV];
+        lds_get<NV>(S, tp, lpn);
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-            qb[v] += drp[v] - dln[v];
+            fb[v] = a.c2 * (lpn[v] - lp[v]);
+            fpb[v] = rb[v] = 0.0;
+        }
+        const double cb = flux_vjp<P>(a, fp, r, fb, fpb, rb);
+        if (outl) chb += cb;
+        lds_put<NV>(T, t, rb);  // belongs to cell k+1
+    }
+    __syncthreads();
+    {
+        double qb[NV], dlb[NV], drb[NV];
+        {
+            double fmb[NV], qc[NV], qm[NV], qp[NV];
+            lds_get<NV>(T, tm, fmb);
+            lds_get<NV>(Q, t, qc);
+            lds_get<NV>(Q, tm, qm);
+            lds_get<NV>(Q, tp, qp);
+            faces_vjp<P, LIM>(a, qm, qc, qp, fpb, fmb, qb, dlb, drb);
+        }
+        __syncthreads();
+        lds_put<NV>(T, t, dlb);
+        lds_put<NV>(Q, t, drb);
+        __syncthreads();
+        lds_get<NV>(T, tp, dlb);
+        lds_get<NV>(Q, tm, drb);
+        double lsp[NV];  // lam* through the floors of stage 1
+#pragma unroll
+        for (int v = 0; v < NV; v++) {
+            qb[v] += drb[v] - dlb[v];
             lsp[v] = 0.0;
         }
-        fetch(K2, Us_pre);
-        {
-            double Usr[NV];
-#pragma unroll
-            for (int v = 0; v < NV; v++) Usr[v] = Us_pre[v];
-            unsigned fl = 0u;
-            double dm = 0.0;
-            floors<P>(Usr, a.smalld, a.smallei, a.use_smalld, a.use_smallei, false, fl, dm);
-            prim_vjp<P>(a, Usr, qb, lsp);
-        }
-        floors_vjp<P>(a, Us_pre, lsp);
-        fetch(K1, R1);
+        double U[NV], R1[NV], W[NV];
+        load_u(U);
+        lds_get<NV>(K, t, R1);
+        stage1(U, R1, W);
+        floored(W);
+        prim_vjp<P>(a, W, qb, lsp);
+        stage1(U, R1, W);
+        floors_vjp<P>(a, W, lsp);
         if (outl) {
             double acc = 0.0;
 #pragma unroll
             for (int v = 0; v < NV; v++) acc += lsp[v] * R1[v];
             dtb += (0.5 * acc) / a.dl;  // c1 = (dt/2)/dl
         }
-        lds_put<NV>(S2, nt, t, lsp);
-        // stage-1 face states of cell k: l1 stays here, fm goes to Q2 (whose
-        // reads all came before the last barrier) for the left neighbour
-        double qc1[NV], qp1[NV], fm1[NV];
-        lds_get<NV>(Q1, nt, t, qc1);
-        lds_get<NV>(Q1, nt, tm, qm);
-        lds_get<NV>(Q1, nt, tp, qp1);
-        faces<P, LIM>(a, qm, qc1, qp1, l1, fm1);
-        lds_put<NV>(Q2, nt, t, fm1);
+        lds_put<NV>(K, t, lsp);
+        // S: the two direct terms lam' + lam* of the own cell
+#pragma unroll
+        for (int v = 0; v < NV; v++) S[t * NV + v] = lsp[v] + S[t * NV + v];
+        double q[NV];
+        prim<P>(U, a.gam_1, q);
+        __syncthreads();
+        lds_put<NV>(Q, t, q);
     }
     __syncthreads();
     // ---- reverse: stage 1 ----
     {
-        double lsn[NV], fb[NV], r[NV], rb[NV];
-        lds_get<NV>(S2, nt, tp, lsn);
-        fetch(K3, lp);
+        double fb[NV], rb[NV];
+        {
+            double qm[NV], q[NV], qp[NV], fm[NV];
+            lds_get<NV>(Q, tm, qm);
+            lds_get<NV>(Q, t, q);
+            lds_get<NV>(Q, tp, qp);
+            faces<P, LIM>(a, qm, q, qp, fp, fm);
+            lds_put<NV>(T, t, fm);
 #pragma unroll
-        for (int v = 0; v < NV; v++) {
-            fb[v] = a.c1 * (lsn[v] - lsp[v]);
-            lsp[v] = lsp[v] + lp[v];  // from here on lam* + lam' (the two direct terms)
+            for (int v = 0; v < NV; v++) {
+                fb[v] = a.c1 * (K[tp * NV + v] - K[t * NV + v]);
+                fpb[v] = rb[v] = 0.0;
+            }
         }
-        lds_get<NV>(Q2, nt, tp, r);  // stage-1 right state of cell k+1
-#pragma unroll
-        for (int v = 0; v < NV; v++) fpb[v] = rb[v] = 0.0;
-        const double cb = flux_vjp<P>(a, l1, r, fb, fpb, rb);
+        __syncthreads();
+        lds_get<NV>(T, tp, r);
+        const double cb = flux_vjp<P>(a, fp, r, fb, fpb, rb);
         if (outl) chb += cb;
-        lds_put<NV>(S1, nt, t, rb);
+        lds_put<NV>(K, t, rb);
     }
     __syncthreads();
     double lam[NV];
     {
-        double fmb[NV], qb[NV], dlb[NV], drb[NV];
-        double qc[NV];
-        lds_get<NV>(S1, nt, tm, fmb);
-        lds_get<NV>(Q1, nt, t, qc);
-        lds_get<NV>(Q1, nt, tm, qm);
-        lds_get<NV>(Q1, nt, tp, qp);
-        faces_vjp<P, LIM>(a, qm, qc, qp, fpb, fmb, qb, dlb, drb);
-        lds_put<NV>(S2, nt, t, dlb);
-        lds_put<NV>(S3, nt, t, drb);
+        double qb[NV], dlb[NV], drb[NV], lsp[NV];
+        {
+            double fmb[NV], qc[NV], qm[NV], qp[NV];
+            lds_get<NV>(K, tm, fmb);
+            lds_get<NV>(Q, t, qc);
+            lds_get<NV>(Q, tm, qm);
+            lds_get<NV>(Q, tp, qp);
+            faces_vjp<P, LIM>(a, qm, qc, qp, fpb, fmb, qb, dlb, drb);
+        }
+        lds_put<NV>(T, t, dlb);
+        lds_get<NV>(S, t, lsp);
+        lds_put<NV>(S, t, drb);
         __syncthreads();
-        double dln[NV], drp[NV];
-        lds_get<NV>(S2, nt, tp, dln);
-        lds_get<NV>(S3, nt, tm, drp);
+        lds_get<NV>(T, tp, dlb);
+        lds_get<NV>(S, tm, drb);
 #pragma unroll
         for (int v = 0; v < NV; v++) {
-            qb[v] += drp[v] - dln[v];
+            qb[v] += drb[v] - dlb[v];
             lam[v] = 0.0;
         }
-        double Ur[NV];  // reloaded: cheaper than holding U across the kernel
-#pragma unroll
-        for (int k = 0; k < NV; k++) Ur[k] = a.u[(long long)plane_of_adj<DIR>(k) * a.sv + idx];
-        prim_vjp<P>(a, Ur, qb, lam);
+        double U[NV];
+        load_u(U);
+        prim_vjp<P>(a, U, qb, lam);
 #pragma unroll
         for (int v = 0; v < NV; v++) lam[v] = lam[v] + lsp[v];
     }
@@ -406,25 +421,42 @@ __device__ __forceinline__ void adjoint_tile(const AdjArgs &a, int bid, double *
 }
 
 template <int DIR, class P, int LIM>
-__global__ __launch_bounds__(256) void k_sweep_adjoint(const AdjArgs a)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_sweep_adjoint(const AdjArgs a)
 {
     extern __shared__ double lds[];
-    adjoint_tile<DIR, P, LIM>(a, blockIdx.x, lds);
+    // XCD-aware order, as k_sweep: tiles whose cells share cache lines (the
+    // pencils of a y or z tile are a fraction of a line wide) share an L2
+    int bid = blockIdx.x;
+    const int nfull = (int)(gridDim.x / 8u) * 8;
+    if (bid < nfull) bid = (bid % 8) * (nfull / 8) + bid / 8;
+    adjoint_tile<DIR, P, LIM>(a, bid, lds);
 }
 
 // Persistent adjoint sweep over a block list (independent instances): as
-// k_sweep_list, tiles from a device queue, per-block arguments from a table.
+// k_sweep_list, tiles from device queues, per-block arguments from a table.
+// The items are cut into kListQueues contiguous ranges with a counter each;
+// a workgroup starts with the range of its XCD (workgroup i runs on XCD
+// i % 8), so tiles that share cache lines share an L2, and goes on to the
+// others when it is empty.  A workgroup leaves after one fetch past the end
+// of every range.
 template <int DIR, class P, int LIM>
-__global__ __launch_bounds__(256) void k_sweep_adjoint_list(const AdjListArgs L)
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_sweep_adjoint_list(const AdjListArgs L)
 {
     extern __shared__ double lds[];
     __shared__ unsigned s_item;
+    unsigned x = blockIdx.x % kListQueues, left = kListQueues;
     for (;;) {
         __syncthreads();  // the previous tile is done with LDS and s_item
-        if (threadIdx.x == 0) s_item = atomicAdd(L.queue, 1u);
+        if (threadIdx.x == 0) s_item = atomicAdd(L.queue + x, 1u);
         __syncthreads();
-        const unsigned item = (unsigned)__builtin_amdgcn_readfirstlane((int)s_item);
-        if (item >= L.nitems) break;
+        const unsigned got = (unsigned)__builtin_amdgcn_readfirstlane((int)s_item);
+        const unsigned lo = list_range(L.nitems, x), hi = list_range(L.nitems, x + 1);
+        if (got >= hi - lo) {
+            if (--left == 0) break;
+            x = (x + 1) % kListQueues;
+            continue;
+        }
+        const unsigned item = lo + got;
         typedef const __attribute__((address_space(4))) unsigned cu32;
         const int blk = __builtin_amdgcn_readfirstlane((int)((cu32 *)L.items)[item]);
         AdjArgs a;
@@ -695,7 +727,7 @@ __global__ void k_dt_apply_jobs(const DtBatchJob *__restrict__ jobs, int njobs)
 template <int DIR, class P, int LIM>
 static hipError_t adj_t(const AdjArgs &a, int nt, long long nblk, hipStream_t st)
 {
-    const size_t lds = sizeof(double) * adj_lds_arrays<P>() * P::NV * nt;
+    const size_t lds = sizeof(double) * kAdjArrays * P::NV * nt;
     static bool raised = false;
     if (!raised) {
         hipError_t e = hipFuncSetAttribute((const void *)k_sweep_adjoint<DIR, P, LIM>,
@@ -728,7 +760,7 @@ static hipError_t adjl_t(const AdjListArgs &L, int grid, hipStream_t st, int *re
 {
     const int nt = 256;
     const void *fn = (const void *)k_sweep_adjoint_list<DIR, P, LIM>;
-    const size_t lds = sizeof(double) * adj_lds_arrays<P>() * P::NV * nt;
+    const size_t lds = sizeof(double) * kAdjArrays * P::NV * nt;
     const size_t lds_max = 160 * 1024 - 256;
     static bool raised = false;
     if (!raised) {

@@ -19,6 +19,7 @@ struct AdjArgs {
     int chunks, ptiles, out;
     int lim, limb;          // limiter of the fluid variables, of B and psi
     double gam, gam_1;
+    double rg, rg1, rch;    // 1/gam, 1/(gam - 1), 1/ch (MHD)
     double c1, c2;          // (dt/2)/dl and dt/dl
     double dl;              // cell size along the sweep
     double ch;              // GLM speed of the sweep (MHD)
@@ -43,15 +44,21 @@ struct DtAdjArgs {
 };
 
 // Persistent adjoint sweep over a block list (workgroups of 256 lanes take
-// tiles from a queue; tile item belongs to block items[item] and is its
+// tiles from queues; tile item belongs to block items[item] and is its
 // tile item - first[block]).  Each block's AdjArgs has its tile shape with
 // TP*TS <= 256 and its dtb/chb partial arrays sized for 4 waves per tile.
+constexpr unsigned kListQueues = 8;  // item ranges of a list launch, one per XCD
+// first item of range x of n items
+__host__ __device__ inline unsigned list_range(unsigned n, unsigned x)
+{
+    return (unsigned)((unsigned long long)n * x / kListQueues);
+}
 struct AdjListArgs {
     const AdjArgs *args;
     const unsigned *first;
     const unsigned *items;
     unsigned nitems;
-    unsigned *queue;
+    unsigned *queue;  // kListQueues counters, zero before the launch
 };
 
 // out[0] = sum of part[0 .. n-1] in a fixed order

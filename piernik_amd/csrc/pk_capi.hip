@@ -1089,6 +1089,9 @@ int do_sweep_adjoint(Block *b, const double *u, int d, double dt, double ch, dou
     a.limb = g_cfg.limiter_b;
     a.gam = g_cfg.fluid[0].gamma;
     a.gam_1 = g_cfg.fluid[0].gamma - 1.0;
+    a.rg = 1.0 / a.gam;
+    a.rg1 = 1.0 / a.gam_1;
+    a.rch = g_mhd ? 1.0 / ch : 0.0;
     a.c1 = (0.5 * dt) / b->dl[d];
     a.c2 = (1.0 * dt) / b->dl[d];
     a.dl = b->dl[d];
@@ -1910,7 +1913,7 @@ int ens_build()
     HIPCHK(hipMalloc((void **)&g_ens.d_dtout, sizeof(double) * 4 * n));
     HIPCHK(hipHostMalloc((void **)&g_ens.h_dtout, sizeof(double) * 4 * n, hipHostMallocDefault));
     HIPCHK(hipMalloc((void **)&g_ens.d_jobs, sizeof(pk::CopyJob) * n));
-    HIPCHK(hipMalloc((void **)&g_ens.d_queue, sizeof(unsigned) * 2));
+    HIPCHK(hipMalloc((void **)&g_ens.d_queue, sizeof(unsigned) * pk::kListQueues));
     g_ens.h_jobs.resize(n);
     g_ens.dt_old.assign(n, -1.0);
     g_ens.fresh = false;
@@ -3762,6 +3765,9 @@ int pk_ensemble_step_adjoint(const double *dts, int32_t slot0, double *dt_bar)
             a.limb = g_cfg.limiter_b;
             a.gam = g_cfg.fluid[0].gamma;
             a.gam_1 = g_cfg.fluid[0].gamma - 1.0;
+            a.rg = 1.0 / a.gam;
+            a.rg1 = 1.0 / a.gam_1;
+            a.rch = g_mhd ? 1.0 / ch[i] : 0.0;
             a.c1 = (0.5 * dts[i]) / b->dl[d];
             a.c2 = (1.0 * dts[i]) / b->dl[d];
             a.dl = b->dl[d];
@@ -3779,7 +3785,7 @@ int pk_ensemble_step_adjoint(const double *dts, int32_t slot0, double *dt_bar)
         HIPCHK(hipMemcpyAsync(g_ens.d_adj, g_ens.h_adj, sizeof(pk::AdjArgs) * n, hipMemcpyHostToDevice, g_stream));
         HIPCHK(hipMemcpyAsync(g_ens.d_sum, g_ens.h_sum.data(), sizeof(pk::SumJob) * 2 * n, hipMemcpyHostToDevice,
                               g_stream));
-        HIPCHK(pk::launch_zero_u32(g_ens.d_queue, 1, g_stream));
+        HIPCHK(pk::launch_zero_u32(g_ens.d_queue, pk::kListQueues, g_stream));
         pk::AdjListArgs L{};
         L.args = g_ens.d_adj;
         L.first = g_ens.d_afirst[d];

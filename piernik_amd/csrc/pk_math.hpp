@@ -20,6 +20,9 @@
 #ifndef PK_RELAXED
 #define PK_RELAXED 0
 #endif
+#ifndef PK_NORMAL_RANGE
+#define PK_NORMAL_RANGE 0
+#endif
 
 // Callable from device code and, for host-side checks of the same
 // arithmetic, from host code.
@@ -40,6 +43,49 @@ enum Limiter : int { LIM_VANLEER = 0, LIM_MINMOD = 1, LIM_MONCEN = 2, LIM_SUPERB
 PK_HD double fmn(double a, double b) { return fmin(a, b); }
 PK_HD double fmx(double a, double b) { return fmax(a, b); }
 
+// 1 / b from the hardware reciprocal and two Newton-Raphson steps: the
+// reciprocal an IEEE division refines before its last correction, without
+// the range scaling (b and 1/b normal), within an ulp of 1/b.
+PK_HD double nrcp(double b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    double r = __builtin_amdgcn_rcp(b);
+    r = fma(fma(-b, r, 1.0), r, r);
+    return fma(fma(-b, r, 1.0), r, r);
+#else
+    return 1.0 / b;
+#endif
+}
+
+// a / b given r = nrcp(b): the last steps of an IEEE division.
+PK_HD double ndiv(double a, double b, double r)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double q = a * r;
+    return fma(fma(-b, q, a), r, q);
+#else
+    return a / b;
+#endif
+}
+
+// sqrt(x) of a normal x >= 2^-767 or 0 without the range scaling of the
+// correctly rounded expansion, the same refinement steps.
+PK_HD double nsqrt(double x)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    const double y = __builtin_amdgcn_rsq(x);
+    double g = x * y, h = 0.5 * y;
+    const double r = fma(-h, g, 0.5);
+    g = fma(g, r, g);
+    h = fma(h, r, h);
+    g = fma(fma(-g, g, x), h, g);
+    g = fma(fma(-g, g, x), h, g);
+    return x > 0.0 ? g : 0.0;
+#else
+    return sqrt(x);
+#endif
+}
+
 // a / b and sqrt(x).  The relaxed build (PK_RELAXED: the FMA-contracted
 // kernels) forms them from the hardware reciprocal and reciprocal square root
 // with one Newton-Raphson step each and a final residual correction, which
@@ -47,7 +93,11 @@ PK_HD double fmx(double a, double b) { return fmax(a, b); }
 // finite, nonzero (division) and positive normal (sqrt) operands of the
 // sweep, in fewer instructions than the compiler's fast expansions (no
 // range scaling, one refinement less); sqrt of 0 is 0.  The exact build
-// uses the correctly rounded operations, as the reference does.
+// uses the correctly rounded operations, as the reference does.  The reverse
+// mode (PK_NORMAL_RANGE) uses ndiv and nsqrt: the same bits as the exact
+// build wherever its expansions apply no range scaling (operands and
+// quotients well inside 2^-767 .. 2^767), in fewer instructions and with
+// one reciprocal for all quotients of a divisor.
 PK_HD double qdiv(double a, double b)
 {
 #if PK_RELAXED && defined(__HIP_DEVICE_COMPILE__)
@@ -55,6 +105,8 @@ PK_HD double qdiv(double a, double b)
     r = fma(fma(-b, r, 1.0), r, r);
     const double q = a * r;
     return fma(fma(-b, q, a), r, q);
+#elif PK_NORMAL_RANGE
+    return ndiv(a, b, nrcp(b));
 #else
     return a / b;
 #endif
@@ -70,6 +122,8 @@ PK_HD double qsqrt(double x)
     h = fma(h, r, h);
     g = fma(fma(-g, g, x), h, g);
     return x > 0.0 ? g : 0.0;
+#elif PK_NORMAL_RANGE
+    return nsqrt(x);
 #else
     return sqrt(x);
 #endif
