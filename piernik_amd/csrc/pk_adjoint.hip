@@ -475,8 +475,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
 // Deterministic sum of n per-wave partials: kRedParts fixed ranges
 // [n*g/kRedParts, n*(g+1)/kRedParts), each summed by one 256-lane workgroup
 // (per-lane strided sums, then a tree), then the range sums added in order g.
-// The one-workgroup-per-job kernel repeats the same ranges and order, so both
-// give the same bits.
+// The kernels over many jobs use the same ranges and order, so both give the
+// same bits.
 __device__ double wg_range_sum(const double *__restrict__ part, long long lo, long long hi, double *red)
 {
     const int t = threadIdx.x;
@@ -495,14 +495,27 @@ __device__ double wg_range_sum(const double *__restrict__ part, long long lo, lo
 
 __device__ __forceinline__ long long range_lo(long long n, int g) { return n * g / kRedParts; }
 
-// one workgroup per job
-__global__ __launch_bounds__(256) void k_sum_parts_jobs(const SumJob *__restrict__ jobs)
+// grid (kRedParts, jobs): range g of a job, into part[n + g].  (One workgroup
+// per job walked its 64 ranges one after the other, ten barriers each: 61 us
+// for the 40 sums of 20 instances.)
+__global__ __launch_bounds__(256) void k_sum_ranges_jobs(const SumJob *__restrict__ jobs)
 {
     __shared__ double red[256];
-    const SumJob j = jobs[blockIdx.x];
+    const SumJob j = jobs[blockIdx.y];
+    const int g = blockIdx.x;
+    const double r = wg_range_sum(j.part, range_lo(j.n, g), range_lo(j.n, g + 1), red);
+    if (threadIdx.x == 0) j.part[j.n + g] = r;
+}
+
+// the range sums of each job in order, a job per lane
+__global__ void k_sum_final_jobs(const SumJob *__restrict__ jobs, int njobs)
+{
+    const int jb = blockIdx.x * blockDim.x + threadIdx.x;
+    if (jb >= njobs) return;
+    const SumJob j = jobs[jb];
     double tot = 0.0;
-    for (int g = 0; g < kRedParts; g++) tot += wg_range_sum(j.part, range_lo(j.n, g), range_lo(j.n, g + 1), red);
-    if (threadIdx.x == 0) j.out[0] = tot;
+    for (int g = 0; g < kRedParts; g++) tot += j.part[j.n + g];
+    j.out[0] = tot;
 }
 
 // grid (kRedParts, 2): range g of partial array y, into part_y[n + g]
@@ -524,51 +537,6 @@ __global__ void k_sum_final(const double *__restrict__ p0, const double *__restr
     double tot = 0.0;
     for (int g = 0; g < kRedParts; g++) tot += p[n + g];
     out[blockIdx.x] = tot;
-}
-
-// Adjoint of the periodic ghost refresh along DIR (k_fill_ghosts): every
-// ghost cell's adjoint is added to its interior image and cleared.  Run for
-// z, then y, then x (the refresh runs x, y, z).
-template <int DIR>
-__global__ void k_fold_ghosts(double *__restrict__ lam, long long sv, int sy, int sz, int ng0, int ng1, int ng2,
-                              int g0, int g1, int g2, int n0, int n1, int n2, int nplanes)
-{
-    const int ng[3] = {ng0, ng1, ng2}, g[3] = {g0, g1, g2}, n[3] = {n0, n1, n2};
-    constexpr int e1 = (DIR == 0) ? 1 : 0;
-    constexpr int e2 = (DIR == 2) ? 1 : 2;
-    const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    // one thread per (plane, transverse cell, interior image along DIR); it
-    // owns the ghosts that copy that image, so no two threads touch one cell
-    const long long per = (long long)n[DIR] * ng[e1] * ng[e2];
-    if (tid >= per * nplanes) return;
-    const int v = (int)(tid / per);
-    long long r = tid % per;
-    const int i = (int)(r % n[DIR]);
-    r /= n[DIR];
-    int xyz[3];
-    xyz[e1] = (int)(r % ng[e1]);
-    xyz[e2] = (int)(r / ng[e1]);
-    double *base = lam + (long long)v * sv;
-    xyz[DIR] = g[DIR] + i;
-    const long long dst = (long long)xyz[0] + (long long)sy * xyz[1] + (long long)sz * xyz[2];
-    double acc = base[dst];
-    // ghost layers whose image is i: low ghost j (0 <= j < g) copies g + n - g + j ... i.e. image n + j - g + g
-    for (int j = 0; j < g[DIR]; j++) {
-        // low ghost at j copies interior index n - g + j; high ghost at g + n + j copies interior index j
-        if (i == n[DIR] - g[DIR] + j) {
-            xyz[DIR] = j;
-            const long long gi = (long long)xyz[0] + (long long)sy * xyz[1] + (long long)sz * xyz[2];
-            acc += base[gi];
-            base[gi] = 0.0;
-        }
-        if (i == j) {
-            xyz[DIR] = g[DIR] + n[DIR] + j;
-            const long long gi = (long long)xyz[0] + (long long)sy * xyz[1] + (long long)sz * xyz[2];
-            acc += base[gi];
-            base[gi] = 0.0;
-        }
-    }
-    base[dst] = acc;
 }
 
 __global__ void k_zero_best(unsigned long long *best)
@@ -648,15 +616,26 @@ __global__ void k_dt_apply(const DtAdjArgs a, const unsigned long long *best, do
     k_dt_apply_body(a, best, lam);
 }
 
-// one workgroup per job: min over the job's cells and directions of dl/c
+__global__ void k_dt_init_jobs(const DtBatchJob *__restrict__ jobs, int njobs)
+{
+    const int jb = blockIdx.x * blockDim.x + threadIdx.x;
+    if (jb >= njobs) return;
+    *jobs[jb].mn = 1.7976931348623157e308;
+    *jobs[jb].best = ~0ull;
+}
+
+// grid (chunks, jobs): min over the job's cells and directions of dl/c
+// (positive: ordered as its bit pattern).  (A workgroup per job took 320 us
+// for the largest of 20 instances, 256^2 cells.)
 __global__ __launch_bounds__(256) void k_dt_mn_jobs(const DtBatchJob *__restrict__ jobs)
 {
-    __shared__ double red[256];
-    const DtBatchJob &J = jobs[blockIdx.x];
+    const DtBatchJob &J = jobs[blockIdx.y];
     const DtAdjArgs &a = J.a;
     const long long ncell = (long long)a.n[0] * a.n[1] * a.n[2];
+    if ((long long)blockIdx.x * 256 >= ncell) return;
     double m = 1.7976931348623157e308;
-    for (long long c = threadIdx.x; c < ncell; c += 256) {
+    for (long long c = (long long)blockIdx.x * blockDim.x + threadIdx.x; c < ncell;
+         c += (long long)gridDim.x * blockDim.x) {
         const int i = (int)(c % a.n[0]);
         const long long r = c / a.n[0];
         const int j = (int)(r % a.n[1]);
@@ -672,16 +651,10 @@ __global__ __launch_bounds__(256) void k_dt_mn_jobs(const DtBatchJob *__restrict
             m = fmn(m, a.dl[q] / fmx(v + cs, 1.17549435082228750797e-38));
         }
     }
-    red[threadIdx.x] = m;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] = fmn(red[threadIdx.x], red[threadIdx.x + w]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        *J.mn = red[0];
-        *J.best = ~0ull;
-    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) m = fmn(m, __shfl_xor(m, o, 64));
+    if ((threadIdx.x & 63) == 0)
+        atomicMin((unsigned long long *)J.mn, (unsigned long long)__double_as_longlong(m));
 }
 
 // grid (chunks, jobs): the smallest cell/direction index attaining the minimum
@@ -822,7 +795,11 @@ hipError_t launch_sweep_adjoint_list(int dir, bool mhd, int lim, int limb, const
 hipError_t launch_sum_parts_jobs(const SumJob *jobs, int njobs, hipStream_t st)
 {
     if (njobs <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_sum_parts_jobs, dim3((unsigned)njobs), dim3(256), 0, st, jobs);
+    for (int j0 = 0; j0 < njobs; j0 += 32768) {
+        const int n = njobs - j0 < 32768 ? njobs - j0 : 32768;
+        hipLaunchKernelGGL(k_sum_ranges_jobs, dim3(kRedParts, (unsigned)n), dim3(256), 0, st, jobs + j0);
+    }
+    hipLaunchKernelGGL(k_sum_final_jobs, dim3((unsigned)((njobs + 63) / 64)), dim3(64), 0, st, jobs, njobs);
     return hipGetLastError();
 }
 
@@ -853,34 +830,15 @@ hipError_t launch_sweep_adjoint(int dir, bool mhd, const AdjArgs &a, double *dtb
     return hipGetLastError();
 }
 
-hipError_t launch_fold_ghosts(double *lam, long long sv, int sy, int sz, const int ng[3], const int g[3],
-                              const int n[3], int nplanes, hipStream_t st)
-{
-    for (int d = 2; d >= 0; d--) {
-        if (g[d] == 0) continue;
-        const int e1 = (d == 0) ? 1 : 0, e2 = (d == 2) ? 1 : 2;
-        const long long total = (long long)n[d] * ng[e1] * ng[e2] * nplanes;
-        const unsigned blocks = (unsigned)((total + 255) / 256);
-        if (d == 0)
-            hipLaunchKernelGGL(k_fold_ghosts<0>, dim3(blocks), dim3(256), 0, st, lam, sv, sy, sz, ng[0], ng[1], ng[2],
-                               g[0], g[1], g[2], n[0], n[1], n[2], nplanes);
-        if (d == 1)
-            hipLaunchKernelGGL(k_fold_ghosts<1>, dim3(blocks), dim3(256), 0, st, lam, sv, sy, sz, ng[0], ng[1], ng[2],
-                               g[0], g[1], g[2], n[0], n[1], n[2], nplanes);
-        if (d == 2)
-            hipLaunchKernelGGL(k_fold_ghosts<2>, dim3(blocks), dim3(256), 0, st, lam, sv, sy, sz, ng[0], ng[1], ng[2],
-                               g[0], g[1], g[2], n[0], n[1], n[2], nplanes);
-        hipError_t e = hipGetLastError();
-        if (e != hipSuccess) return e;
-    }
-    return hipSuccess;
-}
-
 hipError_t launch_dt_adjoint_batch(const DtBatchJob *jobs, int njobs, hipStream_t st)
 {
     if (njobs <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_dt_mn_jobs, dim3((unsigned)njobs), dim3(256), 0, st, jobs);
-    hipLaunchKernelGGL(k_dt_argmin_jobs, dim3(64, (unsigned)njobs), dim3(256), 0, st, jobs);
+    hipLaunchKernelGGL(k_dt_init_jobs, dim3((unsigned)((njobs + 63) / 64)), dim3(64), 0, st, jobs, njobs);
+    for (int j0 = 0; j0 < njobs; j0 += 32768) {
+        const unsigned n = (unsigned)(njobs - j0 < 32768 ? njobs - j0 : 32768);
+        hipLaunchKernelGGL(k_dt_mn_jobs, dim3(64, n), dim3(256), 0, st, jobs + j0);
+        hipLaunchKernelGGL(k_dt_argmin_jobs, dim3(64, n), dim3(256), 0, st, jobs + j0);
+    }
     hipLaunchKernelGGL(k_dt_apply_jobs, dim3((unsigned)((njobs + 63) / 64)), dim3(64), 0, st, jobs, njobs);
     return hipGetLastError();
 }

@@ -61,9 +61,10 @@ struct AdjListArgs {
     unsigned *queue;  // kListQueues counters, zero before the launch
 };
 
-// out[0] = sum of part[0 .. n-1] in a fixed order
+// out[0] = sum of part[0 .. n-1] in a fixed order; part has kRedParts more
+// doubles for the range sums
 struct SumJob {
-    const double *part;
+    double *part;
     long long n;
     double *out;
 };
@@ -88,8 +89,6 @@ hipError_t launch_sweep_adjoint_list(int dir, bool mhd, int lim, int limb, const
 hipError_t launch_sum_parts_jobs(const SumJob *jobs, int njobs, hipStream_t st);
 // dtb_out[0] = dL/d(dt) at fixed ch, dtb_out[1] = dL/d(ch)
 hipError_t launch_sweep_adjoint(int dir, bool mhd, const AdjArgs &a, double *dtb_out, hipStream_t st);
-hipError_t launch_fold_ghosts(double *lam, long long sv, int sy, int sz, const int ng[3], const int g[3],
-                              const int n[3], int nplanes, hipStream_t st);
 hipError_t launch_dt_adjoint(const DtAdjArgs &a, unsigned long long *best, double *lam, hipStream_t st);
 
 }  // namespace pk

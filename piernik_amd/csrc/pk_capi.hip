@@ -48,9 +48,9 @@ struct Block {
            *h_psih = nullptr;
     unsigned *d_flags = nullptr;
     unsigned long long *d_mass = nullptr;  // per fluid: the floor's mass counters (pk_mass.hpp)
-    double *d_dtout = nullptr;
+    double *dtout = nullptr;                  // timestep results (4 per fluid), pinned host memory
     unsigned long long *d_dtslots = nullptr;  // timestep reduction written by the last sweep of a step
-    bool dt_pending = false;                  // d_dtout holds timestep_fluid of the current state
+    bool dt_pending = false;                  // dtout holds timestep_fluid of the current state
     bool ghosts_stale = false;                // stream sweeps read the periodic interior and left the ghosts old
     // reverse mode (pk_adjoint_setup): saved states and the adjoint state
     std::vector<double *> slots;
@@ -112,6 +112,14 @@ size_t g_stage_bytes = 0;
 double *g_part = nullptr;    // partial results of the standalone timestep reduction
 pk_xfer::Ring g_ring;        // pinned chunks for host <-> device copies of the caller's arrays
 
+// Timestep results of the blocks: pinned host memory the final reduction
+// kernels write directly (no copy back), kDtOut doubles per block, in slabs
+// shared by many blocks; a freed block's place is used again, the slabs go
+// with the last block.
+constexpr int kDtOut = 8, kDtSlab = 256;
+std::vector<double *> g_dt_slabs, g_dt_free;
+size_t g_dt_used = 0;
+
 // Tile shapes chosen by pk_autotune, per block shape, direction and physics.
 struct TuneKey {
     int n0, n1, n2, dir, kind, lim, limb;
@@ -168,6 +176,30 @@ int fail(int code, const char *fmt, ...)
 double *state(Block *b, int i) { return b->buf[i] + b->xo; }
 double *fluid_state(Block *b, int i, int f) { return state(b, i) + (long long)g_fplane[f] * b->sv; }
 int nv_of(int f) { return g_fmag[f] ? 9 : 5; }
+
+int dtout_take(double **p)
+{
+    if (g_dt_free.empty()) {
+        double *slab = nullptr;
+        HIPCHK(hipHostMalloc((void **)&slab, sizeof(double) * kDtOut * kDtSlab, hipHostMallocDefault));
+        g_dt_slabs.push_back(slab);
+        for (int i = kDtSlab - 1; i >= 0; i--) g_dt_free.push_back(slab + kDtOut * i);
+    }
+    *p = g_dt_free.back();
+    g_dt_free.pop_back();
+    g_dt_used++;
+    return PK_OK;
+}
+
+void dtout_give(double *p)
+{
+    if (!p) return;
+    g_dt_free.push_back(p);
+    if (--g_dt_used) return;
+    for (double *slab : g_dt_slabs) (void)hipHostFree(slab);
+    g_dt_slabs.clear();
+    g_dt_free.clear();
+}
 
 void list_invalidate();
 void list_touch();
@@ -673,7 +705,6 @@ int do_sweep(Block *b, int ddim, double dt, double ch, double psi_fac, int image
         return PK_OK;
     }
     if (b->g[ddim] < 4) return fail(PK_EINVAL, "fused RK2 sweep needs nb >= 4 (nb = %d)", b->g[ddim]);
-    if (want_dt) HIPCHK(pk::launch_dtslots_init(b->d_dtslots, kDtSlots, g_stream));
     for (int f = 0; f < g_nfl; f++) {
         pk::SweepArgs a{};
         fill_common(b, f, a);
@@ -694,16 +725,17 @@ int do_sweep(Block *b, int ddim, double dt, double ch, double psi_fac, int image
     b->uh = -1;
     b->dt_pending = false;
     if (want_dt) {
-        HIPCHK(pk::launch_dtslots_final(b->d_dtslots, kDtSlots, b->d_dtout, g_stream));
+        HIPCHK(pk::launch_dtslots_final(b->d_dtslots, kDtSlots, 1, b->dtout, g_stream));
         b->dt_pending = true;
     }
     return PK_OK;
 }
 
-int do_fill(Block *b)
+// periodic ghost refresh of one of the block's two buffers
+int fill_buffer(Block *b, int i)
 {
     pk::GhostArgs a{};
-    a.u = state(b, b->cur);
+    a.u = state(b, i);
     a.sv = b->sv;
     a.sy = b->sy;
     a.sz = b->sz;
@@ -714,8 +746,13 @@ int do_fill(Block *b)
     }
     a.plane0 = 0;
     a.nplanes = g_nplanes;
-    for (int d = 0; d < 3; d++)
-        if (b->g[d] > 0) HIPCHK(pk::launch_fill_ghosts(d, a, g_stream));
+    HIPCHK(pk::launch_fill_periodic(a, g_stream));
+    return PK_OK;
+}
+
+int do_fill(Block *b)
+{
+    RCCHK(fill_buffer(b, b->cur));
     b->ghosts_stale = false;
     return PK_OK;
 }
@@ -723,28 +760,31 @@ int do_fill(Block *b)
 // timestep_fluid of every fluid of one block, min over fluids; with
 // cfl > 0 the min commutes with the multiplication by cfl, so one combined
 // reduction over all fluids' cells gives the same dt.
+pk::DtArgs dt_args(Block *b, int f)
+{
+    pk::DtArgs a{};
+    a.u = state(b, b->cur);
+    a.sv = b->sv;
+    a.sy = b->sy;
+    a.sz = b->sz;
+    for (int d = 0; d < 3; d++) {
+        a.ng[d] = b->ng[d];
+        a.g[d] = b->g[d];
+        a.n[d] = b->n[d];
+        a.has_dir[d] = g_cfg.has_dir[d];
+        a.dl[d] = b->dl[d];
+    }
+    a.plane0 = g_fplane[f];
+    a.bplane = g_magf >= 0 ? g_fplane[g_magf] + 5 : 0;
+    a.magnetized = g_fmag[f];
+    a.gam = g_cfg.fluid[f].gamma;
+    a.gam_1 = g_cfg.fluid[f].gamma - 1.0;
+    return a;
+}
+
 int enqueue_dt(Block *b, double *out)
 {
-    for (int f = 0; f < g_nfl; f++) {
-        pk::DtArgs a{};
-        a.u = state(b, b->cur);
-        a.sv = b->sv;
-        a.sy = b->sy;
-        a.sz = b->sz;
-        for (int d = 0; d < 3; d++) {
-            a.ng[d] = b->ng[d];
-            a.g[d] = b->g[d];
-            a.n[d] = b->n[d];
-            a.has_dir[d] = g_cfg.has_dir[d];
-            a.dl[d] = b->dl[d];
-        }
-        a.plane0 = g_fplane[f];
-        a.bplane = g_magf >= 0 ? g_fplane[g_magf] + 5 : 0;
-        a.magnetized = g_fmag[f];
-        a.gam = g_cfg.fluid[f].gamma;
-        a.gam_1 = g_cfg.fluid[f].gamma - 1.0;
-        HIPCHK(pk::launch_dt(a, g_part, out + 4 * f, g_stream));
-    }
+    for (int f = 0; f < g_nfl; f++) HIPCHK(pk::launch_dt(dt_args(b, f), g_part, out + 4 * f, g_stream));
     return PK_OK;
 }
 
@@ -765,17 +805,11 @@ void combine_dt(const double *v, int nsets, double *dt_out, double *c_out)
 
 int do_timestep(Block *b, double *dt_out, double *c_out)
 {
-    if (b->dt_pending) {
-        // reduced by the last sweep from the cells it wrote (same formula, same state)
-        HIPCHK(hipMemcpyAsync(g_pinned, b->d_dtout, 4 * sizeof(double), hipMemcpyDeviceToHost, g_stream));
-        HIPCHK(hipStreamSynchronize(g_stream));
-        combine_dt(g_pinned, 1, dt_out, c_out);
-        return PK_OK;
-    }
-    RCCHK(enqueue_dt(b, b->d_dtout));  // d_dtout holds 4 doubles per fluid
-    HIPCHK(hipMemcpyAsync(g_pinned, b->d_dtout, 4 * g_nfl * sizeof(double), hipMemcpyDeviceToHost, g_stream));
+    // pending: reduced by the last sweep from the cells it wrote (same formula, same state)
+    const bool pending = b->dt_pending;
+    if (!pending) RCCHK(enqueue_dt(b, b->dtout));
     HIPCHK(hipStreamSynchronize(g_stream));
-    combine_dt(g_pinned, g_nfl, dt_out, c_out);
+    combine_dt(b->dtout, pending ? 1 : g_nfl, dt_out, c_out);
     return PK_OK;
 }
 
@@ -863,8 +897,9 @@ int alloc_block(Block *b)
     HIPCHK(hipMalloc((void **)&b->d_mass, kMassBytes));
     HIPCHK(hipMemsetAsync(b->d_flags, 0, sizeof(unsigned), g_stream));
     HIPCHK(hipMemsetAsync(b->d_mass, 0, kMassBytes, g_stream));
-    HIPCHK(hipMalloc((void **)&b->d_dtout, sizeof(double) * 8));
+    RCCHK(dtout_take(&b->dtout));
     HIPCHK(hipMalloc((void **)&b->d_dtslots, sizeof(unsigned long long) * 4 * kDtSlots));
+    HIPCHK(pk::launch_dtslots_init(b->d_dtslots, kDtSlots, g_stream));
     return PK_OK;
 }
 
@@ -895,7 +930,7 @@ void free_block(Block *b)
         if (b->buf[i]) (void)hipFree(b->buf[i]);
     if (b->d_flags) (void)hipFree(b->d_flags);
     if (b->d_mass) (void)hipFree(b->d_mass);
-    if (b->d_dtout) (void)hipFree(b->d_dtout);
+    dtout_give(b->dtout);
     if (b->d_dtslots) (void)hipFree(b->d_dtslots);
     if (b->d_flux) (void)hipFree(b->d_flux);
     if (b->backup) (void)hipFree(b->backup);
@@ -957,58 +992,79 @@ pk::PlaneMap map_psi()
     return m;
 }
 
-// from_device: the source array is in device memory (no host staging)
-int upload_array(Block *b, const double *h, const pk::PlaneMap &m, double *dst, bool from_device)
+// the conversion arguments of a block's state at soa, no arrays yet
+pk::PlanesArgs planes_args(const Block *b, const double *soa)
 {
-    const size_t ncell = (size_t)b->ng[0] * b->ng[1] * b->ng[2];
-    const double *src = h;
-    if (!from_device) {
-        RCCHK(ensure_stage(sizeof(double) * ncell * m.nc));
-        if (ring_ready())
-            HIPCHK(g_ring.h2d(g_stage, h, sizeof(double) * ncell * m.nc, g_stream));
-        else
-            HIPCHK(hipMemcpyAsync(g_stage, h, sizeof(double) * ncell * m.nc, hipMemcpyHostToDevice, g_stream));
-        src = g_stage;
+    pk::PlanesArgs a{};
+    a.soa = const_cast<double *>(soa);
+    a.sv = b->sv;
+    a.nx = b->ng[0];
+    a.ny = b->ng[1];
+    a.nz = b->ng[2];
+    a.sy = b->sy;
+    a.sz = b->sz;
+    a.map[0] = map_u();
+    if (g_mhd) {
+        a.map[1] = map_b();
+        a.map[2] = map_psi();
     }
-    HIPCHK(pk::launch_aos_to_soa(src, m, dst, b->sv, b->ng, b->sy, b->sz, g_stream));
-    HIPCHK(hipStreamSynchronize(g_stream));
-    return PK_OK;
+    return a;
 }
 
-int download_array(Block *b, double *h, const pk::PlaneMap &m, const double *src, bool to_device)
-{
-    const size_t ncell = (size_t)b->ng[0] * b->ng[1] * b->ng[2];
-    if (to_device) {
-        HIPCHK(pk::launch_soa_to_aos(src, b->sv, m, h, b->ng, b->sy, b->sz, g_stream));
-    } else {
-        RCCHK(ensure_stage(sizeof(double) * ncell * m.nc));
-        HIPCHK(pk::launch_soa_to_aos(src, b->sv, m, g_stage, b->ng, b->sy, b->sz, g_stream));
-        if (ring_ready())
-            HIPCHK(g_ring.d2h(h, g_stage, sizeof(double) * ncell * m.nc, g_stream));
-        else
-            HIPCHK(hipMemcpyAsync(h, g_stage, sizeof(double) * ncell * m.nc, hipMemcpyDeviceToHost, g_stream));
-    }
-    HIPCHK(hipStreamSynchronize(g_stream));
-    return PK_OK;
-}
-
+// u, bb, psi (null: left alone) in the reference layout -> planes at dst.
+// dev: the arrays are in device memory, converted by one launch; host arrays
+// go through the staging buffer one after the other.
 int upload_state(Block *b, const double *u, const double *bb, const double *psi, double *dst, bool dev = false)
 {
     b->dt_pending = false;
-    if (u) RCCHK(upload_array(b, u, map_u(), dst, dev));
-    if (g_mhd) {
-        if (bb) RCCHK(upload_array(b, bb, map_b(), dst, dev));
-        if (psi) RCCHK(upload_array(b, psi, map_psi(), dst, dev));
+    const double *h[3] = {u, g_mhd ? bb : nullptr, g_mhd ? psi : nullptr};
+    pk::PlanesArgs a = planes_args(b, dst);
+    if (dev) {
+        for (int k = 0; k < 3; k++) a.aos[k] = const_cast<double *>(h[k]);
+        HIPCHK(pk::launch_planes(true, a, g_stream));
+        HIPCHK(hipStreamSynchronize(g_stream));
+        return PK_OK;
+    }
+    const size_t ncell = (size_t)b->ng[0] * b->ng[1] * b->ng[2];
+    for (int k = 0; k < 3; k++) {
+        if (!h[k]) continue;
+        const size_t bytes = sizeof(double) * ncell * a.map[k].nc;
+        RCCHK(ensure_stage(bytes));
+        if (ring_ready())
+            HIPCHK(g_ring.h2d(g_stage, h[k], bytes, g_stream));
+        else
+            HIPCHK(hipMemcpyAsync(g_stage, h[k], bytes, hipMemcpyHostToDevice, g_stream));
+        pk::PlanesArgs c = a;
+        c.aos[k] = g_stage;
+        HIPCHK(pk::launch_planes(true, c, g_stream));
+        HIPCHK(hipStreamSynchronize(g_stream));
     }
     return PK_OK;
 }
 
 int download_state(Block *b, double *u, double *bb, double *psi, const double *src, bool dev = false)
 {
-    if (u) RCCHK(download_array(b, u, map_u(), src, dev));
-    if (g_mhd) {
-        if (bb) RCCHK(download_array(b, bb, map_b(), src, dev));
-        if (psi) RCCHK(download_array(b, psi, map_psi(), src, dev));
+    double *h[3] = {u, g_mhd ? bb : nullptr, g_mhd ? psi : nullptr};
+    pk::PlanesArgs a = planes_args(b, src);
+    if (dev) {
+        for (int k = 0; k < 3; k++) a.aos[k] = h[k];
+        HIPCHK(pk::launch_planes(false, a, g_stream));
+        HIPCHK(hipStreamSynchronize(g_stream));
+        return PK_OK;
+    }
+    const size_t ncell = (size_t)b->ng[0] * b->ng[1] * b->ng[2];
+    for (int k = 0; k < 3; k++) {
+        if (!h[k]) continue;
+        const size_t bytes = sizeof(double) * ncell * a.map[k].nc;
+        RCCHK(ensure_stage(bytes));
+        pk::PlanesArgs c = a;
+        c.aos[k] = g_stage;
+        HIPCHK(pk::launch_planes(false, c, g_stream));
+        if (ring_ready())
+            HIPCHK(g_ring.d2h(h[k], g_stage, bytes, g_stream));
+        else
+            HIPCHK(hipMemcpyAsync(h[k], g_stage, bytes, hipMemcpyDeviceToHost, g_stream));
+        HIPCHK(hipStreamSynchronize(g_stream));
     }
     return PK_OK;
 }
@@ -1177,17 +1233,18 @@ struct FaceTab {
     size_t wcap = 0;
 };
 
-// Cuts the jobs of t into workgroups of pk::kFaceChunk values and copies the
+// Cuts the jobs of t into workgroups of pk::kFaceCells cells and copies the
 // tables to the device.
 int finish_faces(FaceTab &t)
 {
     t.wgjob.clear();
     for (size_t i = 0; i < t.h.size(); i++) {
         pk::FaceJob &j = t.h[i];
-        const long long vals = (long long)j.ext[0] * j.ext[1] * j.ext[2] * j.nplanes;
-        if (vals >= (1ll << 31)) return fail(PK_EINVAL, "ghost face of %lld values exceeds one exchange job", vals);
+        const long long cells = (long long)j.ext[0] * j.ext[1] * j.ext[2];
+        if (cells * j.nplanes >= (1ll << 31))
+            return fail(PK_EINVAL, "ghost face of %lld values exceeds one exchange job", cells * j.nplanes);
         j.wg0 = (int)t.wgjob.size();
-        const long long nwg = (vals + pk::kFaceChunk - 1) / pk::kFaceChunk;
+        const long long nwg = (cells + pk::kFaceCells - 1) / pk::kFaceCells;
         if ((long long)t.wgjob.size() + nwg >= (1ll << 31)) return fail(PK_EINVAL, "too many ghost faces for one launch");
         t.wgjob.insert(t.wgjob.end(), (size_t)nwg, (int)i);
     }
@@ -1234,10 +1291,15 @@ struct ListState {
     pk::StepScalars *d_step = nullptr;
     pk::StepScalars *h_step = nullptr;  // pinned
     unsigned long long *d_dtslots = nullptr;
-    double *d_dtout = nullptr;
+    double *dtout = nullptr;  // pinned host memory
+    pk::DtArgs *d_dt = nullptr;  // per block and fluid: its timestep (k_dt_list)
+    std::vector<pk::DtArgs> h_dt;
+    size_t dt_cap = 0;
+    long long dt_maxcells = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
-    bool fresh = false;  // ghosts current and d_dtout holds the timestep of the current state
+    bool fresh = false;  // ghosts current and dtout holds the timestep of the current state
+    bool filled = false; // the ghosts were refreshed since the state last changed
     // blocks connected to other blocks (pk_set_neighbour): ghost faces come from
     // the neighbours through an exchange before every sweep instead of the
     // sweep's periodic images
@@ -1251,6 +1313,7 @@ struct ListState {
     FaceTab self[3];
     bool self_built = false;
     bool wrap_any = false;
+    bool wrap_all = false;  // every block's tables do
     bool wrap_stale = false;
 };
 ListState g_list;
@@ -1262,7 +1325,7 @@ struct EnsembleState {
     size_t nblk = 0;
     pk::StepScalars *d_step = nullptr, *h_step = nullptr;  // per block
     unsigned long long *d_dtslots = nullptr;               // per block kEnsSlots slots
-    double *d_dtout = nullptr, *h_dtout = nullptr;         // per block 4 values
+    double *dtout = nullptr;                               // per block 4 values, pinned host memory
     std::vector<double> dt_old;
     bool fresh = false;
     hipGraph_t graph = nullptr;
@@ -1300,6 +1363,7 @@ void list_invalidate()
     (void)settle_ghosts();  // the tables that know which ghosts are old go away
     g_list.built = false;
     g_list.fresh = false;
+    g_list.filled = false;
     destroy_graph();
     ens_free();
 }
@@ -1307,6 +1371,7 @@ void list_invalidate()
 void list_touch()
 {
     g_list.fresh = false;
+    g_list.filled = false;
     g_ens.fresh = false;
 }
 
@@ -1326,8 +1391,7 @@ void ens_free()
     if (g_ens.d_step) (void)hipFree(g_ens.d_step);
     if (g_ens.h_step) (void)hipHostFree(g_ens.h_step);
     if (g_ens.d_dtslots) (void)hipFree(g_ens.d_dtslots);
-    if (g_ens.d_dtout) (void)hipFree(g_ens.d_dtout);
-    if (g_ens.h_dtout) (void)hipHostFree(g_ens.h_dtout);
+    if (g_ens.dtout) (void)hipHostFree(g_ens.dtout);
     if (g_ens.d_jobs) (void)hipFree(g_ens.d_jobs);
     if (g_ens.d_adj) (void)hipFree(g_ens.d_adj);
     if (g_ens.h_adj) (void)hipHostFree(g_ens.h_adj);
@@ -1362,7 +1426,8 @@ void list_free()
     if (g_list.d_step) (void)hipFree(g_list.d_step);
     if (g_list.h_step) (void)hipHostFree(g_list.h_step);
     if (g_list.d_dtslots) (void)hipFree(g_list.d_dtslots);
-    if (g_list.d_dtout) (void)hipFree(g_list.d_dtout);
+    if (g_list.dtout) (void)hipHostFree(g_list.dtout);
+    if (g_list.d_dt) (void)hipFree(g_list.d_dt);
     for (auto &row : g_list.ex)
         for (auto &t : row) {
             if (t.d_jobs) (void)hipFree(t.d_jobs);
@@ -1577,7 +1642,7 @@ int build_faces()
 
 // Face jobs that fill every ghost layer of each block of an unlinked list
 // from the block's own opposite interior (periodic on itself), x then y then
-// z over the full ghosted extents, as k_fill_ghosts does block by block.
+// z over the full ghosted extents, what k_fill_periodic does block by block.
 int build_self_faces()
 {
     g_list.self_built = false;
@@ -1630,7 +1695,10 @@ int exchange_all()
 // ghost refresh of the whole list: periodic images, or the exchange
 int list_fill()
 {
-    if (g_list.linked) return exchange_all();
+    if (g_list.linked) {
+        g_list.filled = true;
+        return exchange_all();
+    }
     if (g_list.self_built) {
         for (int d = 0; d < 3; d++) {
             const FaceTab &t = g_list.self[d];
@@ -1641,6 +1709,7 @@ int list_fill()
         for (Block *b : g_list.blocks) RCCHK(do_fill(b));
     }
     g_list.wrap_stale = false;
+    g_list.filled = true;
     return PK_OK;
 }
 
@@ -1668,6 +1737,7 @@ int list_build()
     if (g_cfg.integration_order != 2) return fail(PK_EINVAL, "the batched list sweep is the fused RK2 sweep");
     g_list.blocks.clear();
     g_list.wrap_any = false;
+    g_list.wrap_all = true;
     g_list.cur0.clear();
     g_list.mdl.clear();
     for (auto &kv : g_blocks) {
@@ -1699,14 +1769,35 @@ int list_build()
             RCCHK(build_tab(g_list.tab[d][f], main, d, f, nt, nullptr, wrap));
             RCCHK(build_tab(g_list.stab[d][f], split, d, f, pk::kStreamListNt, nullptr, wrap));
             for (const LaunchTab *t : {&g_list.tab[d][f], &g_list.stab[d][f]})
-                for (const pk::SweepArgs &a : t->h_args) g_list.wrap_any = g_list.wrap_any || a.images == 2;
+                for (const pk::SweepArgs &a : t->h_args) {
+                    g_list.wrap_any = g_list.wrap_any || a.images == 2;
+                    g_list.wrap_all = g_list.wrap_all && a.images == 2;
+                }
         }
     }
     if (!g_list.d_queue) HIPCHK(hipMalloc((void **)&g_list.d_queue, sizeof(unsigned) * kQueues));
     if (!g_list.d_step) HIPCHK(hipMalloc((void **)&g_list.d_step, sizeof(pk::StepScalars)));
     if (!g_list.h_step) HIPCHK(hipHostMalloc((void **)&g_list.h_step, sizeof(pk::StepScalars), hipHostMallocDefault));
-    if (!g_list.d_dtslots) HIPCHK(hipMalloc((void **)&g_list.d_dtslots, sizeof(unsigned long long) * 4 * kDtSlots));
-    if (!g_list.d_dtout) HIPCHK(hipMalloc((void **)&g_list.d_dtout, sizeof(double) * 4));
+    if (!g_list.d_dtslots) {
+        HIPCHK(hipMalloc((void **)&g_list.d_dtslots, sizeof(unsigned long long) * 4 * kDtSlots));
+        HIPCHK(pk::launch_dtslots_init(g_list.d_dtslots, kDtSlots, g_stream));
+    }
+    if (!g_list.dtout) HIPCHK(hipHostMalloc((void **)&g_list.dtout, sizeof(double) * 4, hipHostMallocDefault));
+    g_list.h_dt.clear();
+    g_list.dt_maxcells = 0;
+    for (Block *b : g_list.blocks) {
+        for (int f = 0; f < g_nfl; f++) g_list.h_dt.push_back(dt_args(b, f));
+        g_list.dt_maxcells = std::max(g_list.dt_maxcells, (long long)b->n[0] * b->n[1] * b->n[2]);
+    }
+    if (g_list.dt_cap < g_list.h_dt.size()) {
+        if (g_list.d_dt) (void)hipFree(g_list.d_dt);
+        g_list.d_dt = nullptr;
+        HIPCHK(hipMalloc((void **)&g_list.d_dt, sizeof(pk::DtArgs) * g_list.h_dt.size()));
+        g_list.dt_cap = g_list.h_dt.size();
+    }
+    HIPCHK(hipMemcpyAsync(g_list.d_dt, g_list.h_dt.data(), sizeof(pk::DtArgs) * g_list.h_dt.size(),
+                          hipMemcpyHostToDevice, g_stream));
+    HIPCHK(hipStreamSynchronize(g_stream));
     g_list.built = true;
     return PK_OK;
 }
@@ -1745,7 +1836,6 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
     if (persistent) HIPCHK(pk::launch_zero_u32(g_list.d_queue, kQueues, g_stream));
     unsigned long long *slots = ens ? g_ens.d_dtslots : g_list.d_dtslots;
     const int nslots = ens ? kEnsSlots : kDtSlots;
-    HIPCHK(pk::launch_dtslots_init(slots, nslots * (ens ? (int)g_ens.nblk : 1), g_stream));
     int q = 0;
     for (size_t k = 0; k < sw.size(); k++) {
         const int d = sw[k].d;
@@ -1808,9 +1898,9 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
         }
     }
     if (ens)
-        HIPCHK(pk::launch_dtslots_final_blocks(g_ens.d_dtslots, kEnsSlots, (int)g_ens.nblk, g_ens.d_dtout, g_stream));
+        HIPCHK(pk::launch_dtslots_final(g_ens.d_dtslots, kEnsSlots, (int)g_ens.nblk, g_ens.dtout, g_stream));
     else
-        HIPCHK(pk::launch_dtslots_final(g_list.d_dtslots, kDtSlots, g_list.d_dtout, g_stream));
+        HIPCHK(pk::launch_dtslots_final(g_list.d_dtslots, kDtSlots, 1, g_list.dtout, g_stream));
     return PK_OK;
 }
 
@@ -1833,31 +1923,35 @@ int ensure_graph()
     return PK_OK;
 }
 
-// Ghost refresh of every block and the list timestep of the current state.
+// The list timestep of the current state, over every block in one launch.
 int list_prepare(double *dt_out, double *c_out)
 {
-    double dt = DBL_MAX, c = 0.0;
-    RCCHK(list_fill());
-    for (Block *b : g_list.blocks) {
-        double dtb, cb;
-        RCCHK(do_timestep(b, &dtb, &cb));
-        if (dtb < dt) dt = dtb;
-        if (cb > c) c = cb;
-    }
-    *dt_out = dt;
-    *c_out = c;
+    HIPCHK(pk::launch_dt_list(g_list.d_dt, (int)g_list.blocks.size(), g_nfl, g_list.dt_maxcells, g_list.d_dtslots,
+                              kDtSlots, 0, g_stream));
+    HIPCHK(pk::launch_dtslots_final(g_list.d_dtslots, kDtSlots, 1, g_list.dtout, g_stream));
+    HIPCHK(hipStreamSynchronize(g_stream));
+    combine_dt(g_list.dtout, 1, dt_out, c_out);
     return PK_OK;
 }
 
 int list_dt(double *dt_out, double *c_out)
 {
     if (g_list.fresh) {
-        HIPCHK(hipMemcpyAsync(g_pinned, g_list.d_dtout, 4 * sizeof(double), hipMemcpyDeviceToHost, g_stream));
         HIPCHK(hipStreamSynchronize(g_stream));
-        combine_dt(g_pinned, 1, dt_out, c_out);
+        combine_dt(g_list.dtout, 1, dt_out, c_out);
         return PK_OK;
     }
     return list_prepare(dt_out, c_out);
+}
+
+// Refreshes the ghosts a step of the list reads before its sweeps write any:
+// none in the persistent modes of a linked list (every sweep follows an
+// exchange) or where every block's sweeps read the periodic interior.
+int list_fill_for_step(int mode)
+{
+    if (g_list.fresh || g_list.filled) return PK_OK;
+    if (mode != PK_BATCH_PER_BLOCK && (g_list.linked || g_list.wrap_all)) return PK_OK;
+    return list_fill();
 }
 
 int list_step(int mode, double dt)
@@ -1883,6 +1977,7 @@ int list_step(int mode, double dt)
         b->dt_pending = false;
     }
     g_list.fresh = true;
+    g_list.filled = false;
     g_list.ghosts_stale = g_list.linked;
     if (g_list.wrap_any && mode != PK_BATCH_PER_BLOCK) g_list.wrap_stale = true;
     g_ens.fresh = false;
@@ -1910,8 +2005,8 @@ int ens_build()
     HIPCHK(hipMalloc((void **)&g_ens.d_step, sizeof(pk::StepScalars) * n));
     HIPCHK(hipHostMalloc((void **)&g_ens.h_step, sizeof(pk::StepScalars) * n, hipHostMallocDefault));
     HIPCHK(hipMalloc((void **)&g_ens.d_dtslots, sizeof(unsigned long long) * 4 * kEnsSlots * n));
-    HIPCHK(hipMalloc((void **)&g_ens.d_dtout, sizeof(double) * 4 * n));
-    HIPCHK(hipHostMalloc((void **)&g_ens.h_dtout, sizeof(double) * 4 * n, hipHostMallocDefault));
+    HIPCHK(pk::launch_dtslots_init(g_ens.d_dtslots, kEnsSlots * (int)n, g_stream));
+    HIPCHK(hipHostMalloc((void **)&g_ens.dtout, sizeof(double) * 4 * n, hipHostMallocDefault));
     HIPCHK(hipMalloc((void **)&g_ens.d_jobs, sizeof(pk::CopyJob) * n));
     HIPCHK(hipMalloc((void **)&g_ens.d_queue, sizeof(unsigned) * pk::kListQueues));
     g_ens.h_jobs.resize(n);
@@ -1943,20 +2038,16 @@ int ens_dt_raw(std::vector<double> &dt)
 {
     const size_t n = g_ens.nblk;
     dt.assign(n, 0.0);
-    if (g_ens.fresh) {
-        HIPCHK(hipMemcpyAsync(g_ens.h_dtout, g_ens.d_dtout, sizeof(double) * 4 * n, hipMemcpyDeviceToHost, g_stream));
-        HIPCHK(hipStreamSynchronize(g_stream));
-        for (size_t i = 0; i < n; i++) {
-            double c;
-            combine_dt(g_ens.h_dtout + 4 * i, 1, &dt[i], &c);
-        }
-        return PK_OK;
+    if (!g_ens.fresh) {
+        if (!g_list.filled) RCCHK(list_fill());
+        HIPCHK(pk::launch_dt_list(g_list.d_dt, (int)n, g_nfl, g_list.dt_maxcells, g_ens.d_dtslots, kEnsSlots, 1,
+                                  g_stream));
+        HIPCHK(pk::launch_dtslots_final(g_ens.d_dtslots, kEnsSlots, (int)n, g_ens.dtout, g_stream));
     }
+    HIPCHK(hipStreamSynchronize(g_stream));
     for (size_t i = 0; i < n; i++) {
-        Block *b = g_list.blocks[i];
-        RCCHK(do_fill(b));
         double c;
-        RCCHK(do_timestep(b, &dt[i], &c));
+        combine_dt(g_ens.dtout + 4 * i, 1, &dt[i], &c);
     }
     return PK_OK;
 }
@@ -2034,26 +2125,6 @@ int ens_adj_build()
 }
 
 // ---- the unsplit Riemann driver (RIEMANN_UNSPLIT) ----
-
-// periodic ghost refresh of one of the block's two buffers
-int fill_buffer(Block *b, int i)
-{
-    pk::GhostArgs a{};
-    a.u = state(b, i);
-    a.sv = b->sv;
-    a.sy = b->sy;
-    a.sz = b->sz;
-    for (int d = 0; d < 3; d++) {
-        a.ng[d] = b->ng[d];
-        a.g[d] = b->g[d];
-        a.n[d] = b->n[d];
-    }
-    a.plane0 = 0;
-    a.nplanes = g_nplanes;
-    for (int d = 0; d < 3; d++)
-        if (b->g[d] > 0) HIPCHK(pk::launch_fill_ghosts(d, a, g_stream));
-    return PK_OK;
-}
 
 // One RK stage of unsplit_sweep on a periodic block (solve_cg_ub / solve_cg_u,
 // then update_boundaries of the stage's arrays, unsplit_sweeps.F90:126-190):
@@ -2428,9 +2499,9 @@ int pk_init(const pk_config *cfg)
     HIPCHK(hipGetDeviceCount(&ndev));
     if (ndev < 1) return fail(PK_EHIP, "no HIP device");
     if (g_init) {
+        list_free();  // waits for the queued work
         for (auto &kv : g_blocks) free_block(kv.second);
         g_blocks.clear();
-        list_free();
     }
     if (!g_stream) HIPCHK(hipStreamCreateWithFlags(&g_stream, hipStreamNonBlocking));
     if (!g_pinned) HIPCHK(hipHostMalloc((void **)&g_pinned, 16 * sizeof(double), hipHostMallocDefault));
@@ -2676,7 +2747,7 @@ int pk_sweep_noalloc(const double *src, double *dst, int64_t sv, int32_t sy, int
         HIPCHK(sweep_kernel(ddim, g_fmag[f], true, a, st));
     }
     if (report) {
-        HIPCHK(pk::launch_dtslots_final(s, kNaSlots, report, st));
+        HIPCHK(pk::launch_dtslots_final(s, kNaSlots, 1, report, st));
         hipLaunchKernelGGL(k_noalloc_report, dim3(1), dim3(64), 0, st, s, g_nfl, report);
         HIPCHK(hipGetLastError());
     }
@@ -2887,7 +2958,8 @@ int pk_run(int64_t cg_id, int32_t nsteps, double *t_out, double *dt_out)
     RCCHK(solo(b));
     if (nsteps < 0) return fail(PK_EINVAL, "nsteps < 0");
     list_touch();
-    RCCHK(do_fill(b));
+    // sweeps that read the periodic interior need no ghosts; they are refreshed after the steps
+    if (nsteps == 0 || g_cfg.integration_order != 2 || !stream_all_dirs(b)) RCCHK(do_fill(b));
     StepLoop L;
     L.blocks = {b};
     L.timestep = [b](double *dt, double *c) { return do_timestep(b, dt, c); };
@@ -3129,6 +3201,7 @@ int pk_timestep_all(double *dt_out, double *c_out)
     if (!g_init) return fail(PK_ESTATE, "pk_init has not been called");
     if (!dt_out || !c_out) return fail(PK_EINVAL, "null output");
     RCCHK(list_build());
+    if (!g_list.fresh && !g_list.filled) RCCHK(list_fill());
     return list_dt(dt_out, c_out);
 }
 
@@ -3138,7 +3211,7 @@ int pk_fluid_update_all(int32_t mode, double dt)
     RCCHK(check_mode(mode));
     if (!(dt > 0.0)) return fail(PK_EINVAL, "dt must be positive");
     RCCHK(list_build());
-    if (!g_list.fresh) RCCHK(list_fill());
+    RCCHK(list_fill_for_step(mode));
     return list_step(mode, dt);  // ghosts left old are refilled when something reads them
 }
 
@@ -3153,7 +3226,7 @@ int pk_run_all(int32_t mode, int32_t nsteps, double *t_out, double *dt_out)
     L.timestep = [](double *dt, double *c) { return list_dt(dt, c); };
     L.update = [mode](double dt) {
         // a redone step starts from restored states: ghosts and dt are recomputed
-        if (!g_list.fresh) RCCHK(list_fill());
+        RCCHK(list_fill_for_step(mode));
         return list_step(mode, dt);
     };
     return run_loop(L, nsteps, t_out, dt_out, &g_last_redone);  // ghosts left old are refilled when read
@@ -3452,11 +3525,12 @@ int pk_adjoint_set(int64_t cg_id, const double *lam_u, const double *lam_b, cons
     RCCHK(get_block(cg_id, &b));
     RCCHK(adj_check(b));
     if (!lam_u || (g_mhd && (!lam_b || !lam_psi))) return fail(PK_EINVAL, "missing adjoint array");
-    double *dst = b->lam[b->lcur];
-    HIPCHK(hipMemsetAsync(dst, 0, state_bytes(b), g_stream));
-    RCCHK(upload_state(b, lam_u, lam_b, lam_psi, dst + b->xo, true));
     // the ghost cells are periodic copies of interior cells
-    HIPCHK(pk::launch_fold_ghosts(dst + b->xo, b->sv, b->sy, b->sz, b->ng, b->g, b->n, g_nplanes, g_stream));
+    pk::PlanesArgs a = planes_args(b, b->lam[b->lcur] + b->xo);
+    const double *h[3] = {lam_u, g_mhd ? lam_b : nullptr, g_mhd ? lam_psi : nullptr};
+    for (int k = 0; k < 3; k++) a.aos[k] = const_cast<double *>(h[k]);
+    HIPCHK(pk::launch_planes_fold(a, b->g, g_stream));
+    HIPCHK(hipStreamSynchronize(g_stream));
     return PK_OK;
 }
 
@@ -3510,7 +3584,7 @@ int pk_fluid_update_record(int64_t cg_id, int32_t slot0, double dt)
     b->cur = 1 - b->cur;
     b->uh = -1;
     b->dt_pending = false;
-    HIPCHK(pk::launch_dtslots_final(b->d_dtslots, kDtSlots, b->d_dtout, g_stream));
+    HIPCHK(pk::launch_dtslots_final(b->d_dtslots, kDtSlots, 1, b->dtout, g_stream));
     b->dt_pending = true;
     return PK_OK;
 }
@@ -3569,12 +3643,11 @@ int pk_timestep_adjoint(int64_t cg_id, int32_t slot, double dt_bar)
     a.magnetized = g_mhd ? 1 : 0;
     a.gam = g_cfg.fluid[0].gamma;
     a.gam_1 = g_cfg.fluid[0].gamma - 1.0;
-    HIPCHK(pk::launch_dt(a, g_part, b->d_dtout, g_stream));
-    HIPCHK(hipMemcpyAsync(g_pinned, b->d_dtout, 4 * sizeof(double), hipMemcpyDeviceToHost, g_stream));
+    HIPCHK(pk::launch_dt(a, g_part, b->dtout, g_stream));
     HIPCHK(hipStreamSynchronize(g_stream));
-    double mn = g_pinned[0];
-    if (g_pinned[1] < mn) mn = g_pinned[1];
-    if (g_pinned[2] < mn) mn = g_pinned[2];
+    double mn = b->dtout[0];
+    if (b->dtout[1] < mn) mn = b->dtout[1];
+    if (b->dtout[2] < mn) mn = b->dtout[2];
     b->dt_pending = false;
     pk::DtAdjArgs q{};
     q.u = a.u;
@@ -3633,6 +3706,7 @@ int pk_ensemble_step(int32_t mode, int32_t first, double *dt_out, int32_t *cappe
         b->dt_pending = false;
     }
     g_list.fresh = false;
+    g_list.filled = false;
     g_ens.fresh = true;
     return PK_OK;
 }

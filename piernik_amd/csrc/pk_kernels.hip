@@ -20,8 +20,6 @@
 
 namespace PK_KNS {
 
-using pk::DtArgs;
-using pk::GhostArgs;
 using pk::ListArgs;
 using pk::StepScalars;
 using pk::SweepArgs;
@@ -580,323 +578,6 @@ __global__ __launch_bounds__(512) void k_sweep_list(const ListArgs L)
     }
 }
 
-__global__ void k_fill_items(const unsigned *__restrict__ first, int nblocks, unsigned *__restrict__ items)
-{
-    // one workgroup per block writes its range of the item table
-    const int b = blockIdx.x;
-    if (b >= nblocks) return;
-    for (unsigned i = first[b] + threadIdx.x; i < first[b + 1]; i += blockDim.x) items[i] = (unsigned)b;
-}
-
-// one workgroup per block: that block's dt slots -> its four results
-__global__ __launch_bounds__(256) void k_dtslots_final_blocks(const unsigned long long *__restrict__ slots, int nslots,
-                                                              double *__restrict__ out)
-{
-    __shared__ double red[4][256];
-    const int t = threadIdx.x;
-    const unsigned long long *s = slots + 4ll * nslots * blockIdx.x;
-    double m0 = 1.7976931348623157e308, m1 = m0, m2 = m0, cmax = 0.0;
-    for (int i = t; i < nslots; i += 256) {
-        m0 = fmn(m0, __longlong_as_double((long long)s[4 * i + 0]));
-        m1 = fmn(m1, __longlong_as_double((long long)s[4 * i + 1]));
-        m2 = fmn(m2, __longlong_as_double((long long)s[4 * i + 2]));
-        cmax = fmx(cmax, __longlong_as_double((long long)s[4 * i + 3]));
-    }
-    red[0][t] = m0;
-    red[1][t] = m1;
-    red[2][t] = m2;
-    red[3][t] = cmax;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w) {
-            red[0][t] = fmn(red[0][t], red[0][t + w]);
-            red[1][t] = fmn(red[1][t], red[1][t + w]);
-            red[2][t] = fmn(red[2][t], red[2][t + w]);
-            red[3][t] = fmx(red[3][t], red[3][t + w]);
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-        double *o = out + 4 * blockIdx.x;
-        o[0] = red[0][0];
-        o[1] = red[1][0];
-        o[2] = red[2][0];
-        o[3] = red[3][0];
-    }
-}
-
-// a batch of device-to-device copies: workgroups stride over the jobs
-__global__ __launch_bounds__(256) void k_copy_blocks(const pk::CopyJob *__restrict__ jobs, int njobs)
-{
-    for (int j = blockIdx.y; j < njobs; j += gridDim.y) {
-        const pk::CopyJob c = jobs[j];
-        for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < c.n;
-             i += (long long)gridDim.x * blockDim.x)
-            c.dst[i] = c.src[i];
-    }
-}
-
-// Ghost exchange between blocks (internal_boundaries_local,
-// cg_list_bnd.F90:269-322): one job per face, cut into chunks of kFaceChunk
-// values, one workgroup per chunk (wgjob names its job); values run x
-// fastest, so rows of y and z faces are coalesced.
-__global__ __launch_bounds__(256) void k_exchange_faces(const pk::FaceJob *__restrict__ jobs,
-                                                      const int *__restrict__ wgjob)
-{
-    const pk::FaceJob &J = jobs[wgjob[blockIdx.x]];
-    const int e0 = J.ext[0], e01 = e0 * J.ext[1], ncell = e01 * J.ext[2];
-    const int total = ncell * J.nplanes;
-    const int base = ((int)blockIdx.x - J.wg0) * pk::kFaceChunk;
-    const int end = min(base + pk::kFaceChunk, total);
-    for (int e = base + (int)threadIdx.x; e < end; e += 256) {
-        const int v = e / ncell, c = e - v * ncell;
-        const int k = c / e01, r = c - k * e01;
-        const int j = r / e0, i = r - j * e0;
-        const long long s = v * J.ssv + (J.sorg[0] + i) + (long long)J.ssy * (J.sorg[1] + j) +
-                            (long long)J.ssz * (J.sorg[2] + k);
-        const long long d = v * J.dsv + (J.dorg[0] + i) + (long long)J.dsy * (J.dorg[1] + j) +
-                            (long long)J.dsz * (J.dorg[2] + k);
-        J.dst[d] = J.src[s];
-    }
-}
-
-__global__ void k_zero_u32(unsigned *p, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = 0u;
-}
-
-// Periodic refresh of the ghost layers along direction DIR over the full
-// extent of the other two directions (run x, then y, then z for corners).
-template <int DIR>
-__global__ void k_fill_ghosts(const GhostArgs a)
-{
-    const long long tid = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    constexpr int d1 = (DIR == 0) ? 1 : 0;
-    constexpr int d2 = (DIR == 2) ? 1 : 2;
-    const int g = a.g[DIR];
-    const long long per_plane = (long long)(2 * g) * a.ng[d1] * a.ng[d2];
-    if (tid >= per_plane * a.nplanes) return;
-    const int v = (int)(tid / per_plane);
-    long long r = tid % per_plane;
-    // fastest index: x when DIR != 0, else the ghost layer index
-    int xyz[3];
-    int gi;
-    if (DIR == 0) {
-        gi = (int)(r % (2 * g));
-        r /= (2 * g);
-        xyz[d1] = (int)(r % a.ng[d1]);
-        xyz[d2] = (int)(r / a.ng[d1]);
-    } else {
-        xyz[d1] = (int)(r % a.ng[d1]);
-        r /= a.ng[d1];
-        gi = (int)(r % (2 * g));
-        xyz[d2] = (int)(r / (2 * g));
-    }
-    const int n = a.n[DIR];
-    const int dstc = (gi < g) ? gi : n + gi;          // low ghosts 0..g-1, high ghosts g+n..
-    const int srcc = (gi < g) ? gi + n : gi;          // periodic images inside the interior
-    int s3[3] = {xyz[0], xyz[1], xyz[2]};
-    xyz[DIR] = dstc;
-    s3[DIR] = srcc;
-    const long long di = (long long)xyz[0] + (long long)a.sy * xyz[1] + (long long)a.sz * xyz[2];
-    const long long si = (long long)s3[0] + (long long)a.sy * s3[1] + (long long)a.sz * s3[2];
-    double *base = a.u + (long long)(a.plane0 + v) * a.sv;
-    base[di] = base[si];
-}
-
-__global__ void k_scale(double *__restrict__ x, long long n, double fac)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) x[i] = x[i] * fac;
-}
-
-// timestep_fluid (timestep.F90:460-490) with ion_cs / neu_cs
-// (initionized.F90:137-141, initneutral.F90:102-105): per-workgroup partial
-// min of dl_d/c_d for d = x, y, z and max of c.
-template <bool MAG>
-__global__ __launch_bounds__(256) void k_dt_partial(const DtArgs a, double *__restrict__ part)
-{
-    __shared__ double red[4][256];
-    const int t = threadIdx.x;
-    const long long ncell = (long long)a.n[0] * a.n[1] * a.n[2];
-    double m0 = 1.7976931348623157e308, m1 = m0, m2 = m0, cmax = 1.17549435082228750797e-38;
-    for (long long c = (long long)blockIdx.x * blockDim.x + t; c < ncell; c += (long long)gridDim.x * blockDim.x) {
-        const int i = (int)(c % a.n[0]);
-        const long long r = c / a.n[0];
-        const int j = (int)(r % a.n[1]);
-        const int k = (int)(r / a.n[1]);
-        const long long idx = (long long)(i + a.g[0]) + (long long)a.sy * (j + a.g[1]) + (long long)a.sz * (k + a.g[2]);
-        const double *u = a.u + (long long)a.plane0 * a.sv + idx;
-        const double d = u[0], mx = u[a.sv], my = u[2 * a.sv], mz = u[3 * a.sv], e = u[4 * a.sv];
-        double v0 = 0.0, v1 = 0.0, v2 = 0.0;
-        if (d > 0.0) {
-            v0 = fabs(qdiv(mx, d));
-            v1 = fabs(qdiv(my, d));
-            v2 = fabs(qdiv(mz, d));
-        }
-        const double ek = qdiv(0.5 * ((mx * mx + my * my) + mz * mz), d);
-        double cs;
-        if (MAG) {
-            const double *b = a.u + (long long)a.bplane * a.sv + idx;
-            const double bx = b[0], by = b[a.sv], bz = b[2 * a.sv];
-            const double pmag = 0.5 * ((bx * bx + by * by) + bz * bz);
-            const double ps = (e - ek) * a.gam_1 + (2.0 - a.gam) * pmag;
-            const double pr = ps - pmag;
-            cs = qsqrt(fabs(qdiv(2.0 * pmag + a.gam * pr, d)));
-        } else {
-            const double pr = (e - ek) * a.gam_1;
-            cs = qsqrt(fabs(qdiv(a.gam * pr, d)));
-        }
-        const double small = 1.17549435082228750797e-38;
-        const double c0 = fmx(v0 + cs, small), c1 = fmx(v1 + cs, small), c2 = fmx(v2 + cs, small);
-        cmax = fmx(cmax, fmx(fmx(c0, c1), c2));
-        if (a.has_dir[0]) m0 = fmn(m0, qdiv(a.dl[0], c0));
-        if (a.has_dir[1]) m1 = fmn(m1, qdiv(a.dl[1], c1));
-        if (a.has_dir[2]) m2 = fmn(m2, qdiv(a.dl[2], c2));
-    }
-    red[0][t] = m0;
-    red[1][t] = m1;
-    red[2][t] = m2;
-    red[3][t] = cmax;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w) {
-            red[0][t] = fmn(red[0][t], red[0][t + w]);
-            red[1][t] = fmn(red[1][t], red[1][t + w]);
-            red[2][t] = fmn(red[2][t], red[2][t + w]);
-            red[3][t] = fmx(red[3][t], red[3][t + w]);
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-        part[4 * blockIdx.x + 0] = red[0][0];
-        part[4 * blockIdx.x + 1] = red[1][0];
-        part[4 * blockIdx.x + 2] = red[2][0];
-        part[4 * blockIdx.x + 3] = red[3][0];
-    }
-}
-
-__global__ __launch_bounds__(256) void k_dt_final(const double *__restrict__ part, int nparts,
-                                                  double *__restrict__ out)
-{
-    __shared__ double red[4][256];
-    const int t = threadIdx.x;
-    double m0 = 1.7976931348623157e308, m1 = m0, m2 = m0, cmax = 0.0;
-    for (int i = t; i < nparts; i += 256) {
-        m0 = fmn(m0, part[4 * i + 0]);
-        m1 = fmn(m1, part[4 * i + 1]);
-        m2 = fmn(m2, part[4 * i + 2]);
-        cmax = fmx(cmax, part[4 * i + 3]);
-    }
-    red[0][t] = m0;
-    red[1][t] = m1;
-    red[2][t] = m2;
-    red[3][t] = cmax;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w) {
-            red[0][t] = fmn(red[0][t], red[0][t + w]);
-            red[1][t] = fmn(red[1][t], red[1][t + w]);
-            red[2][t] = fmn(red[2][t], red[2][t + w]);
-            red[3][t] = fmx(red[3][t], red[3][t + w]);
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-        out[0] = red[0][0];
-        out[1] = red[1][0];
-        out[2] = red[2][0];
-        out[3] = red[3][0];
-    }
-}
-
-// Fortran AoS block (nc, nxg, nyg, nzg) <-> device planes m.planes[c].
-__global__ void k_aos_to_soa(const double *__restrict__ aos, const pk::PlaneMap m, double *__restrict__ soa,
-                             long long sv, int nx, int ny, int nz, int sy, int sz)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long ncell = (long long)nx * ny * nz;
-    if (i >= ncell) return;
-    const int x = (int)(i % nx);
-    const long long r = i / nx;
-    const int y = (int)(r % ny);
-    const int z = (int)(r / ny);
-    const long long di = (long long)x + (long long)sy * y + (long long)sz * z;
-    for (int c = 0; c < m.nc; c++) soa[(long long)m.planes[c] * sv + di] = aos[i * m.nc + c];
-}
-
-__global__ void k_soa_to_aos(const double *__restrict__ soa, long long sv, const pk::PlaneMap m,
-                             double *__restrict__ aos, int nx, int ny, int nz, int sy, int sz)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long ncell = (long long)nx * ny * nz;
-    if (i >= ncell) return;
-    const int x = (int)(i % nx);
-    const long long r = i / nx;
-    const int y = (int)(r % ny);
-    const int z = (int)(r / ny);
-    const long long si = (long long)x + (long long)sy * y + (long long)sz * z;
-    for (int c = 0; c < m.nc; c++) aos[i * m.nc + c] = soa[(long long)m.planes[c] * sv + si];
-}
-
-__global__ void k_dtslots_init(unsigned long long *slots, int nslots)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nslots) return;
-    const unsigned long long huge = (unsigned long long)__double_as_longlong(1.7976931348623157e308);
-    slots[4 * i + 0] = huge;
-    slots[4 * i + 1] = huge;
-    slots[4 * i + 2] = huge;
-    slots[4 * i + 3] = 0ull;
-}
-
-__global__ __launch_bounds__(256) void k_dtslots_final(const unsigned long long *__restrict__ slots, int nslots,
-                                                       double *__restrict__ out)
-{
-    __shared__ double red[4][256];
-    const int t = threadIdx.x;
-    double m0 = 1.7976931348623157e308, m1 = m0, m2 = m0, cmax = 0.0;
-    for (int i = t; i < nslots; i += 256) {
-        m0 = fmn(m0, __longlong_as_double((long long)slots[4 * i + 0]));
-        m1 = fmn(m1, __longlong_as_double((long long)slots[4 * i + 1]));
-        m2 = fmn(m2, __longlong_as_double((long long)slots[4 * i + 2]));
-        cmax = fmx(cmax, __longlong_as_double((long long)slots[4 * i + 3]));
-    }
-    red[0][t] = m0;
-    red[1][t] = m1;
-    red[2][t] = m2;
-    red[3][t] = cmax;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (t < w) {
-            red[0][t] = fmn(red[0][t], red[0][t + w]);
-            red[1][t] = fmn(red[1][t], red[1][t + w]);
-            red[2][t] = fmn(red[2][t], red[2][t + w]);
-            red[3][t] = fmx(red[3][t], red[3][t + w]);
-        }
-        __syncthreads();
-    }
-    if (t == 0) {
-        out[0] = red[0][0];
-        out[1] = red[1][0];
-        out[2] = red[2][0];
-        out[3] = red[3][0];
-    }
-}
-
-hipError_t launch_dtslots_init(unsigned long long *slots, int nslots, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_dtslots_init, dim3((unsigned)((nslots + 255) / 256)), dim3(256), 0, st, slots, nslots);
-    return hipGetLastError();
-}
-
-hipError_t launch_dtslots_final(const unsigned long long *slots, int nslots, double *out, hipStream_t st)
-{
-    hipLaunchKernelGGL(k_dtslots_final, dim3(1), dim3(256), 0, st, slots, nslots, out);
-    return hipGetLastError();
-}
-
 // ------------------------------------------------------------ launchers ----
 
 template <int DIR, class P, bool FUSED, int LIM>
@@ -1146,100 +827,5 @@ int sweep_list_resident(int dir, bool mhd, int lim, int limb, int nt)
     return r;
 }
 
-size_t sweep_lds_bytes(bool mhd, int TP, int TS) { return sizeof(double) * 2 * (mhd ? 9 : 5) * TP * TS; }
-
-hipError_t launch_fill_ghosts(int dir, const GhostArgs &a, hipStream_t st)
-{
-    const int d1 = (dir == 0) ? 1 : 0, d2 = (dir == 2) ? 1 : 2;
-    const long long total = (long long)(2 * a.g[dir]) * a.ng[d1] * a.ng[d2] * a.nplanes;
-    if (total == 0) return hipSuccess;
-    const unsigned blocks = (unsigned)((total + 255) / 256);
-    if (dir == 0) hipLaunchKernelGGL(k_fill_ghosts<0>, dim3(blocks), dim3(256), 0, st, a);
-    if (dir == 1) hipLaunchKernelGGL(k_fill_ghosts<1>, dim3(blocks), dim3(256), 0, st, a);
-    if (dir == 2) hipLaunchKernelGGL(k_fill_ghosts<2>, dim3(blocks), dim3(256), 0, st, a);
-    return hipGetLastError();
-}
-
-hipError_t launch_scale(double *x, long long n, double fac, hipStream_t st)
-{
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_scale, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, n, fac);
-    return hipGetLastError();
-}
-
-int dt_partial_blocks(const DtArgs &a)
-{
-    const long long ncell = (long long)a.n[0] * a.n[1] * a.n[2];
-    long long b = (ncell + 255) / 256;
-    if (b > 2048) b = 2048;
-    if (b < 1) b = 1;
-    return (int)b;
-}
-
-hipError_t launch_dt(const DtArgs &a, double *part, double *out, hipStream_t st)
-{
-    const int nb = PK_KNS::dt_partial_blocks(a);
-    if (a.magnetized)
-        hipLaunchKernelGGL(k_dt_partial<true>, dim3(nb), dim3(256), 0, st, a, part);
-    else
-        hipLaunchKernelGGL(k_dt_partial<false>, dim3(nb), dim3(256), 0, st, a, part);
-    hipLaunchKernelGGL(k_dt_final, dim3(1), dim3(256), 0, st, part, nb, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_aos_to_soa(const double *aos, const pk::PlaneMap &m, double *soa, long long sv, const int ng[3],
-                             int sy, int sz, hipStream_t st)
-{
-    const long long n = (long long)ng[0] * ng[1] * ng[2];
-    hipLaunchKernelGGL(k_aos_to_soa, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, aos, m, soa, sv, ng[0],
-                       ng[1], ng[2], sy, sz);
-    return hipGetLastError();
-}
-
-hipError_t launch_soa_to_aos(const double *soa, long long sv, const pk::PlaneMap &m, double *aos, const int ng[3],
-                             int sy, int sz, hipStream_t st)
-{
-    const long long n = (long long)ng[0] * ng[1] * ng[2];
-    hipLaunchKernelGGL(k_soa_to_aos, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, soa, sv, m, aos, ng[0],
-                       ng[1], ng[2], sy, sz);
-    return hipGetLastError();
-}
-
-hipError_t launch_fill_items(const unsigned *first, int nblocks, unsigned *items, hipStream_t st)
-{
-    if (nblocks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_fill_items, dim3((unsigned)nblocks), dim3(256), 0, st, first, nblocks, items);
-    return hipGetLastError();
-}
-
-hipError_t launch_dtslots_final_blocks(const unsigned long long *slots, int nslots, int nblocks, double *out,
-                                       hipStream_t st)
-{
-    if (nblocks <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_dtslots_final_blocks, dim3((unsigned)nblocks), dim3(256), 0, st, slots, nslots, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_exchange_faces(const pk::FaceJob *jobs, const int *wgjob, int nwg, hipStream_t st)
-{
-    if (nwg <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_exchange_faces, dim3((unsigned)nwg), dim3(256), 0, st, jobs, wgjob);
-    return hipGetLastError();
-}
-
-hipError_t launch_copy_blocks(const pk::CopyJob *jobs, int njobs, hipStream_t st)
-{
-    if (njobs <= 0) return hipSuccess;
-    const unsigned gy = (unsigned)(njobs < 65535 ? njobs : 65535);
-    hipLaunchKernelGGL(k_copy_blocks, dim3(256, gy), dim3(256), 0, st, jobs, njobs);
-    return hipGetLastError();
-}
-
-hipError_t launch_zero_u32(unsigned *p, int n, hipStream_t st)
-{
-    if (n <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_zero_u32, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, p, n);
-    return hipGetLastError();
-}
 
 }  // namespace PK_KNS

@@ -129,10 +129,21 @@ struct FaceJob {
     int ssy, ssz, dsy, dsz;
     int sorg[3], dorg[3], ext[3];
     int nplanes;
-    int wg0;             // the job's first workgroup in its launch (kFaceChunk values each)
+    int wg0;             // the job's first workgroup in its launch (kFaceCells cells each)
 };
-// Values one workgroup of k_exchange_faces copies.
-constexpr int kFaceChunk = 4096;
+// Cells one workgroup of k_exchange_faces copies (every plane of each).
+constexpr int kFaceCells = 512;
+
+// Arrays of the reference layout and the planes of a state (k_planes):
+// aos[k] holds map[k].nc components per cell, null: not converted.
+struct PlanesArgs {
+    double *aos[3];
+    PlaneMap map[3];
+    double *soa;
+    long long sv;
+    int nx, ny, nz;  // ghosted extents
+    int sy, sz;
+};
 
 hipError_t launch_sweep(int dir, bool mhd, bool fused, const SweepArgs &a, hipStream_t st);
 // Workgroup size that selects the stream form of the persistent list sweep
@@ -152,25 +163,28 @@ hipError_t launch_sweep_list(int dir, bool mhd, int lim, int limb, const ListArg
                              hipStream_t st);
 int sweep_list_resident(int dir, bool mhd, int lim, int limb, int nt);
 hipError_t launch_fill_items(const unsigned *first, int nblocks, unsigned *items, hipStream_t st);
-// per-block dt slots -> per-block (min dl_x/c, min dl_y/c, min dl_z/c, max c)
-hipError_t launch_dtslots_final_blocks(const unsigned long long *slots, int nslots, int nblocks, double *out,
-                                       hipStream_t st);
 hipError_t launch_copy_blocks(const CopyJob *jobs, int njobs, hipStream_t st);
-// the faces of one exchange; maxvals = the largest ext product times nplanes
-// jobs[wgjob[w]] is the job of workgroup w (nwg workgroups)
+// the faces of one exchange: jobs[wgjob[w]] is the job of workgroup w (nwg workgroups)
 hipError_t launch_exchange_faces(const FaceJob *jobs, const int *wgjob, int nwg, hipStream_t st);
 hipError_t launch_zero_u32(unsigned *p, int n, hipStream_t st);
-size_t sweep_lds_bytes(bool mhd, int TP, int TS);
-hipError_t launch_fill_ghosts(int dir, const GhostArgs &a, hipStream_t st);
+// every ghost cell of a block periodic on itself, in one launch
+hipError_t launch_fill_periodic(const GhostArgs &a, hipStream_t st);
 hipError_t launch_scale(double *x, long long n, double fac, hipStream_t st);
-int dt_partial_blocks(const DtArgs &a);
+// timestep slots: cleared once, and again by each launch_dtslots_final, which
+// reduces nsets sets of nslots slots to (min dl_x/c, min dl_y/c, min dl_z/c,
+// max c) each, written to device or pinned host memory
 hipError_t launch_dtslots_init(unsigned long long *slots, int nslots, hipStream_t st);
-hipError_t launch_dtslots_final(const unsigned long long *slots, int nslots, double *out, hipStream_t st);
+hipError_t launch_dtslots_final(unsigned long long *slots, int nslots, int nsets, double *out, hipStream_t st);
 hipError_t launch_dt(const DtArgs &a, double *part, double *out, hipStream_t st);
-hipError_t launch_aos_to_soa(const double *aos, const PlaneMap &m, double *soa, long long sv, const int ng[3],
-                             int sy, int sz, hipStream_t st);
-hipError_t launch_soa_to_aos(const double *soa, long long sv, const PlaneMap &m, double *aos, const int ng[3],
-                             int sy, int sz, hipStream_t st);
+// timestep_fluid of nblocks blocks of nfl fluids (jobs: device table, fluids
+// of a block together) into the slots; maxcells: cells of the largest block
+hipError_t launch_dt_list(const DtArgs *jobs, int nblocks, int nfl, long long maxcells, unsigned long long *slots,
+                          int nslots, int per_block, hipStream_t st);
+// reference arrays -> planes (in) or planes -> reference arrays
+hipError_t launch_planes(bool in, const PlanesArgs &a, hipStream_t st);
+// reference arrays -> planes with the ghosts' values added to the interior
+// cells they copy (g: ghost layers) and the ghosts cleared
+hipError_t launch_planes_fold(const PlanesArgs &a, const int g[3], hipStream_t st);
 
 }  // namespace pk
 
