@@ -432,44 +432,22 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     adjoint_tile<DIR, P, LIM>(a, bid, lds);
 }
 
-// Persistent adjoint sweep over a block list (independent instances): as
-// k_sweep_list, tiles from device queues, per-block arguments from a table.
-// The items are cut into kListQueues contiguous ranges with a counter each;
-// a workgroup starts with the range of its XCD (workgroup i runs on XCD
-// i % 8), so tiles that share cache lines share an L2, and goes on to the
-// others when it is empty.  A workgroup leaves after one fetch past the end
-// of every range.
+// Adjoint sweep over a block list (independent instances): as k_sweep_list, a
+// tile per workgroup, per-block arguments from a table.
 template <int DIR, class P, int LIM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k_sweep_adjoint_list(const AdjListArgs L)
 {
     extern __shared__ double lds[];
-    __shared__ unsigned s_item;
-    unsigned x = blockIdx.x % kListQueues, left = kListQueues;
-    for (;;) {
-        __syncthreads();  // the previous tile is done with LDS and s_item
-        if (threadIdx.x == 0) s_item = atomicAdd(L.queue + x, 1u);
-        __syncthreads();
-        const unsigned got = (unsigned)__builtin_amdgcn_readfirstlane((int)s_item);
-        const unsigned lo = list_range(L.nitems, x), hi = list_range(L.nitems, x + 1);
-        if (got >= hi - lo) {
-            if (--left == 0) break;
-            x = (x + 1) % kListQueues;
-            continue;
-        }
-        const unsigned item = lo + got;
-        typedef const __attribute__((address_space(4))) unsigned cu32;
-        const int blk = __builtin_amdgcn_readfirstlane((int)((cu32 *)L.items)[item]);
-        AdjArgs a;
-        {
-            static_assert(sizeof(AdjArgs) % 4 == 0, "AdjArgs is copied in dwords");
-            cu32 *w = (cu32 *)(L.args + blk);
-            unsigned *aw = reinterpret_cast<unsigned *>(&a);
+    typedef const __attribute__((address_space(4))) unsigned cu32;
+    const unsigned item = L.item0 + xcd_order();
+    const int blk = __builtin_amdgcn_readfirstlane((int)((cu32 *)L.items)[item]);
+    AdjArgs a;
+    static_assert(sizeof(AdjArgs) % 4 == 0, "AdjArgs is copied in dwords");
+    cu32 *w = (cu32 *)(L.args + blk);
+    unsigned *aw = reinterpret_cast<unsigned *>(&a);
 #pragma unroll
-            for (int i = 0; i < (int)(sizeof(AdjArgs) / 4); i++) aw[i] = w[i];
-        }
-        const unsigned first = ((cu32 *)L.first)[blk];
-        adjoint_tile<DIR, P, LIM>(a, (int)(item - first), lds);
-    }
+    for (int i = 0; i < (int)(sizeof(AdjArgs) / 4); i++) aw[i] = w[i];
+    adjoint_tile<DIR, P, LIM>(a, (int)(item - ((cu32 *)L.first)[blk]), lds);
 }
 
 // Deterministic sum of n per-wave partials: kRedParts fixed ranges
@@ -729,12 +707,12 @@ static hipError_t adj_lim(const AdjArgs &a, int nt, long long nblk, hipStream_t 
 }
 
 template <int DIR, class P, int LIM>
-static hipError_t adjl_t(const AdjListArgs &L, int grid, hipStream_t st, int *resident)
+static hipError_t adjl_t(const AdjListArgs &L, hipStream_t st)
 {
     const int nt = 256;
     const void *fn = (const void *)k_sweep_adjoint_list<DIR, P, LIM>;
     const size_t lds = sizeof(double) * kAdjArrays * P::NV * nt;
-    const size_t lds_max = 160 * 1024 - 256;
+    const size_t lds_max = 160 * 1024;
     static bool raised = false;
     if (!raised) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max);
@@ -742,54 +720,47 @@ static hipError_t adjl_t(const AdjListArgs &L, int grid, hipStream_t st, int *re
         raised = true;
     }
     if (lds > lds_max) return hipErrorInvalidValue;
-    if (resident) {
-        int per = 0, dev = 0, ncu = 0;
-        hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, nt, lds);
-        if (e == hipSuccess) e = hipGetDevice(&dev);
-        if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-        *resident = per * ncu;
-        return e;
+    AdjListArgs l = L;
+    for (l.item0 = 0; l.item0 < L.nitems; l.item0 += kListPiece) {
+        const unsigned n = L.nitems - l.item0 < kListPiece ? L.nitems - l.item0 : kListPiece;
+        hipLaunchKernelGGL((k_sweep_adjoint_list<DIR, P, LIM>), dim3(n), dim3(nt), lds, st, l);
+        if (l.item0 + n == L.nitems) break;  // (the next item0 may not fit 32 bits)
     }
-    hipLaunchKernelGGL((k_sweep_adjoint_list<DIR, P, LIM>), dim3((unsigned)grid), dim3(nt), lds, st, L);
     return hipGetLastError();
 }
 
 template <int DIR, class P>
-static hipError_t adjl_lim(int lim, int limb, const AdjListArgs &L, int grid, hipStream_t st, int *resident)
+static hipError_t adjl_lim(int lim, int limb, const AdjListArgs &L, hipStream_t st)
 {
     if (lim == limb || !P::MAG) {
         switch (lim) {
-        case LIM_VANLEER: return adjl_t<DIR, P, LIM_VANLEER>(L, grid, st, resident);
-        case LIM_MINMOD: return adjl_t<DIR, P, LIM_MINMOD>(L, grid, st, resident);
-        case LIM_MONCEN: return adjl_t<DIR, P, LIM_MONCEN>(L, grid, st, resident);
-        case LIM_SUPERBEE: return adjl_t<DIR, P, LIM_SUPERBEE>(L, grid, st, resident);
+        case LIM_VANLEER: return adjl_t<DIR, P, LIM_VANLEER>(L, st);
+        case LIM_MINMOD: return adjl_t<DIR, P, LIM_MINMOD>(L, st);
+        case LIM_MONCEN: return adjl_t<DIR, P, LIM_MONCEN>(L, st);
+        case LIM_SUPERBEE: return adjl_t<DIR, P, LIM_SUPERBEE>(L, st);
         default: return hipErrorInvalidValue;
         }
     }
-    return adjl_t<DIR, P, -1>(L, grid, st, resident);
+    return adjl_t<DIR, P, -1>(L, st);
 }
 
-static hipError_t adjl_dispatch(int dir, bool mhd, int lim, int limb, const AdjListArgs &L, int grid, hipStream_t st,
-                                int *resident)
+static hipError_t adjl_dispatch(int dir, bool mhd, int lim, int limb, const AdjListArgs &L, hipStream_t st)
 {
     if (mhd) {
-        if (dir == 0) return adjl_lim<0, MHD>(lim, limb, L, grid, st, resident);
-        if (dir == 1) return adjl_lim<1, MHD>(lim, limb, L, grid, st, resident);
-        if (dir == 2) return adjl_lim<2, MHD>(lim, limb, L, grid, st, resident);
+        if (dir == 0) return adjl_lim<0, MHD>(lim, limb, L, st);
+        if (dir == 1) return adjl_lim<1, MHD>(lim, limb, L, st);
+        if (dir == 2) return adjl_lim<2, MHD>(lim, limb, L, st);
     } else {
-        if (dir == 0) return adjl_lim<0, HD>(lim, limb, L, grid, st, resident);
-        if (dir == 1) return adjl_lim<1, HD>(lim, limb, L, grid, st, resident);
-        if (dir == 2) return adjl_lim<2, HD>(lim, limb, L, grid, st, resident);
+        if (dir == 0) return adjl_lim<0, HD>(lim, limb, L, st);
+        if (dir == 1) return adjl_lim<1, HD>(lim, limb, L, st);
+        if (dir == 2) return adjl_lim<2, HD>(lim, limb, L, st);
     }
     return hipErrorInvalidValue;
 }
 
 hipError_t launch_sweep_adjoint_list(int dir, bool mhd, int lim, int limb, const AdjListArgs &L, hipStream_t st)
 {
-    int r = 0;
-    hipError_t e = adjl_dispatch(dir, mhd, lim, limb, L, 0, st, &r);
-    if (e != hipSuccess) return e;
-    return adjl_dispatch(dir, mhd, lim, limb, L, r > 0 ? r : 1, st, nullptr);
+    return adjl_dispatch(dir, mhd, lim, limb, L, st);
 }
 
 hipError_t launch_sum_parts_jobs(const SumJob *jobs, int njobs, hipStream_t st)
@@ -813,7 +784,7 @@ static hipError_t adj_dir(int dir, const AdjArgs &a, int nt, long long nblk, hip
 }
 
 // Every adjoint tile runs on a 256-lane workgroup (lanes past TP*TS idle),
-// as in the persistent list kernel: four partial slots per tile in both, so
+// as in the list kernel: four partial slots per tile in both, so
 // their sums of the same partials agree bit for bit.
 long long sweep_adjoint_parts(const AdjArgs &a) { return (long long)a.chunks * a.ptiles * 4; }
 

@@ -2,6 +2,7 @@
 // (reverse-mode) kernels in pk_adjoint.hip.
 #pragma once
 #include <hip/hip_runtime.h>
+#include "pk_kernels.hpp"
 
 namespace pk {
 
@@ -43,22 +44,15 @@ struct DtAdjArgs {
     double dtb;  // dL/d(dt)
 };
 
-// Persistent adjoint sweep over a block list (workgroups of 256 lanes take
-// tiles from queues; tile item belongs to block items[item] and is its
-// tile item - first[block]).  Each block's AdjArgs has its tile shape with
+// Adjoint sweep over a block list (a 256-lane workgroup per tile; tile item
+// belongs to block items[item] and is its tile item - first[block]).  Each block's AdjArgs has its tile shape with
 // TP*TS <= 256 and its dtb/chb partial arrays sized for 4 waves per tile.
-constexpr unsigned kListQueues = 8;  // item ranges of a list launch, one per XCD
-// first item of range x of n items
-__host__ __device__ inline unsigned list_range(unsigned n, unsigned x)
-{
-    return (unsigned)((unsigned long long)n * x / kListQueues);
-}
 struct AdjListArgs {
     const AdjArgs *args;
-    const unsigned *first;
+    const unsigned *first;  // one more entry than blocks
     const unsigned *items;
     unsigned nitems;
-    unsigned *queue;  // kListQueues counters, zero before the launch
+    unsigned item0;  // first item of the launch (set by the launcher)
 };
 
 // out[0] = sum of part[0 .. n-1] in a fixed order; part has kRedParts more

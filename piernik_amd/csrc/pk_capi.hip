@@ -8,7 +8,7 @@
 // src/scheme/sweeps.F90:114-279, src/base/timestep.F90:112-240) for one
 // periodic block with cflcontrol='warn'; the list driver (pk_*_all) does the
 // same for the whole registered block list, every block periodic on itself,
-// with one persistent launch per sweep and fluid, captured in a HIP graph.
+// with one launch per sweep and fluid, captured in a HIP graph.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -54,6 +54,7 @@ struct Block {
     bool ghosts_stale = false;                // stream sweeps read the periodic interior and left the ghosts old
     // reverse mode (pk_adjoint_setup): saved states and the adjoint state
     std::vector<double *> slots;
+    std::vector<char> slot_stale;  // the slot's ghosts are old (periodic images of its interior replace them)
     double *lam[2] = {nullptr, nullptr};
     int lcur = 0;
     double *d_dtb_part = nullptr;
@@ -251,7 +252,7 @@ void fill_common(const Block *b, int f, pk::SweepArgs &a)
     a.dmass = b->d_mass + pk::kMassDigits * f;
     a.psi_fac = 1.0;
     a.ch = 0.0;
-    a.images = 0;
+    a.wrap = 0;
     a.dtslots = nullptr;
     a.nslots = kDtSlots;
     for (int d = 0; d < 3; d++) {
@@ -320,8 +321,52 @@ void march_geometry(const Block *b, int d, int &TP, int &out, int &chunks, int &
     out = b->n[d];
 }
 
+// The tile along d of at most nt lanes that needs the fewest workgroups: over
+// the pencil counts tp, the pencil in equal chunks of the longest tile that
+// fits.  Returns the workgroups.  Along x ties go to the longer tile (fewer
+// halo cells read).  Along y and z the lanes of a tile read tp cells in a row,
+// so at least 3 pencils are taken and ties go to the longest tile of 4 or more
+// (HD 224^3, y, 256 lanes: 4x64 575 us, 2x120 586, 1x232 > 640; HD 96^3, y:
+// 4x56 62 us, 2x104 65; MHD 131x98x77, y: 4x57 140 us, 2x106 147).
+long long even_tile(const Block *b, int d, bool fused, int nt, int &tp_out, int &ts_out)
+{
+    const int halo = fused ? 4 : 2;
+    const int span = fused ? b->n[d] : b->ng[d];
+    const int d1 = (d == 0) ? 1 : 0, d2 = (d == 2) ? 1 : 2;
+    const long long npen = (long long)b->n[d1] * b->n[d2];
+    long long best = -1;
+    tp_out = 1;
+    ts_out = 2 * halo + 1;
+    const int tp0 = d == 0 ? 1 : (int)std::min(3ll, npen);
+    for (int tp = tp0; tp <= nt / (2 * halo + 1) && (tp <= npen || tp == tp0); tp++) {
+        const int k = (span + nt / tp - 2 * halo - 1) / (nt / tp - 2 * halo);
+        const int out = (span + k - 1) / k;
+        const long long wgs = (long long)((span + out - 1) / out) * ((npen + tp - 1) / tp);
+        if (best < 0 || wgs < best || (wgs == best && d > 0 && tp_out < 4)) {
+            best = wgs;
+            tp_out = tp;
+            ts_out = out + 2 * halo;
+        }
+    }
+    return best;
+}
+
+// Default tile: 256 lanes (MHD 64^3, z: 256 lanes 47 us, 512 lanes 56; the
+// register budget of the kernels holds two or three 4-wave workgroups per CU,
+// which hide each other's barriers, but one 8-wave workgroup), fewer where
+// that leaves some of the 256 CUs without a workgroup (HD 32^3: 4x40 in 256
+// workgroups 12.4 us, 6x40 in 171 13.3; HD 16^3: 2x24 in 128 11.3 us, 10x24 in
+// 26 12.3 - 13.5).  Against a fixed 3 x 72, which leaves the last chunk of
+// most lengths nearly empty: MHD 131x98x77 206, 179, 212 us along x, y, z there,
+// 147, 140, 125 here; HD 96^3 82, 77, 82 there, 65, 62, 65 here.
+void default_tile(const Block *b, int d, bool fused, int &tp, int &ts)
+{
+    for (int nt = 256; nt >= 64; nt -= 64)
+        if (even_tile(b, d, fused, nt, tp, ts) >= 256) return;
+}
+
 // Precedence: the shape given in pk_config, then the one pk_autotune
-// measured for this block shape, then 3 x 72 (4-wave workgroups, two per CU).
+// measured for this block shape, then default_tile.
 // A tile length of kMarch selects the march kernel for the fused sweep.
 void choose_tile(const Block *b, int d, bool fused, bool mag, int &TP, int &TS, int &out, int &chunks, int &ptiles)
 {
@@ -347,8 +392,9 @@ void choose_tile(const Block *b, int d, bool fused, bool mag, int &TP, int &TS, 
         return;
     }
     if (ts <= 0) {
-        ts = 72;
-        if (tp <= 0) tp = 3;
+        int dtp;
+        default_tile(b, d, fused, dtp, ts);
+        if (tp <= 0) tp = dtp;
     }
     tile_geometry(b, d, fused, tp, ts, TP, TS, out, chunks, ptiles);
 }
@@ -687,12 +733,13 @@ int do_stage(Block *b, int ddim, int istep, double dt, double ch)
     return PK_OK;
 }
 
-// One directional sweep, both RK2 stages, every fluid.  images: write the
-// periodic ghost images too (the block is periodic on itself); want_dt:
-// reduce the next step's timestep_fluid from the cells written.  With
-// src/dst (whole state buffers, one fluid) the sweep reads src and writes
-// dst instead of the block's ping-pong pair, whose state is left alone.
-int do_sweep(Block *b, int ddim, double dt, double ch, double psi_fac, int images = 0, bool want_dt = false,
+// One directional sweep, both RK2 stages, every fluid.  wrap: the block is
+// periodic on itself and the sweep reads its interior in place of the ghosts,
+// which it leaves old (b->ghosts_stale); want_dt: reduce the next step's
+// timestep_fluid from the cells written.  With src/dst (whole state buffers,
+// one fluid) the sweep reads src and writes dst instead of the block's
+// ping-pong pair, whose state is left alone.
+int do_sweep(Block *b, int ddim, double dt, double ch, double psi_fac, bool wrap = false, bool want_dt = false,
              double *src = nullptr, double *dst = nullptr)
 {
     RCCHK(no_fc(b, "a whole sweep runs both stages in one pass"));
@@ -715,12 +762,12 @@ int do_sweep(Block *b, int ddim, double dt, double ch, double psi_fac, int image
         a.src = src ? src + b->xo + (long long)g_fplane[f] * b->sv : fluid_state(b, b->cur, f);
         a.base = a.src;
         a.dst = dst ? dst + b->xo + (long long)g_fplane[f] * b->sv : fluid_state(b, 1 - b->cur, f);
-        a.images = images;
+        a.wrap = wrap ? 1 : 0;
         a.dtslots = want_dt ? b->d_dtslots : nullptr;
         RCCHK(launch(ddim, true, a, b, f));
     }
-    if (images == 2) b->ghosts_stale = true;
     if (src || dst) return PK_OK;
+    if (wrap) b->ghosts_stale = true;
     b->cur = 1 - b->cur;
     b->uh = -1;
     b->dt_pending = false;
@@ -831,30 +878,12 @@ void glm_scalars(const std::vector<double> &mdls, double dt, double *ch_out, dou
     *fac_out = std::exp(-f);
 }
 
-// The fused sweep along every active direction of every fluid of b runs the
-// stream kernel (its shape in pk_config, tuned or given): then its sweeps may
-// read ghost positions from their periodic pre-images and leave the ghosts
-// old (images == 2), to be refilled once by the caller.
-bool stream_all_dirs(const Block *b)
-{
-    for (int f = 0; f < g_nfl; f++)
-        for (int d = 0; d < 3; d++) {
-            if (!g_cfg.has_dir[d]) continue;
-            int TP, TS, out, chunks, ptiles;
-            choose_tile(b, d, true, g_fmag[f], TP, TS, out, chunks, ptiles);
-            if (!is_stream(TS)) return false;
-        }
-    return true;
-}
-
-// One step of fluid_update.  allow_wrap: the sweeps may leave the periodic
-// ghosts old when every one of them is a stream sweep (b->ghosts_stale; the
-// caller refills them with do_fill before they are read).
-int do_fluid_update(Block *b, double dt, bool allow_wrap = false)
+// One step of fluid_update.  The RK2 sweeps leave the periodic ghosts old
+// (b->ghosts_stale): the caller refills them with do_fill before they are read.
+int do_fluid_update(Block *b, double dt)
 {
     double ch = 0.0, fac = 1.0;
     if (g_mhd) glm_scalars({min_dl(b)}, dt, &ch, &fac);
-    const int images = (allow_wrap && g_cfg.integration_order == 2 && stream_all_dirs(b)) ? 2 : 1;
     for (int half = 0; half < 2; half++) {
         int last = -1;
         for (int s = 0; s < 3; s++) {
@@ -865,9 +894,8 @@ int do_fluid_update(Block *b, double dt, bool allow_wrap = false)
             const int d = half == 0 ? s : 2 - s;
             if (!g_cfg.has_dir[d]) continue;
             if (g_cfg.integration_order == 2) {
-                // the sweep refreshes the periodic ghosts itself; the last one of
-                // the step also reduces the next step's timestep
-                RCCHK(do_sweep(b, d, dt, ch, (d == last) ? fac : 1.0, images, half == 1 && d == last));
+                // the last sweep of the step also reduces the next step's timestep
+                RCCHK(do_sweep(b, d, dt, ch, (d == last) ? fac : 1.0, true, half == 1 && d == last));
             } else {
                 RCCHK(do_sweep(b, d, dt, ch, (d == last) ? fac : 1.0));
                 RCCHK(do_fill(b));
@@ -908,6 +936,7 @@ void free_adjoint(Block *b)
     for (double *p : b->slots)
         if (p) (void)hipFree(p);
     b->slots.clear();
+    b->slot_stale.clear();
     for (int i = 0; i < 2; i++) {
         if (b->lam[i]) (void)hipFree(b->lam[i]);
         b->lam[i] = nullptr;
@@ -1201,14 +1230,14 @@ std::vector<int> step_dirs(std::vector<bool> *damp = nullptr)
 
 // ---------------------------------------------------------------- block list
 //
-// The whole registered list (ascending cg_id), swept by one persistent
+// The whole registered list (ascending cg_id), swept by one
 // launch per direction and fluid.  Per block and (direction, fluid) the
 // host builds the kernel arguments once; the per-step scalars live in
 // device memory (StepScalars), so the step's launches are captured once in a
 // HIP graph and replayed.
 
 struct LaunchTab {
-    int nt = 256;                       // workgroup lanes of the persistent launch
+    int nt = 256;                       // workgroup lanes of the launch
     std::vector<Block *> blocks;        // the blocks of the launch, in item order
     std::vector<pk::SweepArgs> h_args;  // per block, src = buffer of the block's cur at build time
     std::vector<unsigned> h_first;      // per block first item, nblocks + 1 entries, then each
@@ -1218,10 +1247,8 @@ struct LaunchTab {
     unsigned *d_items = nullptr;
     size_t cap_blocks = 0, cap_items = 0;
     unsigned nitems = 0;
-    int grid = 0;
+    int grid = 0;                       // workgroups of a stream launch (tiles: one per item)
 };
-
-const int kQueues = 32;
 
 // The face jobs of one exchange direction over the list.
 struct FaceTab {
@@ -1287,7 +1314,6 @@ struct ListState {
     LaunchTab stab[3][2];
     int nt_pref[3][2] = {{0, 0}, {0, 0}, {0, 0}};  // workgroup lanes chosen by pk_autotune_all (0: default)
     int ts_force[3][2] = {{0, 0}, {0, 0}, {0, 0}};  // tile length (stream: -iterations) set by pk_set_list_tiles
-    unsigned *d_queue = nullptr;
     pk::StepScalars *d_step = nullptr;
     pk::StepScalars *h_step = nullptr;  // pinned
     unsigned long long *d_dtslots = nullptr;
@@ -1307,13 +1333,10 @@ struct ListState {
     bool ghosts_stale = false;  // linked list after a step: the ghosts other than the swept faces are old
     FaceTab ex[3][2];           // per direction and buffer parity
     // blocks periodic on themselves: each ghost face from the block's own
-    // opposite interior (one launch per direction fills the whole list), and
-    // whether some block's stream sweeps read ghost positions from their
-    // pre-images and leave the ghosts old (images == 2 in its tables)
+    // opposite interior (one launch per direction fills the whole list);
+    // wrap_stale: the sweeps, which read the interior instead, left the ghosts old
     FaceTab self[3];
     bool self_built = false;
-    bool wrap_any = false;
-    bool wrap_all = false;  // every block's tables do
     bool wrap_stale = false;
 };
 ListState g_list;
@@ -1344,7 +1367,6 @@ struct EnsembleState {
     double *d_mn = nullptr;
     unsigned long long *d_best = nullptr;
     double *d_sums = nullptr, *h_sums = nullptr;  // per block, per sweep: dtb, chb
-    unsigned *d_queue = nullptr;
 };
 EnsembleState g_ens;
 
@@ -1405,7 +1427,6 @@ void ens_free()
     if (g_ens.d_best) (void)hipFree(g_ens.d_best);
     if (g_ens.d_sums) (void)hipFree(g_ens.d_sums);
     if (g_ens.h_sums) (void)hipHostFree(g_ens.h_sums);
-    if (g_ens.d_queue) (void)hipFree(g_ens.d_queue);
     g_ens = EnsembleState();
 }
 
@@ -1422,7 +1443,6 @@ void list_free()
         if (t.d_jobs) (void)hipFree(t.d_jobs);
         if (t.d_wgjob) (void)hipFree(t.d_wgjob);
     }
-    if (g_list.d_queue) (void)hipFree(g_list.d_queue);
     if (g_list.d_step) (void)hipFree(g_list.d_step);
     if (g_list.h_step) (void)hipHostFree(g_list.h_step);
     if (g_list.d_dtslots) (void)hipFree(g_list.d_dtslots);
@@ -1436,34 +1456,13 @@ void list_free()
     g_list = ListState();
 }
 
-// Default list tile along d for nt lanes: the split of the pencil into
-// chunks that needs the fewest nt-lane tiles; ties go to the longer tile.
-// Tiles a workgroup of the persistent list sweep takes per queue fetch: one
-// atomic per tile on the shared counter cost 9 % of a 4096-block step; four
-// per fetch (or sixteen) remove it.
-constexpr unsigned kListGrab = 4;
-
+// Default list tile along d for nt lanes (even_tile).
 int list_default_ts(const Block *b, int d, int nt)
 {
     if (nt == pk::kStreamListNt) return -16;  // the stream: 16 iterations per item
-    const int span = b->n[d];
-    const int d1 = (d == 0) ? 1 : 0, d2 = (d == 2) ? 1 : 2;
-    const long long npen = (long long)b->n[d1] * b->n[d2];
-    long long best = -1;
-    int best_ts = 0;
-    for (int k = 1; k <= span; k++) {
-        const int out = (span + k - 1) / k;
-        const int ts = out + 8;
-        if (ts > nt) continue;
-        const int tp = nt / ts;
-        const long long tiles = (long long)((span + out - 1) / out) * ((npen + tp - 1) / tp);
-        if (best < 0 || tiles < best) {
-            best = tiles;
-            best_ts = ts;
-        }
-        if (out <= 1) break;
-    }
-    return best_ts > 0 ? best_ts : 9;
+    int tp, ts;
+    even_tile(b, d, true, nt, tp, ts);
+    return ts;
 }
 
 int list_ts(const Block *b, int d, int f, int nt)
@@ -1477,26 +1476,11 @@ int list_ts(const Block *b, int d, int f, int nt)
     return list_default_ts(b, d, nt);
 }
 
-// Kernel arguments and item table of one persistent launch over `blks`.
-// Block b's fluid f is swept in the stream form along every active direction
-// (the list's workgroup size, or its split shapes).
-bool list_wrap_ok(const Block *b, int f)
-{
-    const int mag = g_fmag[f];
-    for (int d = 0; d < 3; d++) {
-        if (!g_cfg.has_dir[d]) continue;
-        const int nt = g_list.nt_pref[d][mag] > 0 ? g_list.nt_pref[d][mag] : 256;
-        if (nt != pk::kStreamListNt && !g_list.split_cls[d][mag].count({b->n[0], b->n[1], b->n[2]})) return false;
-    }
-    return true;
-}
-
-// wrap: 0 every block writes its images; 1 the blocks whose every sweep is a
-// stream sweep read their ghost positions from the pre-images (list_wrap_ok);
-// 2 every block of a stream table does (timing only: the autotuner's
-// candidates, whose results are discarded)
+// Kernel arguments and item table of one launch over `blks`.  The
+// blocks of an unlinked list are periodic on themselves: their sweeps read the
+// interior in place of the ghosts.
 int build_tab(LaunchTab &t, const std::vector<Block *> &blks, int d, int f, int nt,
-              const std::vector<int> *ts_override = nullptr, int wrap = 0)
+              const std::vector<int> *ts_override = nullptr)
 {
     t.nt = nt;
     t.blocks = blks;
@@ -1525,8 +1509,7 @@ int build_tab(LaunchTab &t, const std::vector<Block *> &blks, int d, int f, int 
         a.src = fluid_state(b, b->cur, f);
         a.base = a.src;
         a.dst = fluid_state(b, 1 - b->cur, f);
-        const bool wr = wrap == 2 ? nt == pk::kStreamListNt : (wrap == 1 && list_wrap_ok(b, f));
-        a.images = g_list.linked ? 0 : (wr ? 2 : 1);
+        a.wrap = g_list.linked ? 0 : 1;
         const int ts = ts_override ? (*ts_override)[i] : list_ts(b, d, f, nt);
         if (nt == pk::kStreamListNt) {
             // the stream form: items are ranges of -ts iterations of the block's stream
@@ -1540,8 +1523,7 @@ int build_tab(LaunchTab &t, const std::vector<Block *> &blks, int d, int f, int 
         }
         t.h_first[i] = items;
         const unsigned long long n = (unsigned long long)a.chunks * (unsigned long long)a.ptiles;
-        // headroom for the fetches past the end (at most grab per resident workgroup)
-        if (items + n > 0xffffffffull - (1ull << 24)) return fail(PK_EINVAL, "block list has too many tiles");
+        if (items + n > 0xffffffffull) return fail(PK_EINVAL, "block list has too many tiles");
         items += (unsigned)n;
     }
     t.h_first[blks.size()] = items;
@@ -1567,6 +1549,7 @@ int build_tab(LaunchTab &t, const std::vector<Block *> &blks, int d, int f, int 
                           g_stream));
     HIPCHK(pk::launch_fill_items(t.d_first, (int)blks.size(), t.d_items, g_stream));
     t.grid = list_resident(d, g_fmag[f], nt);
+    if (t.grid > 0 && t.nitems < (unsigned)t.grid) t.grid = (int)t.nitems;
     if (t.grid <= 0) return fail(PK_EHIP, "no resident workgroups for the list sweep (nt = %d)", nt);
     HIPCHK(hipStreamSynchronize(g_stream));
     return PK_OK;
@@ -1714,7 +1697,7 @@ int list_fill()
 }
 
 // The ghosts the list's stream sweeps left old (every block of the list, as
-// their images would have left them), before anything reads them.
+// its sweeps read them), before anything reads them.
 int settle_ghosts()
 {
     if (!g_list.wrap_stale || !g_list.built) return PK_OK;
@@ -1736,8 +1719,6 @@ int list_build()
     if (g_blocks.empty()) return fail(PK_ESTATE, "no registered blocks");
     if (g_cfg.integration_order != 2) return fail(PK_EINVAL, "the batched list sweep is the fused RK2 sweep");
     g_list.blocks.clear();
-    g_list.wrap_any = false;
-    g_list.wrap_all = true;
     g_list.cur0.clear();
     g_list.mdl.clear();
     for (auto &kv : g_blocks) {
@@ -1765,17 +1746,10 @@ int list_build()
             std::vector<Block *> main, split;
             for (Block *b : g_list.blocks)
                 (nt != pk::kStreamListNt && sc.count({b->n[0], b->n[1], b->n[2]}) ? split : main).push_back(b);
-            const int wrap = (!g_list.linked && g_list.self_built) ? 1 : 0;
-            RCCHK(build_tab(g_list.tab[d][f], main, d, f, nt, nullptr, wrap));
-            RCCHK(build_tab(g_list.stab[d][f], split, d, f, pk::kStreamListNt, nullptr, wrap));
-            for (const LaunchTab *t : {&g_list.tab[d][f], &g_list.stab[d][f]})
-                for (const pk::SweepArgs &a : t->h_args) {
-                    g_list.wrap_any = g_list.wrap_any || a.images == 2;
-                    g_list.wrap_all = g_list.wrap_all && a.images == 2;
-                }
+            RCCHK(build_tab(g_list.tab[d][f], main, d, f, nt));
+            RCCHK(build_tab(g_list.stab[d][f], split, d, f, pk::kStreamListNt));
         }
     }
-    if (!g_list.d_queue) HIPCHK(hipMalloc((void **)&g_list.d_queue, sizeof(unsigned) * kQueues));
     if (!g_list.d_step) HIPCHK(hipMalloc((void **)&g_list.d_step, sizeof(pk::StepScalars)));
     if (!g_list.h_step) HIPCHK(hipHostMalloc((void **)&g_list.h_step, sizeof(pk::StepScalars), hipHostMallocDefault));
     if (!g_list.d_dtslots) {
@@ -1827,13 +1801,11 @@ std::vector<SweepStep> step_sweeps()
 // Enqueue the launches of one step on g_stream.  mode PK_BATCH_PER_BLOCK
 // launches the single-block sweep once per block with the same tile shapes
 // (for items of the stream form, the block's single-block shape); the
-// persistent modes launch the list sweep once per sweep and fluid.
+// list modes launch the list sweep once per sweep and fluid.
 int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
 {
     const std::vector<SweepStep> sw = step_sweeps();
     const bool persistent = mode != PK_BATCH_PER_BLOCK;
-    if (sw.size() * (size_t)g_nfl * 2 > (size_t)kQueues) return fail(PK_EINVAL, "too many launches per step");
-    if (persistent) HIPCHK(pk::launch_zero_u32(g_list.d_queue, kQueues, g_stream));
     unsigned long long *slots = ens ? g_ens.d_dtslots : g_list.d_dtslots;
     const int nslots = ens ? kEnsSlots : kDtSlots;
     int q = 0;
@@ -1853,8 +1825,6 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
                     L.first = t.d_first;
                     L.items = t.d_items;
                     L.nitems = t.nitems;
-                    L.queue = g_list.d_queue + q++;
-                    L.grab = kListGrab;
                     L.parity = parity;
                     L.apply_fac = sw[k].fac && g_fmag[f];
                     L.step = ens ? g_ens.d_step : g_list.d_step;
@@ -1862,7 +1832,6 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
                     L.nslots = nslots;
                     L.per_block = ens ? 1 : 0;
                     L.bpos = t.d_first + t.blocks.size() + 1;
-                    L.no_wrap = ens ? 1 : 0;  // an ensemble keeps its ghosts current (the adjoint reads them)
                     if (mode == PK_BATCH_GRAPH) {
                         HIPCHK(list_kernel(d, g_fmag[f], L, t.nt, t.grid));
                     } else {
@@ -1871,7 +1840,6 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
                 } else {
                     for (size_t i = 0; i < t.blocks.size(); i++) {
                         pk::SweepArgs a = t.h_args[i];
-                        if (a.images == 2) a.images = 1;  // one block at a time writes its images
                         if (is_stream(a.TS)) {
                             // list items of the stream form are sized for the whole list
                             // sharing the device; one block alone gets the single-block shape
@@ -1944,19 +1912,8 @@ int list_dt(double *dt_out, double *c_out)
     return list_prepare(dt_out, c_out);
 }
 
-// Refreshes the ghosts a step of the list reads before its sweeps write any:
-// none in the persistent modes of a linked list (every sweep follows an
-// exchange) or where every block's sweeps read the periodic interior.
-int list_fill_for_step(int mode)
-{
-    if (g_list.fresh || g_list.filled) return PK_OK;
-    if (mode != PK_BATCH_PER_BLOCK && (g_list.linked || g_list.wrap_all)) return PK_OK;
-    return list_fill();
-}
-
 int list_step(int mode, double dt)
 {
-    if (mode == PK_BATCH_PER_BLOCK) RCCHK(settle_ghosts());  // one block at a time reads its ghosts
     pk::StepScalars sc{};
     sc.dt = dt;
     sc.ch = 0.0;
@@ -1979,7 +1936,7 @@ int list_step(int mode, double dt)
     g_list.fresh = true;
     g_list.filled = false;
     g_list.ghosts_stale = g_list.linked;
-    if (g_list.wrap_any && mode != PK_BATCH_PER_BLOCK) g_list.wrap_stale = true;
+    if (!g_list.linked) g_list.wrap_stale = true;
     g_ens.fresh = false;
     return PK_OK;
 }
@@ -1995,7 +1952,6 @@ int check_mode(int mode)
 
 int ens_build()
 {
-    RCCHK(settle_ghosts());  // the ensemble's sweeps read the ghosts
     RCCHK(list_build());
     if (g_list.linked) return fail(PK_EINVAL, "ensemble instances must be periodic on themselves (no neighbours)");
     const size_t n = g_list.blocks.size();
@@ -2008,7 +1964,6 @@ int ens_build()
     HIPCHK(pk::launch_dtslots_init(g_ens.d_dtslots, kEnsSlots * (int)n, g_stream));
     HIPCHK(hipHostMalloc((void **)&g_ens.dtout, sizeof(double) * 4 * n, hipHostMallocDefault));
     HIPCHK(hipMalloc((void **)&g_ens.d_jobs, sizeof(pk::CopyJob) * n));
-    HIPCHK(hipMalloc((void **)&g_ens.d_queue, sizeof(unsigned) * pk::kListQueues));
     g_ens.h_jobs.resize(n);
     g_ens.dt_old.assign(n, -1.0);
     g_ens.fresh = false;
@@ -2039,7 +1994,6 @@ int ens_dt_raw(std::vector<double> &dt)
     const size_t n = g_ens.nblk;
     dt.assign(n, 0.0);
     if (!g_ens.fresh) {
-        if (!g_list.filled) RCCHK(list_fill());
         HIPCHK(pk::launch_dt_list(g_list.d_dt, (int)n, g_nfl, g_list.dt_maxcells, g_ens.d_dtslots, kEnsSlots, 1,
                                   g_stream));
         HIPCHK(pk::launch_dtslots_final(g_ens.d_dtslots, kEnsSlots, (int)n, g_ens.dtout, g_stream));
@@ -2073,6 +2027,7 @@ int ens_set_step(const double *dts)
 // block's other buffer (between the sweeps of a step)
 int ens_copy_slots(int slot, bool save, int parity = 0)
 {
+    bool stale = false;
     for (size_t i = 0; i < g_ens.nblk; i++) {
         Block *b = g_list.blocks[i];
         if (b->lam[0] == nullptr || slot < 0 || slot >= (int)b->slots.size())
@@ -2082,7 +2037,10 @@ int ens_copy_slots(int slot, bool save, int parity = 0)
         j.dst = save ? b->slots[slot] : b->buf[b->cur ^ parity];
         j.n = (long long)b->sv * g_nplanes;
         g_ens.h_jobs[i] = j;
+        if (save) b->slot_stale[slot] = parity != 0 || g_list.wrap_stale;
+        stale = stale || b->slot_stale[slot];
     }
+    if (!save) g_list.wrap_stale = stale;  // every block's state is replaced
     HIPCHK(hipMemcpyAsync(g_ens.d_jobs, g_ens.h_jobs.data(), sizeof(pk::CopyJob) * g_ens.nblk, hipMemcpyHostToDevice,
                           g_stream));
     HIPCHK(pk::launch_copy_blocks(g_ens.d_jobs, (int)g_ens.nblk, g_stream));
@@ -2090,7 +2048,7 @@ int ens_copy_slots(int slot, bool save, int parity = 0)
     return PK_OK;
 }
 
-// tile tables of the persistent adjoint sweep (per direction) and the sum jobs
+// tile tables of the list adjoint sweep (per direction) and the sum jobs
 int ens_adj_build()
 {
     if (g_ens.adj_built) return PK_OK;
@@ -2742,7 +2700,7 @@ int pk_sweep_noalloc(const double *src, double *dst, int64_t sv, int32_t sy, int
         a.src = src + (long long)g_fplane[f] * sv;
         a.base = a.src;
         a.dst = dst + (long long)g_fplane[f] * sv;
-        a.images = 0;
+        a.wrap = 0;
         choose_tile(&b, ddim, true, g_fmag[f], a.TP, a.TS, a.out, a.chunks, a.ptiles);
         HIPCHK(sweep_kernel(ddim, g_fmag[f], true, a, st));
     }
@@ -2948,7 +2906,9 @@ int pk_fluid_update(int64_t cg_id, double dt)
     RCCHK(solo(b));
     if (!(dt > 0.0)) return fail(PK_EINVAL, "dt must be positive");
     list_touch();
-    return do_fluid_update(b, dt);
+    RCCHK(do_fluid_update(b, dt));
+    if (b->ghosts_stale) RCCHK(do_fill(b));
+    return PK_OK;
 }
 
 int pk_run(int64_t cg_id, int32_t nsteps, double *t_out, double *dt_out)
@@ -2958,14 +2918,14 @@ int pk_run(int64_t cg_id, int32_t nsteps, double *t_out, double *dt_out)
     RCCHK(solo(b));
     if (nsteps < 0) return fail(PK_EINVAL, "nsteps < 0");
     list_touch();
-    // sweeps that read the periodic interior need no ghosts; they are refreshed after the steps
-    if (nsteps == 0 || g_cfg.integration_order != 2 || !stream_all_dirs(b)) RCCHK(do_fill(b));
+    // the RK2 sweeps read the periodic interior; the ghosts are refreshed after the steps
+    if (nsteps == 0 || g_cfg.integration_order != 2) RCCHK(do_fill(b));
     StepLoop L;
     L.blocks = {b};
     L.timestep = [b](double *dt, double *c) { return do_timestep(b, dt, c); };
-    L.update = [b](double dt) { return do_fluid_update(b, dt, true); };
+    L.update = [b](double dt) { return do_fluid_update(b, dt); };
     RCCHK(run_loop(L, nsteps, t_out, dt_out, &g_last_redone));
-    if (b->ghosts_stale) RCCHK(do_fill(b));  // the ghosts as the sweeps' images would have left them
+    if (b->ghosts_stale) RCCHK(do_fill(b));
     return PK_OK;
 }
 
@@ -3114,39 +3074,43 @@ int pk_autotune(int64_t cg_id, double dt, double chspeed, int32_t tiles_out[6])
             // pencils to give every SIMD a wave (x pencils are rows: uncoalesced)
             const int d1 = (d == 0) ? 1 : 0, d2 = (d == 2) ? 1 : 2;
             const bool try_march = d > 0 && (long long)b->n[d1] * b->n[d2] >= 65536;
-            for (int ts : ts_list) {
+            std::vector<std::pair<int, int>> tiles(1);  // the default first
+            default_tile(b, d, true, tiles[0].first, tiles[0].second);
+            for (int ts : ts_list)
                 for (int w : waves_list) {
-                    int TP, TS, out, chunks, ptiles;
-                    int tp = (64 * w) / (ts < b->n[d] + 8 ? ts : b->n[d] + 8);
-                    if (tp < 1) continue;
-                    tile_geometry(b, d, true, tp, ts, TP, TS, out, chunks, ptiles);
-                    if (TP * TS > 512) continue;
-                    bool dup = false;
-                    for (auto &p : seen) dup = dup || (p.first == TP && p.second == TS);
-                    if (dup) continue;
-                    seen.push_back({TP, TS});
-                    a.TP = TP;
-                    a.TS = TS;
-                    a.out = out;
-                    a.chunks = chunks;
-                    a.ptiles = ptiles;
-                    HIPCHK(sweep_kernel(d, g_fmag[f], true, a));  // warm-up
-                    HIPCHK(hipEventRecord(e0, g_stream));
-                    for (int rep = 0; rep < 3; rep++) HIPCHK(sweep_kernel(d, g_fmag[f], true, a));
-                    HIPCHK(hipEventRecord(e1, g_stream));
-                    HIPCHK(hipEventSynchronize(e1));
-                    float ms = 0.0f;
-                    HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-                    if (ms < best) {
-                        best = ms;
-                        best_t = {TP, TS};
-                    }
+                    const int tp = (64 * w) / (ts < b->n[d] + 8 ? ts : b->n[d] + 8);
+                    if (tp >= 1) tiles.push_back({tp, ts});
+                }
+            for (auto &cand : tiles) {
+                const int tp = cand.first, ts = cand.second;
+                int TP, TS, out, chunks, ptiles;
+                tile_geometry(b, d, true, tp, ts, TP, TS, out, chunks, ptiles);
+                if (TP * TS > 512) continue;
+                bool dup = false;
+                for (auto &p : seen) dup = dup || (p.first == TP && p.second == TS);
+                if (dup) continue;
+                seen.push_back({TP, TS});
+                a.TP = TP;
+                a.TS = TS;
+                a.out = out;
+                a.chunks = chunks;
+                a.ptiles = ptiles;
+                HIPCHK(sweep_kernel(d, g_fmag[f], true, a));  // warm-up
+                HIPCHK(hipEventRecord(e0, g_stream));
+                for (int rep = 0; rep < 3; rep++) HIPCHK(sweep_kernel(d, g_fmag[f], true, a));
+                HIPCHK(hipEventRecord(e1, g_stream));
+                HIPCHK(hipEventSynchronize(e1));
+                float ms = 0.0f;
+                HIPCHK(hipEventElapsedTime(&ms, e0, e1));
+                if (ms < best) {
+                    best = ms;
+                    best_t = {TP, TS};
                 }
             }
             // the stream kernel: 1, 2, 4 or 8 pencils per lane group,
-            // workgroups of about 8 to 64 iterations
+            // workgroups of about 4 to 64 iterations
             for (int tp : {1, 2, 4, 8}) {
-                for (int m : {8, 16, 32, 64}) {
+                for (int m : {4, 8, 16, 32, 64}) {
                     a.TS = -m;
                     stream_geometry(b, d, tp, m, a.TP, a.out, a.chunks, a.ptiles);
                     HIPCHK(sweep_kernel(d, g_fmag[f], true, a));  // warm-up
@@ -3211,7 +3175,6 @@ int pk_fluid_update_all(int32_t mode, double dt)
     RCCHK(check_mode(mode));
     if (!(dt > 0.0)) return fail(PK_EINVAL, "dt must be positive");
     RCCHK(list_build());
-    RCCHK(list_fill_for_step(mode));
     return list_step(mode, dt);  // ghosts left old are refilled when something reads them
 }
 
@@ -3224,11 +3187,7 @@ int pk_run_all(int32_t mode, int32_t nsteps, double *t_out, double *dt_out)
     StepLoop L;
     L.blocks = g_list.blocks;
     L.timestep = [](double *dt, double *c) { return list_dt(dt, c); };
-    L.update = [mode](double dt) {
-        // a redone step starts from restored states: ghosts and dt are recomputed
-        RCCHK(list_fill_for_step(mode));
-        return list_step(mode, dt);
-    };
+    L.update = [mode](double dt) { return list_step(mode, dt); };
     return run_loop(L, nsteps, t_out, dt_out, &g_last_redone);  // ghosts left old are refilled when read
 }
 
@@ -3290,16 +3249,12 @@ int pk_autotune_all(double dt, double chspeed)
                     int best_ts = cand.empty() ? 9 : cand[0];
                     for (int ts : cand) {
                         std::vector<int> tsv(cl.second.size(), ts);
-                        // stream candidates timed as they run when every sweep of the block is one:
-                        // ghost positions from their pre-images, no images written
-                        if ((rc = build_tab(tmp, cl.second, d, f, nt, &tsv, g_list.self_built ? 2 : 0))) break;
+                        if ((rc = build_tab(tmp, cl.second, d, f, nt, &tsv))) break;
                         pk::ListArgs L{};
                         L.args = tmp.d_args;
                         L.first = tmp.d_first;
                         L.items = tmp.d_items;
                         L.nitems = tmp.nitems;
-                        L.queue = g_list.d_queue;
-                        L.grab = kListGrab;
                         L.parity = 0;
                         L.apply_fac = 0;
                         L.step = g_list.d_step;
@@ -3307,7 +3262,6 @@ int pk_autotune_all(double dt, double chspeed)
                         L.nslots = kDtSlots;
                         float ms = 0.0f;
                         for (int rep = 0; rep < 2; rep++) {  // warm-up, then timed
-                            HIPCHK(pk::launch_zero_u32(g_list.d_queue, 1, g_stream));
                             HIPCHK(hipEventRecord(e0, g_stream));
                             HIPCHK(list_kernel(d, g_fmag[f], L, nt, tmp.grid));
                             HIPCHK(hipEventRecord(e1, g_stream));
@@ -3475,6 +3429,7 @@ int pk_adjoint_setup(int64_t cg_id, int32_t nslots)
         HIPCHK(hipMemsetAsync(b->lam[i], 0, bytes, g_stream));
     }
     b->slots.assign(nslots, nullptr);
+    b->slot_stale.assign(nslots, 0);
     for (int i = 0; i < nslots; i++) HIPCHK(hipMalloc((void **)&b->slots[i], bytes));
     long long parts = 1;
     for (int d = 0; d < 3; d++) {
@@ -3502,6 +3457,7 @@ int pk_state_save(int64_t cg_id, int32_t slot)
     RCCHK(adj_check(b));
     RCCHK(slot_ptr(b, slot, &p));
     HIPCHK(hipMemcpyAsync(p, b->buf[b->cur], state_bytes(b), hipMemcpyDeviceToDevice, g_stream));
+    b->slot_stale[slot] = 0;
     return PK_OK;
 }
 
@@ -3514,6 +3470,7 @@ int pk_state_load(int64_t cg_id, int32_t slot)
     RCCHK(slot_ptr(b, slot, &p));
     list_touch();
     HIPCHK(hipMemcpyAsync(b->buf[b->cur], p, state_bytes(b), hipMemcpyDeviceToDevice, g_stream));
+    if (b->slot_stale[slot]) RCCHK(do_fill(b));
     b->dt_pending = false;
     b->uh = -1;
     return PK_OK;
@@ -3574,7 +3531,8 @@ int pk_fluid_update_record(int64_t cg_id, int32_t slot0, double dt)
     double ch, fac;
     block_glm(b, dt, &ch, &fac);
     // the state before sweep i lands in slot0 + i: one copy, then each sweep
-    // but the last writes the next slot directly (periodic images included)
+    // but the last writes the next slot's interior directly
+    for (size_t i = 0; i < dirs.size(); i++) b->slot_stale[slot0 + i] = i > 0;
     HIPCHK(hipMemcpyAsync(b->slots[slot0], b->buf[b->cur], state_bytes(b), hipMemcpyDeviceToDevice, g_stream));
     for (size_t i = 0; i + 1 < dirs.size(); i++)
         RCCHK(do_sweep(b, dirs[i], dt, ch, damp[i] ? fac : 1.0, true, false, b->slots[slot0 + i],
@@ -3586,7 +3544,7 @@ int pk_fluid_update_record(int64_t cg_id, int32_t slot0, double dt)
     b->dt_pending = false;
     HIPCHK(pk::launch_dtslots_final(b->d_dtslots, kDtSlots, 1, b->dtout, g_stream));
     b->dt_pending = true;
-    return PK_OK;
+    return do_fill(b);
 }
 
 int pk_fluid_update_adjoint(int64_t cg_id, int32_t slot0, double dt, double *dt_bar)
@@ -3707,6 +3665,7 @@ int pk_ensemble_step(int32_t mode, int32_t first, double *dt_out, int32_t *cappe
     }
     g_list.fresh = false;
     g_list.filled = false;
+    g_list.wrap_stale = true;
     g_ens.fresh = true;
     return PK_OK;
 }
@@ -3761,7 +3720,6 @@ int pk_ensemble_record_step(const double *dts, int32_t slot0)
     std::vector<bool> damp;
     const std::vector<int> dirs = step_dirs(&damp);
     RCCHK(ens_set_step(dts));
-    HIPCHK(pk::launch_zero_u32(g_list.d_queue, kQueues, g_stream));
     for (size_t k = 0; k < dirs.size(); k++) {
         RCCHK(ens_copy_slots(slot0 + (int)k, true, (int)(k % 2)));
         const int d = dirs[k];
@@ -3774,8 +3732,6 @@ int pk_ensemble_record_step(const double *dts, int32_t slot0)
                 L.first = t.d_first;
                 L.items = t.d_items;
                 L.nitems = t.nitems;
-                L.queue = g_list.d_queue + (int)((k * g_nfl + f) * 2 + part);
-                L.grab = kListGrab;
                 L.parity = (int)(k % 2);
                 L.apply_fac = damp[k] && g_fmag[f];
                 L.step = g_ens.d_step;
@@ -3783,12 +3739,12 @@ int pk_ensemble_record_step(const double *dts, int32_t slot0)
                 L.nslots = kEnsSlots;
                 L.per_block = 1;
                 L.bpos = t.d_first + t.blocks.size() + 1;
-                L.no_wrap = 1;
                 HIPCHK(list_kernel(d, g_fmag[f], L, t.nt, t.grid));
             }
         }
     }
     list_touch();
+    g_list.wrap_stale = true;
     for (Block *b : g_list.blocks) {
         b->dt_pending = false;
         b->uh = -1;
@@ -3859,13 +3815,11 @@ int pk_ensemble_step_adjoint(const double *dts, int32_t slot0, double *dt_bar)
         HIPCHK(hipMemcpyAsync(g_ens.d_adj, g_ens.h_adj, sizeof(pk::AdjArgs) * n, hipMemcpyHostToDevice, g_stream));
         HIPCHK(hipMemcpyAsync(g_ens.d_sum, g_ens.h_sum.data(), sizeof(pk::SumJob) * 2 * n, hipMemcpyHostToDevice,
                               g_stream));
-        HIPCHK(pk::launch_zero_u32(g_ens.d_queue, pk::kListQueues, g_stream));
         pk::AdjListArgs L{};
         L.args = g_ens.d_adj;
         L.first = g_ens.d_afirst[d];
         L.items = g_ens.d_aitems[d];
         L.nitems = g_ens.anitems[d];
-        L.queue = g_ens.d_queue;
         HIPCHK(pk::launch_sweep_adjoint_list(d, g_mhd, g_cfg.limiter, g_cfg.limiter_b, L, g_stream));
         HIPCHK(pk::launch_sum_parts_jobs(g_ens.d_sum, (int)(2 * n), g_stream));
         for (Block *b : g_list.blocks) b->lcur = 1 - b->lcur;

@@ -63,6 +63,22 @@ __device__ __forceinline__ void fc_points(const SweepArgs &a, int pf, int cs, bo
     }
 }
 
+// One lane's NV values in an LDS array of the tile, lane by lane (NV is odd,
+// so consecutive lanes fall on different banks): one address per lane and
+// neighbour, the variables at immediate offsets, read two at a time.
+template <int NV>
+__device__ __forceinline__ void lds_get(const double *A, int t, double (&x)[NV])
+{
+#pragma unroll
+    for (int v = 0; v < NV; v++) x[v] = A[t * NV + v];
+}
+template <int NV>
+__device__ __forceinline__ void lds_put(double *A, int t, const double (&x)[NV])
+{
+#pragma unroll
+    for (int v = 0; v < NV; v++) A[t * NV + v] = x[v];
+}
+
 // One RK stage of the tile.  A holds primitives then fluxes, B face states.
 // LIM >= 0 fixes both limiters at compile time; LIM < 0 reads them from a.
 // FC: apply the fine/coarse flux points of pencil fc_pf (-1: none) at the
@@ -71,39 +87,41 @@ template <class P, int LIM, bool FC = false>
 __device__ __forceinline__ void tile_stage(const SweepArgs &a, const double (&W)[P::NV],
                                            const double (&W0)[P::NV], double coef, bool upd,
                                            bool lo_end, bool hi_end, double *__restrict__ A,
-                                           double *__restrict__ B, int t, int tm, int tp, int nt,
+                                           double *__restrict__ B, int t, int tm, int tp,
                                            double (&Wn)[P::NV], int fc_pf = -1, int fc_cs = 0,
                                            bool fc_own = false)
 {
     constexpr int NV = P::NV;
-    double q[NV];
-    prim<P>(W, a.gam_1, q);
-#pragma unroll
-    for (int v = 0; v < NV; v++) A[v * nt + t] = q[v];
-    __syncthreads();
-
     double fp[NV];
+    {
+        double q[NV], qm[NV], qp[NV], fm[NV];
+        prim<P>(W, a.gam_1, q);
+        lds_put<NV>(A, t, q);
+        __syncthreads();
+        lds_get<NV>(A, tm, qm);
+        lds_get<NV>(A, tp, qp);
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-        const int lim = (LIM >= 0) ? LIM : ((v < 5) ? a.lim : a.limb);
-        const double dl = q[v] - A[v * nt + tm];
-        const double dr = A[v * nt + tp] - q[v];
-        double dq;
-        if (lo_end)
-            dq = (lim == LIM_VANLEER) ? 0.0 : limit(lim, dr, dr);
-        else if (hi_end)
-            dq = (lim == LIM_VANLEER) ? 0.0 : limit(lim, dl, dl);
-        else
-            dq = limit(lim, dl, dr);
-        const double h = 0.5 * dq;
-        fp[v] = q[v] + h;
-        B[v * nt + t] = q[v] - h;
+        for (int v = 0; v < NV; v++) {
+            const int lim = (LIM >= 0) ? LIM : ((v < 5) ? a.lim : a.limb);
+            const double dl = q[v] - qm[v];
+            const double dr = qp[v] - q[v];
+            double dq;
+            if (lo_end)
+                dq = (lim == LIM_VANLEER) ? 0.0 : limit(lim, dr, dr);
+            else if (hi_end)
+                dq = (lim == LIM_VANLEER) ? 0.0 : limit(lim, dl, dl);
+            else
+                dq = limit(lim, dl, dr);
+            const double h = 0.5 * dq;
+            fp[v] = q[v] + h;
+            fm[v] = q[v] - h;
+        }
+        lds_put<NV>(B, t, fm);
     }
     __syncthreads();
 
     double fr[NV], F[NV];
-#pragma unroll
-    for (int v = 0; v < NV; v++) fr[v] = B[v * nt + tp];
+    lds_get<NV>(B, tp, fr);
     if constexpr (P::MAG)
         flux_hlld(fp, fr, a.gam, a.ch, F);
     else
@@ -111,14 +129,14 @@ __device__ __forceinline__ void tile_stage(const SweepArgs &a, const double (&W)
     if constexpr (FC) {
         if (a.fc_at && fc_pf >= 0) fc_points<P>(a, fc_pf, fc_cs, fc_own, F);
     }
-#pragma unroll
-    for (int v = 0; v < NV; v++) A[v * nt + t] = F[v];
+    lds_put<NV>(A, t, F);
     __syncthreads();
 
+    double Fm[NV];
+    lds_get<NV>(A, tm, Fm);
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-        const double fm = A[v * nt + tm];
-        const double un = upd ? W0[v] + coef * (fm - F[v]) : W[v];
+        const double un = upd ? W0[v] + coef * (Fm[v] - F[v]) : W[v];
         Wn[v] = (v < 5) ? un + 0.0 : un;  // internal_sources adds +0 to the fluid part
     }
 }
@@ -201,31 +219,21 @@ __device__ __forceinline__ void dt_contribution(const SweepArgs &a, const double
     dt_reduce(a, mn, cmax, slot_id);
 }
 
-// Periodic images of a written cell: each ghost cell has exactly one interior
-// pre-image, so writing every output cell's images refreshes all ghosts.
-template <int DIR, class P>
-__device__ __forceinline__ void write_images(const SweepArgs &a, const int (&xyz)[3], long long idx,
-                                             const double (&Wn)[P::NV])
+// Cell index c along the sweep (ghosts included) -> the interior cell a ghost
+// of a block periodic on itself copies (wrap: the sweep reads those instead of
+// the ghosts, which it leaves as they are).
+__device__ __forceinline__ int wrap_cell(int c, int g, int n)
 {
-    int off[3][3], cnt[3];
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        const int ic = xyz[d] - a.g[d];
-        cnt[d] = 1;
-        off[d][0] = 0;
-        if (a.g[d] > 0) {
-            if (ic < a.g[d]) off[d][cnt[d]++] = a.n[d];
-            if (ic >= a.n[d] - a.g[d]) off[d][cnt[d]++] = -a.n[d];
-        }
-    }
-    for (int i0 = 0; i0 < cnt[0]; i0++)
-        for (int i1 = 0; i1 < cnt[1]; i1++)
-            for (int i2 = 0; i2 < cnt[2]; i2++) {
-                if ((i0 | i1 | i2) == 0) continue;
-                const long long j = idx + off[0][i0] + (long long)a.sy * off[1][i1] + (long long)a.sz * off[2][i2];
-#pragma unroll
-                for (int k = 0; k < P::NV; k++) a.dst[(long long)plane_of<DIR>(k) * a.sv + j] = Wn[k];
-            }
+    return c < g ? c + n : (c >= g + n ? c - n : c);
+}
+
+// q = t / d for 0 <= t < 512 and 1 <= d <= 512: (t + 1/2) / d is at least
+// 1/(2 d) > 9e-4 away from a whole number, far more than the roundings of the
+// reciprocal and the product (below 2e-4 at 512); an integer division takes
+// three times the instructions.
+__device__ __forceinline__ int small_div(int t, int d)
+{
+    return (int)(((float)t + 0.5f) * __builtin_amdgcn_rcpf((float)d));
 }
 
 // One tile of a sweep: chunk `bid % chunks` along the sweep direction times
@@ -247,34 +255,54 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs &a, int bid, unsigned
 
     int p, s, tm, tp;
     if (DIR == 0) {
-        s = t % a.TS;
-        p = t / a.TS;
+        p = small_div(t, a.TS);
+        s = t - p * a.TS;
         tm = t - 1;
         tp = t + 1;
     } else {
-        p = t % a.TP;
-        s = t / a.TP;
+        s = small_div(t, a.TP);
+        p = t - s * a.TP;
         tm = t - a.TP;
         tp = t + a.TP;
     }
     tm = tm < 0 ? 0 : tm;
     tp = tp >= nt ? nt - 1 : tp;
 
-    const int chunk = bid % a.chunks;
-    const int ptile = bid / a.chunks;
+    const int ptile = a.chunks == 1 ? bid : bid / a.chunks;
+    const int chunk = bid - ptile * a.chunks;
     const int n1 = a.n[d1];
     const int npen = n1 * a.n[d2];
     const int pf = ptile * a.TP + p;
     const bool pvalid = t < a.TP * a.TS && pf < npen;
-    const int pfc = pf < npen ? pf : npen - 1;
-    const int c1 = a.g[d1] + pfc % n1;
-    const int c2 = a.g[d2] + pfc / n1;
+    // transverse coordinates of pencil pf (of the tile's first one, a uniform
+    // division, then p further along d1); lanes past the last pencil use it
+    int c1, c2;
+    if (a.TP <= n1) {
+        const int p0 = ptile * a.TP;
+        c2 = p0 / n1;
+        c1 = p0 - c2 * n1 + p;
+        if (c1 >= n1) {
+            c1 -= n1;
+            c2++;
+        }
+        if (pf >= npen) {
+            c1 = n1 - 1;
+            c2 = a.n[d2] - 1;
+        }
+    } else {
+        const int pfc = pf < npen ? pf : npen - 1;
+        c2 = pfc / n1;
+        c1 = pfc - c2 * n1;
+    }
+    c1 += a.g[d1];
+    c2 += a.g[d2];
     const int ng = a.ng[ds];
     const int os = (FUSED ? a.g[ds] : 0) + chunk * a.out;
     const int oe = FUSED ? a.g[ds] + a.n[ds] : ng;
     const int cs = os - HALO + s;
     const bool svalid = cs >= 0 && cs < ng;
-    const int csc = cs < 0 ? 0 : (cs >= ng ? ng - 1 : cs);
+    int csc = cs < 0 ? 0 : (cs >= ng ? ng - 1 : cs);
+    if (FUSED && a.wrap) csc = wrap_cell(csc, a.g[ds], a.n[ds]);
     const bool outl = pvalid && s >= HALO && s < HALO + a.out && cs < oe;
 
     int xyz[3];
@@ -295,14 +323,14 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs &a, int bid, unsigned
     unsigned flags = 0u;
     if constexpr (FUSED) {
         double Ws[NV];
-        tile_stage<P, LIM>(a, W, W, a.c1, true, false, false, LA, LB, t, tm, tp, nt, Ws);
+        tile_stage<P, LIM>(a, W, W, a.c1, true, false, false, LA, LB, t, tm, tp, Ws);
         double dm = 0.0;
         unsigned fl = 0u;
         floors<P>(Ws, a.smalld, a.smallei, a.use_smalld, a.use_smallei, a.ei_flag, fl, dm);
         const int g = a.g[ds];
         if (pvalid && s >= 2 && s <= a.TS - 3 && cs >= g - 2 && cs < g + a.n[ds] + 2) flags |= fl;
         pk::mass_add(a.dmass, outl ? dm : 0.0);
-        tile_stage<P, LIM>(a, Ws, W, a.c2, true, false, false, LB, LA, t, tm, tp, nt, Wn);
+        tile_stage<P, LIM>(a, Ws, W, a.c2, true, false, false, LB, LA, t, tm, tp, Wn);
     } else {
         const bool lo = cs == 0, hi = cs == ng - 1;
         if (outl && a.base != a.src) {
@@ -312,7 +340,7 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs &a, int bid, unsigned
 #pragma unroll
             for (int k = 0; k < NV; k++) W0[k] = W[k];
         }
-        tile_stage<P, LIM, true>(a, W, W0, a.c1, !(lo || hi), lo, hi, LA, LB, t, tm, tp, nt, Wn, pvalid ? pf : -1,
+        tile_stage<P, LIM, true>(a, W, W0, a.c1, !(lo || hi), lo, hi, LA, LB, t, tm, tp, Wn, pvalid ? pf : -1,
                                  cs, outl && svalid);
     }
     {
@@ -331,7 +359,6 @@ __device__ __forceinline__ void sweep_tile(const SweepArgs &a, int bid, unsigned
     if (outl && svalid) {
 #pragma unroll
         for (int k = 0; k < NV; k++) a.dst[(long long)plane_of<DIR>(k) * a.sv + idx] = Wn[k];
-        if (FUSED && a.images) write_images<DIR, P>(a, xyz, idx, Wn);
     }
     // negative values are rare: one atomic per lane that saw one
     if (flags) atomicOr(a.flags, flags);
@@ -414,6 +441,7 @@ __global__ __launch_bounds__(64) void k_march(const SweepArgs a)
 
     auto load = [&](int c, double (&W)[NV]) {
         c = c < t0 ? t0 : (c >= t1 ? t1 - 1 : c);
+        if (a.wrap) c = wrap_cell(c, g, n);
         const long long o = base + step * c;
 #pragma unroll
         for (int k = 0; k < NV; k++) W[k] = a.src[(long long)plane_of<DIR>(k) * a.sv + o];
@@ -476,11 +504,9 @@ __global__ __launch_bounds__(64) void k_march(const SweepArgs a)
             if (a.dtslots && pvalid) dt_cell<DIR, P>(a, Wn, mn, cmax);
             if constexpr (P::MAG) Wn[8] = Wn[8] * a.psi_fac;
             if (pvalid) {
-                xyz[ds] = c;
                 const long long idx = base + step * c;
 #pragma unroll
                 for (int k = 0; k < NV; k++) a.dst[(long long)plane_of<DIR>(k) * a.sv + idx] = Wn[k];
-                if (a.images) write_images<DIR, P>(a, xyz, idx, Wn);
             }
         }
         // advance the window
@@ -499,10 +525,10 @@ __global__ __launch_bounds__(64) void k_march(const SweepArgs a)
 
 // The kernel arguments of list item `item` (its block's table entry with
 // the step's scalars and buffer parity applied); returns the block's first
-// item.  The tables are read-only while a kernel runs: they are read through
+// item, and in `next` the first item past it.  The tables are read-only while a kernel runs: they are read through
 // the constant address space, so the uniform loads go to scalar registers.
 template <int DIR>
-__device__ __forceinline__ unsigned load_list_args(const ListArgs &L, unsigned item, SweepArgs &a)
+__device__ __forceinline__ unsigned load_list_args(const ListArgs &L, unsigned item, SweepArgs &a, unsigned &next)
 {
     typedef const __attribute__((address_space(4))) unsigned cu32;
     const int blk = __builtin_amdgcn_readfirstlane((int)((cu32 *)L.items)[item]);
@@ -514,7 +540,7 @@ __device__ __forceinline__ unsigned load_list_args(const ListArgs &L, unsigned i
         for (int i = 0; i < (int)(sizeof(SweepArgs) / 4); i++) aw[i] = w[i];
     }
     const unsigned first = ((cu32 *)L.first)[blk];
-    if (L.no_wrap && a.images == 2) a.images = 1;
+    next = ((cu32 *)L.first)[blk + 1];
     if (L.parity) {
         const double *s0 = a.src;
         a.src = a.dst;
@@ -536,46 +562,27 @@ __device__ __forceinline__ unsigned load_list_args(const ListArgs &L, unsigned i
 
 #include "pk_stream.hpp"
 
-// The hydro sweep fits four waves per SIMD in 128 VGPRs (2 spilled; 5 % faster
-// at 128^3 than three waves); the MHD sweep keeps its two (227-256 VGPRs).
+// Hydro tiles hold five waves per SIMD (86 VGPRs), fused MHD tiles are held to
+// three (168 VGPRs, 8-10 of them spilled; unconstrained 175-185, two waves):
+// four steps of a 131x98x77 MHD block took 4020 us with two, 3770 with three.
+// The one-stage MHD sweep would spill 24 and keeps two (100 against 90 us).
 template <int DIR, class P, bool FUSED, int LIM>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(P::MAG ? 1 : 4))) void k_sweep(const SweepArgs a)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(P::MAG ? (FUSED ? 3 : 2) : 5))) void k_sweep(const SweepArgs a)
 {
     extern __shared__ double lds[];
-    // XCD-aware order: workgroup i runs on XCD i % 8, so give each XCD a
-    // contiguous range of tiles; tiles that share halo cells then share an L2.
-    int bid = blockIdx.x;
-    const int nfull = (int)(gridDim.x / 8u) * 8;
-    if (bid < nfull) bid = (bid % 8) * (nfull / 8) + bid / 8;
-    sweep_tile<DIR, P, FUSED, LIM>(a, bid, blockIdx.x, lds, lds + P::NV * blockDim.x);
+    sweep_tile<DIR, P, FUSED, LIM>(a, (int)pk::xcd_order(), blockIdx.x, lds, lds + P::NV * blockDim.x);
 }
 
-// Persistent fused sweep over a block list.  Each workgroup takes the next
-// `grab` tiles from the queue (one atomic per fetch), and for each loads
-// that block's arguments and runs the tile; it leaves when the queue is
-// empty, so every workgroup ends after at most nitems / grab + gridDim.x
-// fetches in total.
+// Fused sweep over a block list, a tile per workgroup.
 template <int DIR, class P, int LIM>
-__global__ __launch_bounds__(512) void k_sweep_list(const ListArgs L)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(P::MAG ? 3 : 5))) void k_sweep_list(const ListArgs L)
 {
     extern __shared__ double lds[];
-    __shared__ unsigned s_item;
-    const unsigned grab = L.grab > 1u ? L.grab : 1u;
-    unsigned item = 0u, end = 0u;
-    for (;;) {
-        __syncthreads();  // the previous tile is done with LDS and s_item
-        if (item >= end) {
-            if (threadIdx.x == 0) s_item = atomicAdd(L.queue, grab);
-            __syncthreads();
-            item = (unsigned)__builtin_amdgcn_readfirstlane((int)s_item);
-            if (item >= L.nitems) break;
-            end = min(item + grab, L.nitems);
-        }
-        SweepArgs a;
-        const unsigned first = load_list_args<DIR>(L, item, a);
-        sweep_tile<DIR, P, true, LIM>(a, (int)(item - first), item, lds, lds + P::NV * blockDim.x);
-        item++;
-    }
+    const unsigned item = L.item0 + pk::xcd_order();
+    SweepArgs a;
+    unsigned next;
+    const unsigned first = load_list_args<DIR>(L, item, a, next);
+    sweep_tile<DIR, P, true, LIM>(a, (int)(item - first), item, lds, lds + P::NV * blockDim.x);
 }
 
 // ------------------------------------------------------------ launchers ----
@@ -634,8 +641,7 @@ static int stream_slots(const void *fn, int *cache)
 // launch of more ranges than the device holds at once runs in rounds; it is
 // rounded to a whole number of rounds, the ranges made equal to within one
 // group, so that the last round does not leave the device partly idle.
-// IMG: the kernel that writes periodic ghost images (a.images == 1).
-template <int DIR, class P, int LIM, int TP, bool IMG>
+template <int DIR, class P, int LIM, int TP>
 static hipError_t launch_stream_tp(const SweepArgs &a, hipStream_t st)
 {
     constexpr int d1 = (DIR == 0) ? 1 : 0, d2 = (DIR == 2) ? 1 : 2;
@@ -648,7 +654,7 @@ static hipError_t launch_stream_tp(const SweepArgs &a, hipStream_t st)
         return hipErrorInvalidValue;
     long long nblk = (npos + span - 1) / span;
     if (nblk != a.ptiles) return hipErrorInvalidValue;
-    const void *fn = (const void *)k_stream<DIR, P, LIM, TP, IMG>;
+    const void *fn = (const void *)k_stream<DIR, P, LIM, TP>;
     static int cache[kMaxDevices] = {};
     const long long slots = stream_slots(fn, cache);
     if (slots > 0 && nblk >= slots) {
@@ -657,19 +663,18 @@ static hipError_t launch_stream_tp(const SweepArgs &a, hipStream_t st)
         while (r > 1 && r * slots > ngroups) r--;
         nblk = r * slots;
     }
-    hipLaunchKernelGGL((k_stream<DIR, P, LIM, TP, IMG>), dim3((unsigned)nblk), dim3(64), 0, st, a, (int)ngroups);
+    hipLaunchKernelGGL((k_stream<DIR, P, LIM, TP>), dim3((unsigned)nblk), dim3(64), 0, st, a, (int)ngroups);
     return hipGetLastError();
 }
 
 template <int DIR, class P, int LIM>
 static hipError_t launch_stream_t(const SweepArgs &a, hipStream_t st)
 {
-    const bool img = a.images == 1;
     switch (a.TP) {
-    case 1: return img ? launch_stream_tp<DIR, P, LIM, 1, true>(a, st) : launch_stream_tp<DIR, P, LIM, 1, false>(a, st);
-    case 2: return img ? launch_stream_tp<DIR, P, LIM, 2, true>(a, st) : launch_stream_tp<DIR, P, LIM, 2, false>(a, st);
-    case 4: return img ? launch_stream_tp<DIR, P, LIM, 4, true>(a, st) : launch_stream_tp<DIR, P, LIM, 4, false>(a, st);
-    case 8: return img ? launch_stream_tp<DIR, P, LIM, 8, true>(a, st) : launch_stream_tp<DIR, P, LIM, 8, false>(a, st);
+    case 1: return launch_stream_tp<DIR, P, LIM, 1>(a, st);
+    case 2: return launch_stream_tp<DIR, P, LIM, 2>(a, st);
+    case 4: return launch_stream_tp<DIR, P, LIM, 4>(a, st);
+    case 8: return launch_stream_tp<DIR, P, LIM, 8>(a, st);
     default: return hipErrorInvalidValue;
     }
 }
@@ -717,8 +722,6 @@ static hipError_t launch_lim(const SweepArgs &a, hipStream_t st)
 
 hipError_t launch_sweep(int dir, bool mhd, bool fused, const SweepArgs &a, hipStream_t st)
 {
-    // reading ghost positions from their interior pre-images is the stream kernel's only
-    if (a.images == 2 && !(fused && a.TS <= -2)) return hipErrorInvalidValue;
 #define PK_CASE(D, PP, F) \
     if (dir == D && (mhd == PP::MAG) && fused == F) return launch_lim<D, PP, F>(a, st);
     PK_CASE(0, HD, true) PK_CASE(1, HD, true) PK_CASE(2, HD, true)
@@ -729,10 +732,9 @@ hipError_t launch_sweep(int dir, bool mhd, bool fused, const SweepArgs &a, hipSt
     return hipErrorInvalidValue;
 }
 
-// Persistent list sweep: launch (resident == nullptr) or report how many
-// workgroups of nt lanes the device holds at once.
-// Persistent stream over a list (nt == 64: k_stream_list, one pencil per
-// lane group along x, eight along y and z).
+// List sweep: launch (resident == nullptr) or report how many workgroups of nt
+// lanes the device holds at once.  nt == 64: the stream (k_stream_list, one
+// pencil per lane group along x, eight along y and z).
 template <int DIR, class P, int LIM>
 static hipError_t stream_list_t(const ListArgs *L, int grid, hipStream_t st, int *resident)
 {
@@ -757,7 +759,7 @@ static hipError_t list_t(const ListArgs *L, int nt, int grid, hipStream_t st, in
     if (nt == pk::kStreamListNt) return stream_list_t<DIR, P, LIM>(L, grid, st, resident);
     const void *fn = (const void *)k_sweep_list<DIR, P, LIM>;
     const size_t lds = sizeof(double) * 2 * P::NV * nt;
-    const size_t lds_max = 160 * 1024 - 256;  // static LDS (the queue slot) comes out of the same 160 KiB
+    const size_t lds_max = 160 * 1024;
     static bool lds_raised = false;
     if (!lds_raised) {
         hipError_t e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max);
@@ -773,8 +775,12 @@ static hipError_t list_t(const ListArgs *L, int nt, int grid, hipStream_t st, in
         *resident = per * ncu;
         return e;
     }
-    if (grid <= 0) return hipErrorInvalidValue;
-    hipLaunchKernelGGL((k_sweep_list<DIR, P, LIM>), dim3((unsigned)grid), dim3(nt), lds, st, *L);
+    ListArgs l = *L;
+    for (; l.item0 < L->nitems; l.item0 += pk::kListPiece) {
+        const unsigned n = L->nitems - l.item0 < pk::kListPiece ? L->nitems - l.item0 : pk::kListPiece;
+        hipLaunchKernelGGL((k_sweep_list<DIR, P, LIM>), dim3(n), dim3(nt), lds, st, l);
+        if (l.item0 + n == L->nitems) break;  // (the next item0 may not fit 32 bits)
+    }
     return hipGetLastError();
 }
 
@@ -811,11 +817,12 @@ static hipError_t list_dispatch(int dir, bool mhd, int lim, int limb, const List
 hipError_t launch_sweep_list(int dir, bool mhd, int lim, int limb, const ListArgs &L, int nt, int grid,
                              hipStream_t st)
 {
-    if (grid <= 0) {
+    if (nt == pk::kStreamListNt && grid <= 0) {
         int r = 0;
         hipError_t e = list_dispatch(dir, mhd, lim, limb, &L, nt, 0, st, &r);
         if (e != hipSuccess) return e;
         grid = r > 0 ? r : 1;
+        if (L.nitems < (unsigned)grid) grid = L.nitems > 0 ? (int)L.nitems : 1;
     }
     return list_dispatch(dir, mhd, lim, limb, &L, nt, grid, st, nullptr);
 }
@@ -826,6 +833,5 @@ int sweep_list_resident(int dir, bool mhd, int lim, int limb, int nt)
     if (list_dispatch(dir, mhd, lim, limb, nullptr, nt, 0, nullptr, &r) != hipSuccess) return 0;
     return r;
 }
-
 
 }  // namespace PK_KNS

@@ -34,9 +34,8 @@ struct SweepArgs {
     unsigned *flags;     // device: bit 0 negative density, bit 1 negative internal energy
     unsigned long long *dmass;  // device: floor-added mass / cell volume, exact counters (pk_mass.hpp)
     // fused mode only:
-    int images;          // 1: also write every output cell's periodic ghost images (one periodic block);
-                         // 2 (stream kernels): read each ghost position's interior pre-image instead
-                         // and write no images (the ghosts are left stale)
+    int wrap;            // 1: read each ghost position's interior pre-image (a block periodic on itself)
+                         // instead of the ghost; no sweep writes ghosts
     unsigned long long *dtslots;  // if set: per slot, min of dl_d/c_d (d = x, y, z) and max c of the
                                   // cells written, as FP64 bit patterns (timestep_fluid of the next step)
     int nslots;
@@ -90,15 +89,37 @@ struct StepScalars {
     double pad;
 };
 
-// One persistent launch over a block list: workgroups take tiles from a
-// device queue until it is empty.  Tile `item` belongs to block items[item]
-// and is that block's tile item - first[block].
+#if defined(__HIPCC__)
+// This workgroup's place in an XCD-aware order: workgroup i runs on XCD i % 8,
+// so each XCD gets a contiguous range of places, and tiles that share halo
+// cells or cache lines share an L2.
+__device__ __forceinline__ unsigned xcd_order()
+{
+    const unsigned full = gridDim.x / 8u * 8u, w = blockIdx.x;
+    return w < full ? (w % 8u) * (full / 8u) + w / 8u : w;
+}
+#endif
+
+// Most workgroups of one list launch (the runtime takes fewer than 2^32
+// lanes); longer lists take several launches.
+constexpr unsigned kListPiece = 1u << 22;
+
+// One launch over a block list, an item per workgroup (k_sweep_list,
+// k_sweep_adjoint_list; k_stream_list walks a range of items).  Item `item`
+// belongs to block items[item] and is that block's tile (or range of its
+// stream) item - first[block].  The hardware hands the workgroups out: with
+// resident workgroups taking items from a queue, or each walking a fixed range
+// of them, a sweep of 6 MHD blocks of 81x64x45 (12 launches of them in a step) is
+// limited by the latency of a workgroup's successive tiles and by the block
+// arguments a loop keeps in scalar registers (40 spilled); a step took 935 us
+// with queues, 821 with ranges, 727 an item a workgroup (48 blocks of two
+// fluids: 3190, 2950, 2427; 20 2-D blocks: 369, 355, 280).
 struct ListArgs {
     const SweepArgs *args;   // per block: geometry, pointers (src = buffer 0), tile shape
     const unsigned *first;   // per block: first item (nblocks + 1 entries)
     const unsigned *items;   // per item: block index
     unsigned nitems;
-    unsigned *queue;         // item counter, zero before the launch
+    unsigned item0;          // first item of the launch
     int parity;              // 1: read buffer 1, write buffer 0
     int apply_fac;           // multiply psi by step->psi_fac
     const StepScalars *step;      // one for the whole list, or one per block (per_block)
@@ -107,8 +128,6 @@ struct ListArgs {
     int per_block;                // independent instances: each block has its own dt, ch, psi factor
                                   // and its own nslots dt slots
     const unsigned *bpos;         // per_block: each block's position among the instances (null: its index)
-    int no_wrap;                  // blocks with images == 2 write their images instead (ghosts kept current)
-    unsigned grab;                // consecutive items taken per queue fetch (0 or 1: one)
 };
 
 // One device-to-device copy of a batch (k_copy_blocks).
@@ -146,7 +165,7 @@ struct PlanesArgs {
 };
 
 hipError_t launch_sweep(int dir, bool mhd, bool fused, const SweepArgs &a, hipStream_t st);
-// Workgroup size that selects the stream form of the persistent list sweep
+// Workgroup size that selects the stream form of the list sweep
 // (k_stream_list: one-wave workgroups, each list item a range of a block's
 // stream of a.out positions, a.TP pencils per lane group: 1 along x, 8 along
 // y and z).
@@ -157,8 +176,9 @@ constexpr int stream_list_tp(int d) { return d == 0 ? 1 : 8; }
 // resources over three planes each, whose byte ranges (24 sv) must stay
 // below 2^31.
 constexpr bool stream_stores_fit(long long sv) { return sv >= 0 && 24 * sv < (1ll << 31); }
-// Persistent batched fused sweep with workgroups of nt lanes; grid = 0 picks
-// the number of workgroups the device holds at once.
+// Batched fused sweep with workgroups of nt lanes: a tile each, or, for the
+// stream, grid of them, a range of items each (grid = 0: as many as the device
+// holds at once, at most one per item).
 hipError_t launch_sweep_list(int dir, bool mhd, int lim, int limb, const ListArgs &L, int nt, int grid,
                              hipStream_t st);
 int sweep_list_resident(int dir, bool mhd, int lim, int limb, int nt);

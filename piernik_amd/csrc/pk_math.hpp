@@ -189,76 +189,63 @@ PK_HD void prim(const double (&u)[P::NV], double gam_1, double (&q)[P::NV])
 }
 
 // HLLC (riemann_hlld_u, adiabatic) for one interface.  l, r: primitive face
-// states; f: fluxes of rho, m_n, m_t1, m_t2, E.
+// states; f: fluxes of rho, m_n, m_t1, m_t2, E.  Energy, flux and star state
+// are formed for the one side the interface needs (both only for the sm == 0
+// average): its inputs are selected first.
 PK_HD void flux_hllc(const double *l, const double *r, double gam, double *f)
 {
-    const double prl = l[4], prr = r[4];
-    const double enl = qdiv(l[4], gam - 1.0) + (0.5 * l[0]) * ((l[1] * l[1] + l[2] * l[2]) + l[3] * l[3]);
-    const double enr = qdiv(r[4], gam - 1.0) + (0.5 * r[0]) * ((r[1] * r[1] + r[2] * r[2]) + r[3] * r[3]);
     const double c = qsqrt(fmx(qdiv(gam * l[4], l[0]), qdiv(gam * r[4], r[0])));
     const double sl = fmn(l[1], r[1]) - c;
     const double sr = fmx(l[1], r[1]) + c;
-
-    double fl[5], fr[5];
-    fl[0] = l[0] * l[1];
-    fl[1] = l[0] * (l[1] * l[1]) + prl;
-    fl[2] = (l[0] * l[2]) * l[1];
-    fl[3] = (l[0] * l[3]) * l[1];
-    fl[4] = (enl + prl) * l[1];
-    fr[0] = r[0] * r[1];
-    fr[1] = r[0] * (r[1] * r[1]) + prr;
-    fr[2] = (r[0] * r[2]) * r[1];
-    fr[3] = (r[0] * r[3]) * r[1];
-    fr[4] = (enr + prr) * r[1];
-
-    if (sl >= 0.0) {
-#pragma unroll
-        for (int v = 0; v < 5; v++) f[v] = fl[v];
-        return;
+    const bool upl = sl >= 0.0, up = upl || sr <= 0.0;  // supersonic: the upwind physical flux
+    bool L = upl;
+    double sm = 0.0, dn_l = 0.0, dn_r = 0.0, prt_star = 0.0;
+    if (!up) {
+        const double auxr = (sr - r[1]) * r[0], auxl = (sl - l[1]) * l[0];
+        sm = (fabs(auxr - auxl) < spacing(auxr + auxl))
+                 ? (sl + sr) / 2.0
+                 : qdiv((auxr * r[1] - r[4]) - (auxl * l[1] - l[4]), auxr - auxl);
+        dn_l = l[0] * (sl - l[1]);
+        dn_r = r[0] * (sr - r[1]);
+        prt_star = 0.5 * ((l[4] + dn_l * (sm - l[1])) + (r[4] + dn_r * (sm - r[1])));
+        L = sm > 0.0;
     }
-    if (sr <= 0.0) {
-#pragma unroll
-        for (int v = 0; v < 5; v++) f[v] = fr[v];
-        return;
-    }
-    const double auxr = (sr - r[1]) * r[0], auxl = (sl - l[1]) * l[0];
-    const double sm = (fabs(auxr - auxl) < spacing(auxr + auxl))
-                          ? (sl + sr) / 2.0
-                          : qdiv((auxr * r[1] - prr) - (auxl * l[1] - prl), auxr - auxl);
-    const double slvxl = sl - l[1], srvxr = sr - r[1];
-    const double dn_l = l[0] * slvxl, dn_r = r[0] * srvxr;
-    const double prt_star = 0.5 * ((prl + dn_l * (sm - l[1])) + (prr + dn_r * (sm - r[1])));
-    if (sm != 0.0) {
-        // one side only: pick its inputs, then evaluate the reference's
-        // formula once (hlld.F90:771-815)
-        const bool L = sm > 0.0;
-        const double s_ = L ? sl : sr;
-        const double svx = L ? slvxl : srvxr;
-        const double en = L ? enl : enr;
-        const double pr = L ? prl : prr;
-        const double dn = L ? dn_l : dn_r;
-        const double* q = L ? l : r;
-        const double* f0 = L ? fl : fr;
-        const double ssm = s_ - sm;
+    // physical flux, conserved state and, with w, star flux f0 + s*(us - U) of
+    // side q (hlld.F90:771-815)
+    auto side = [&](const double *q, double s_, double dn, bool w, double *o) {
+        const double en = qdiv(q[4], gam - 1.0) + (0.5 * q[0]) * ((q[1] * q[1] + q[2] * q[2]) + q[3] * q[3]);
+        o[0] = q[0] * q[1];
+        o[1] = q[0] * (q[1] * q[1]) + q[4];
+        o[2] = (q[0] * q[2]) * q[1];
+        o[3] = (q[0] * q[3]) * q[1];
+        o[4] = (en + q[4]) * q[1];
+        if (!w) return;
+        const double ssm = s_ - sm, svx = s_ - q[1];
         const double d = qdiv(dn, ssm);
-        const double us[5] = {d, d * sm, d * q[2], d * q[3], qdiv(((svx * en) - (pr * q[1])) + (prt_star * sm), ssm)};
+        const double us[5] = {d, d * sm, d * q[2], d * q[3], qdiv(((svx * en) - (q[4] * q[1])) + (prt_star * sm), ssm)};
         const double U[5] = {q[0], q[0] * q[1], q[0] * q[2], q[0] * q[3], en};
 #pragma unroll
-        for (int v = 0; v < 5; v++) f[v] = f0[v] + s_ * (us[v] - U[v]);
-    } else {
-        // sm == 0: half*(fl + sl*(us_l - U_l) + fr + sr*(us_r - U_r)), hlld.F90:822
-        const double slsm = sl - sm, srsm = sr - sm;
-        const double dl_ = dn_l / slsm, dr_ = dn_r / srsm;
-        const double usl[5] = {dl_, dl_ * sm, dl_ * l[2], dl_ * l[3],
-                               (((slvxl * enl) - (prl * l[1])) + (prt_star * sm)) / slsm};
-        const double usr[5] = {dr_, dr_ * sm, dr_ * r[2], dr_ * r[3],
-                               (((srvxr * enr) - (prr * r[1])) + (prt_star * sm)) / srsm};
-        const double Ul[5] = {l[0], l[0] * l[1], l[0] * l[2], l[0] * l[3], enl};
-        const double Ur[5] = {r[0], r[0] * r[1], r[0] * r[2], r[0] * r[3], enr};
+        for (int v = 0; v < 5; v++) o[v] = o[v] + s_ * (us[v] - U[v]);
+    };
+    if (!up && sm == 0.0) {
+        // half*(fl + sl*(us_l - U_l) + fr + sr*(us_r - U_r)), hlld.F90:822
+        double a[5], b[5];
+        side(l, sl, dn_l, true, a);
+        side(r, sr, dn_r, false, b);
+        // the reference adds fr before the right star term
+        const double en = qdiv(r[4], gam - 1.0) + (0.5 * r[0]) * ((r[1] * r[1] + r[2] * r[2]) + r[3] * r[3]);
+        const double ssm = sr - sm, d = dn_r / ssm;
+        const double us[5] = {d, d * sm, d * r[2], d * r[3],
+                              ((((sr - r[1]) * en) - (r[4] * r[1])) + (prt_star * sm)) / ssm};
+        const double U[5] = {r[0], r[0] * r[1], r[0] * r[2], r[0] * r[3], en};
 #pragma unroll
-        for (int v = 0; v < 5; v++)
-            f[v] = 0.5 * (((fl[v] + sl * (usl[v] - Ul[v])) + fr[v]) + sr * (usr[v] - Ur[v]));
+        for (int v = 0; v < 5; v++) f[v] = 0.5 * ((a[v] + b[v]) + sr * (us[v] - U[v]));
+        return;
     }
+    double q[5];
+#pragma unroll
+    for (int v = 0; v < 5; v++) q[v] = L ? l[v] : r[v];
+    side(q, L ? sl : sr, L ? dn_l : dn_r, !up, f);
 }
 
 // One side of an HLLD interface: face state q = [rho, v_n, v_t1, v_t2, p,

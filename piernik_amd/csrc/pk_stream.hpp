@@ -102,11 +102,8 @@ __host__ __device__ constexpr int stream_stride()
 // of the calling workgroup.  AK (NV * stream_stride<TP>()) and U
 // (NV * stream_su<TP>()) are the workgroup's LDS; the wave's earlier
 // contents there are never read for an owned output.  slot_id picks the
-// timestep slot.  IMG: 1 the launch writes periodic ghost images
-// (a.images == 1), 0 it writes none (a.images 0 or 2), -1 as a.images says
-// (lists, whose blocks differ); a fixed IMG keeps the image code, and the
-// registers it holds, out of kernels that never run it.
-template <int DIR, class P, int LIM, int TP, int IMG>
+// timestep slot.
+template <int DIR, class P, int LIM, int TP>
 __device__ __forceinline__ void stream_range(const SweepArgs &a, const int s0, const int span, unsigned slot_id,
                                              double *AK, double *U)
 {
@@ -196,12 +193,12 @@ __device__ __forceinline__ void stream_range(const SweepArgs &a, const int s0, c
     // the stream or past the last pencil read a valid cell of the block
     // (wrap: a ghost position reads the interior cell it images, for a block
     // periodic on itself whose ghosts this launch leaves unwritten)
-    const bool wrap = a.images == 2;
+    const bool wrap = a.wrap != 0;
     const int n = a.n[ds];
     auto cell_index = [&](int jj, bool &pv, bool wr) -> long long {
         pv = grp >= 0 && (grp * TP + p) < npen;
         const int cc1 = pv ? c1 : 0, cc2 = pv ? c2 : 0;
-        if (wr) jj = (jj < 4) ? jj + n : ((jj >= n + 4) ? jj - n : jj);
+        if (wr) jj = wrap_cell(jj, 4, n);
         int xyz[3];
         xyz[ds] = a.g[ds] - 4 + jj;
         xyz[d1] = a.g[d1] + cc1;
@@ -381,16 +378,7 @@ __device__ __forceinline__ void stream_range(const SweepArgs &a, const int s0, c
             pk::mass_add(a.dmass, out ? dm : 0.0);
             if constexpr (P::MAG) Wn[8] = Wn[8] * a.psi_fac;
             const long long oidx = idx - 4 * st;
-            if (out) {
-                if (a.dtslots) dt_cell<DIR, P>(a, Wn, mn, cmax);
-                if ((IMG < 0) ? (a.images == 1) : (IMG == 1)) {
-                    int xyz[3];
-                    xyz[ds] = g - 4 + jo;
-                    xyz[d1] = a.g[d1] + cc1;
-                    xyz[d2] = a.g[d2] + cc2;
-                    write_images<DIR, P>(a, xyz, oidx, Wn);
-                }
-            }
+            if (out && a.dtslots) dt_cell<DIR, P>(a, Wn, mn, cmax);
             // every lane issues the stores: a lane without an output stores
             // past the end of the plane's buffer range, which the hardware drops
             const PlaneStores<NV> ps(a.dst, a.sv);
@@ -416,7 +404,7 @@ __device__ __forceinline__ void stream_range(const SweepArgs &a, const int s0, c
 // Both stream kernels are held to two waves per SIMD (256 registers): at
 // 253-256 VGPRs the allocator otherwise spills into AGPRs for some template
 // instances and halves their occupancy.
-template <int DIR, class P, int LIM, int TP, bool IMG>
+template <int DIR, class P, int LIM, int TP>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_stream(const SweepArgs a,
                                                                                      const int ngroups)
 {
@@ -432,26 +420,28 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     if (bid < nfull) bid = (bid % 8) * (nfull / 8) + bid / 8;
     const int L = a.n[DIR] + 8;
     const int g0 = (int)((long long)bid * ngroups / gridDim.x), g1 = (int)((long long)(bid + 1) * ngroups / gridDim.x);
-    stream_range<DIR, P, LIM, TP, IMG ? 1 : 0>(a, g0 * L, (g1 - g0) * L, blockIdx.x, AK, U);
+    stream_range<DIR, P, LIM, TP>(a, g0 * L, (g1 - g0) * L, blockIdx.x, AK, U);
 }
 
-// The stream over a block list: one-wave workgroups take items from a
-// device queue until it is empty; item `item` of block items[item] is the
-// range of a.out positions starting at (item - first[block]) * a.out of
-// that block's stream.  Each wave leaves after its first fetch past the
-// end, so the grid drains after at most nitems + gridDim.x fetches.
+// The stream over a block list: item `item` of block items[item] is the range
+// of a.out positions starting at (item - first[block]) * a.out of that block's
+// stream.  Each one-wave workgroup walks a contiguous range of the items, equal
+// to within one, and those of a block in it as one range, so that the stream's
+// start-up (a group's two halos) is paid once per block and workgroup.
 template <int DIR, class P, int LIM, int TP>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_stream_list(const ListArgs L)
 {
     __shared__ double AK[P::NV * stream_stride<TP>()];
     __shared__ double U[P::NV * stream_su<TP>()];
-    for (;;) {
-        unsigned got = 0u;
-        if (threadIdx.x == 0) got = atomicAdd(L.queue, 1u);
-        const unsigned item = (unsigned)__builtin_amdgcn_readfirstlane((int)__shfl((int)got, 0, 64));
-        if (item >= L.nitems) break;
+    const unsigned w = pk::xcd_order();
+    unsigned item = (unsigned)((unsigned long long)L.nitems * w / gridDim.x);
+    const unsigned hi = (unsigned)((unsigned long long)L.nitems * (w + 1u) / gridDim.x);
+    while (item < hi) {
         SweepArgs a;
-        const unsigned first = load_list_args<DIR>(L, item, a);
-        stream_range<DIR, P, LIM, TP, -1>(a, (int)(item - first) * a.out, a.out, item, AK, U);
+        unsigned next;
+        const unsigned first = load_list_args<DIR>(L, item, a, next);
+        next = min(next, hi);
+        stream_range<DIR, P, LIM, TP>(a, (int)(item - first) * a.out, (int)(next - item) * a.out, item, AK, U);
+        item = next;
     }
 }

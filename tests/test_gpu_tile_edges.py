@@ -1,0 +1,80 @@
+"""Sweep tiles at their edges: lengths either side of where the default shape
+changes (whole pencil, two chunks, three pencils a tile, few pencils), blocks
+as short as their ghosts (every halo is read from its pre-image in the
+interior, which wraps more than once), pencils that leave the last tile
+partly empty, and lists whose launches have fewer items than CUs.
+
+Bit for bit against the oracle, as the rest of the exact build.  A pinned
+tile runs beside the default: a tile changes who computes a cell, never how.
+"""
+import numpy as np
+import pytest
+
+import piernik_amd as pk
+from piernik_amd import setups
+
+pytestmark = pytest.mark.gpu
+
+# (shape, active directions)
+BLOCKS = [((4, 4, 4), (True, True, True)), ((5, 4, 9), (True, True, True)), ((77, 6, 5), (True, True, True)),
+          ((6, 78, 5), (True, True, True)), ((249, 4, 4), (True, True, True)), ((7, 5, 57), (True, True, True)),
+          ((40, 36, 33), (True, True, True)), ((124, 5, 1), (True, True, False)), ((9, 65, 1), (True, True, False)),
+          ((300, 1, 1), (True, False, False))]
+
+
+def assert_same(cg, ob, where):
+    for name in ("u", "b", "psi"):
+        a, o = getattr(cg, name), getattr(ob, name)
+        if a is None:
+            continue
+        bad = np.argwhere(~(a == o))
+        assert bad.size == 0, f"{where} {name}: {len(bad)} differ, first at {tuple(bad[0])}"
+
+
+@pytest.mark.parametrize("mag", [False, True])
+@pytest.mark.parametrize("shape,has_dir", BLOCKS)
+def test_block_tiles_bit_exact(oracle, shape, has_dir, mag):
+    out = None
+    # default; tiles of one and several pencils; (1D: no y, z); whole pencils (march); streams
+    for tile in [(0, 0), (1, 9), (7, 23), (64, -1), (2, -3)]:
+        cfg = pk.Config(magnetized=mag, limiter="vanleer", smalld=1e-3, smallei=1e-4, has_dir=has_dir,
+                        tile_x=tile, tile_yz=tile)
+        print(f"block {shape} magnetized {mag} tile {tile}", flush=True)
+        pk.load_library()
+        pk.finalize()
+        pk.init(cfg)
+        cg = setups.smooth_random(shape, nb=4, seed=sum(shape), magnetized=mag, gamma=cfg.gamma, has_dir=has_dir)
+        if out is None:
+            out = oracle.OBlock.from_cg(cg)
+            t_o = oracle.run(oracle.params_from_config(cfg), out, 2)
+        cg.upload()
+        t_g, _ = pk.run(cg, 2)
+        cg.download()
+        assert t_g == t_o
+        assert_same(cg, out, f"{shape} {tile}")
+        pk.finalize()
+
+
+@pytest.mark.parametrize("lanes,ts", [(0, 0), (64, -2), (128, 0), (256, 9), (512, 0)])
+@pytest.mark.parametrize("shapes", [[(4, 4, 4)], [(5, 6, 4), (33, 30, 34), (4, 77, 5)]])
+def test_list_items_bit_exact(oracle, shapes, lanes, ts):
+    cfg = setups.batch_config(fluids=((5.0 / 3.0, True), (1.4, False)))
+    cgs = setups.batch_blocks(shapes, cfg, seed=5)
+    obs = [oracle.OBlock.from_cg(c) for c in cgs]
+    print(f"list {shapes} lanes {lanes} ts {ts}", flush=True)
+    pk.load_library()
+    pk.finalize()
+    pk.init(cfg)
+    for cg in cgs:
+        cg.registered = False
+        cg.upload()
+    if lanes:
+        for d in range(3):
+            for f in range(2):
+                pk.set_list_tiles(d, f, lanes, ts)
+    t_g, _ = pk.run_all(2)
+    assert t_g == oracle.run_list(oracle.params_from_config(cfg), obs, 2)
+    for cg, ob in zip(cgs, obs):
+        cg.download()
+        assert_same(cg, ob, f"list {cg.n}")
+    pk.finalize()
