@@ -321,48 +321,16 @@ void march_geometry(const Block *b, int d, int &TP, int &out, int &chunks, int &
     out = b->n[d];
 }
 
-// The tile along d of at most nt lanes that needs the fewest workgroups: over
-// the pencil counts tp, the pencil in equal chunks of the longest tile that
-// fits.  Returns the workgroups.  Along x ties go to the longer tile (fewer
-// halo cells read).  Along y and z the lanes of a tile read tp cells in a row,
-// so at least 3 pencils are taken and ties go to the longest tile of 4 or more
-// (HD 224^3, y, 256 lanes: 4x64 575 us, 2x120 586, 1x232 > 640; HD 96^3, y:
-// 4x56 62 us, 2x104 65; MHD 131x98x77, y: 4x57 140 us, 2x106 147).
-long long even_tile(const Block *b, int d, bool fused, int nt, int &tp_out, int &ts_out)
+// even_tile and full_tile of a block's pencils along d: halo 4 (fused) or 2 (one stage)
+long long even_tile(const Block *b, int d, bool fused, int nt, int &tp, int &ts)
 {
-    const int halo = fused ? 4 : 2;
-    const int span = fused ? b->n[d] : b->ng[d];
     const int d1 = (d == 0) ? 1 : 0, d2 = (d == 2) ? 1 : 2;
-    const long long npen = (long long)b->n[d1] * b->n[d2];
-    long long best = -1;
-    tp_out = 1;
-    ts_out = 2 * halo + 1;
-    const int tp0 = d == 0 ? 1 : (int)std::min(3ll, npen);
-    for (int tp = tp0; tp <= nt / (2 * halo + 1) && (tp <= npen || tp == tp0); tp++) {
-        const int k = (span + nt / tp - 2 * halo - 1) / (nt / tp - 2 * halo);
-        const int out = (span + k - 1) / k;
-        const long long wgs = (long long)((span + out - 1) / out) * ((npen + tp - 1) / tp);
-        if (best < 0 || wgs < best || (wgs == best && d > 0 && tp_out < 4)) {
-            best = wgs;
-            tp_out = tp;
-            ts_out = out + 2 * halo;
-        }
-    }
-    return best;
+    return pk::even_tile(fused ? b->n[d] : b->ng[d], (long long)b->n[d1] * b->n[d2], fused ? 8 : 4, d == 0, nt, tp, ts);
 }
-
-// Default tile: 256 lanes (MHD 64^3, z: 256 lanes 47 us, 512 lanes 56; the
-// register budget of the kernels holds two or three 4-wave workgroups per CU,
-// which hide each other's barriers, but one 8-wave workgroup), fewer where
-// that leaves some of the 256 CUs without a workgroup (HD 32^3: 4x40 in 256
-// workgroups 12.4 us, 6x40 in 171 13.3; HD 16^3: 2x24 in 128 11.3 us, 10x24 in
-// 26 12.3 - 13.5).  Against a fixed 3 x 72, which leaves the last chunk of
-// most lengths nearly empty: MHD 131x98x77 206, 179, 212 us along x, y, z there,
-// 147, 140, 125 here; HD 96^3 82, 77, 82 there, 65, 62, 65 here.
 void default_tile(const Block *b, int d, bool fused, int &tp, int &ts)
 {
-    for (int nt = 256; nt >= 64; nt -= 64)
-        if (even_tile(b, d, fused, nt, tp, ts) >= 256) return;
+    const int d1 = (d == 0) ? 1 : 0, d2 = (d == 2) ? 1 : 2;
+    pk::full_tile(fused ? b->n[d] : b->ng[d], (long long)b->n[d1] * b->n[d2], fused ? 8 : 4, d == 0, tp, ts);
 }
 
 // Precedence: the shape given in pk_config, then the one pk_autotune
@@ -2088,11 +2056,15 @@ int ens_adj_build()
 // then update_boundaries of the stage's arrays, unsplit_sweeps.F90:126-190):
 // the first stage reads u and writes uh (the other buffer), the last reads
 // uh and adds its fluxes to u in place.
-// psi_fac: with the fused passes, psi of the stage's result is multiplied by
-// it in the last pass (*fac_applied set); the in-place Euler stage leaves it.
-int unsplit_stage(Block *b, int istep, double dt, double ch, double psi_fac = 1.0, bool *fac_applied = nullptr)
+// u_fac: psi of u (the step's initial state) counts as multiplied by it, and
+// psi_fac: psi of the stage's result is; want_dt: the stage also reduces the
+// timestep of its result; wrap: the input's ghosts are read from their
+// pre-images.  All with the fused passes only (RK2), which leave the ghosts of
+// the result old: the in-place Euler stage takes 1, 1 and false, reads the
+// ghosts and refreshes them.
+int unsplit_stage(Block *b, int istep, double dt, double ch, bool wrap, double u_fac = 1.0,
+                  double psi_fac = 1.0, bool want_dt = false)
 {
-    if (fac_applied) *fac_applied = false;
     RCCHK(no_fc(b, "the unsplit solver"));
     if (g_nfl != 1) return fail(PK_EINVAL, "the unsplit solver covers one fluid");
     if (block_linked(b)) return fail(PK_EINVAL, "the unsplit solver covers blocks periodic on themselves");
@@ -2137,7 +2109,12 @@ int unsplit_stage(Block *b, int istep, double dt, double ch, double psi_fac = 1.
     a.dt = dt;
     a.rk = rk_coef(istep);
     a.last = last ? 1 : 0;
+    a.src_fac = first ? u_fac : 1.0;
+    a.base_fac = u_fac;
+    a.wrap = wrap ? 1 : 0;
     a.psi_fac = 1.0;
+    a.dtslots = want_dt ? b->d_dtslots : nullptr;
+    a.nslots = kDtSlots;
     a.smalld = g_cfg.smalld;
     a.smallei = g_cfg.smallei;
     a.use_smalld = g_cfg.use_smalld;
@@ -2175,10 +2152,16 @@ int unsplit_stage(Block *b, int istep, double dt, double ch, double psi_fac = 1.
         HIPCHK(g_cfg.fast_math ? pk_fast::launch_unsplit_update(g_mhd, a, F, g_stream)
                                : pk::launch_unsplit_update(g_mhd, a, F, g_stream));
     }
-    if (src == dst) RCCHK(fill_buffer(b, dst));  // the fused passes wrote the periodic images already
-    else if (fac_applied) *fac_applied = true;
+    if (src == dst)
+        RCCHK(fill_buffer(b, dst));
+    else if (last)
+        b->ghosts_stale = true;
     b->uh = euler ? -1 : (first ? dst : b->uh);
     b->dt_pending = false;
+    if (want_dt && src != dst) {
+        HIPCHK(pk::launch_dtslots_final(b->d_dtslots, kDtSlots, 1, b->dtout, g_stream));
+        b->dt_pending = true;
+    }
     return PK_OK;
 }
 
@@ -2190,8 +2173,10 @@ int damp_psi(Block *b, double fac)
 }
 
 // fluid_update_unsplit (unsplit_fluidupdate.F90:45-126) on one periodic block:
-// update_chspeed, glmdamping(half), the stages, glmdamping(half)
-int fluid_update_unsplit(Block *b, double dt)
+// update_chspeed, glmdamping(half), the stages, glmdamping(half).  wrap: the
+// block's ghosts are its periodic images (the first stage need not read them).
+// The RK2 stages leave them old (b->ghosts_stale).
+int fluid_update_unsplit(Block *b, double dt, bool wrap)
 {
     double ch = 0.0, fac = 1.0;
     if (g_mhd) {
@@ -2202,17 +2187,16 @@ int fluid_update_unsplit(Block *b, double dt)
         const double r = (g_cfg.glm_alpha * ch) / (mdl / (dt / 2.0));
         if (r > f) f = r;
         fac = exp(-f);
-        RCCHK(damp_psi(b, fac));
     }
     if (g_cfg.integration_order == 1) {
-        RCCHK(unsplit_stage(b, PK_EULER, dt, ch));
-    } else {
-        RCCHK(unsplit_stage(b, PK_RK2_1, dt, ch));
+        if (g_mhd) RCCHK(damp_psi(b, fac));
+        RCCHK(unsplit_stage(b, PK_EULER, dt, ch, false));
+        if (g_mhd) RCCHK(damp_psi(b, fac));
+        return PK_OK;
     }
-    bool damped = false;  // the last fused pass applies glmdamping's second half itself
-    if (g_cfg.integration_order != 1) RCCHK(unsplit_stage(b, PK_RK2_2, dt, ch, g_mhd ? fac : 1.0, &damped));
-    if (g_mhd && !damped) RCCHK(damp_psi(b, fac));
-    return PK_OK;
+    // both halves of glmdamping are factors on psi as the fused passes read and write it
+    RCCHK(unsplit_stage(b, PK_RK2_1, dt, ch, wrap, fac, 1.0, false));
+    return unsplit_stage(b, PK_RK2_2, dt, ch, true, fac, fac, true);
 }
 
 // ---- step retries (cflcontrol = 'redo' / 'flexible') ----
@@ -2972,7 +2956,11 @@ int pk_unsplit_stage(int64_t cg_id, int32_t istep, double dt, double chspeed)
     Block *b;
     RCCHK(get_block(cg_id, &b));
     list_touch();
-    return unsplit_stage(b, istep, dt, chspeed);
+    RCCHK(unsplit_stage(b, istep, dt, chspeed, false));
+    // the stage's ghost refresh (the in-place stage has done it)
+    if (g_cfg.integration_order != 1) RCCHK(fill_buffer(b, istep == PK_RK2_1 ? b->uh : b->cur));
+    b->ghosts_stale = false;
+    return PK_OK;
 }
 
 int pk_fluid_update_unsplit(int64_t cg_id, double dt)
@@ -2982,7 +2970,9 @@ int pk_fluid_update_unsplit(int64_t cg_id, double dt)
     if (!(dt > 0.0)) return fail(PK_EINVAL, "dt must be positive");
     RCCHK(solo(b));
     list_touch();
-    return fluid_update_unsplit(b, dt);
+    RCCHK(fluid_update_unsplit(b, dt, false));
+    if (b->ghosts_stale) RCCHK(do_fill(b));
+    return PK_OK;
 }
 
 int pk_run_unsplit(int64_t cg_id, double tend, int32_t nmax, double *t_out, int32_t *nsteps_out)
@@ -3006,11 +2996,12 @@ int pk_run_unsplit(int64_t cg_id, double tend, int32_t nmax, double *t_out, int3
         const double rem = tend - t;
         const double cl = rem + (2.0 * DBL_EPSILON) * rem;
         if (cl < dt) dt = cl;
-        RCCHK(fluid_update_unsplit(b, dt));
+        RCCHK(fluid_update_unsplit(b, dt, true));
         t = t + dt;
         dt_old = dt;
         s++;
     }
+    if (b->ghosts_stale) RCCHK(do_fill(b));
     HIPCHK(hipStreamSynchronize(g_stream));
     if (t_out) *t_out = t;
     if (nsteps_out) *nsteps_out = s;

@@ -109,7 +109,7 @@ constexpr unsigned kListPiece = 1u << 22;
 // belongs to block items[item] and is that block's tile (or range of its
 // stream) item - first[block].  The hardware hands the workgroups out: with
 // resident workgroups taking items from a queue, or each walking a fixed range
-// of them, a sweep of 6 MHD blocks of 81x64x45 (12 launches of them in a step) is
+// of them, a sweep of 12 linked MHD blocks (120x96x80 cells in all) is
 // limited by the latency of a workgroup's successive tiles and by the block
 // arguments a loop keeps in scalar registers (40 spilled); a step took 935 us
 // with queues, 821 with ranges, 727 an item a workgroup (48 blocks of two
@@ -163,6 +163,46 @@ struct PlanesArgs {
     int nx, ny, nz;  // ghosted extents
     int sy, sz;
 };
+
+// The tile of at most nt lanes that needs the fewest workgroups for npen pencils
+// of span cells, where a tile of ts cells finishes ts - lost of them: over the
+// pencil counts tp, the pencil in equal chunks of the longest tile that fits.  Returns the workgroups.  Along x ties go to the longer tile (fewer
+// halo cells read).  Along y and z the lanes of a tile read tp cells in a row,
+// so at least 3 pencils are taken and ties go to the longest tile of 4 or more
+// (HD 224^3, y, 256 lanes: 4x64 575 us, 2x120 586, 1x232 > 640; HD 96^3, y:
+// 4x56 62 us, 2x104 65; MHD 131x98x77, y: 4x57 140 us, 2x106 147).
+inline long long even_tile(int span, long long npen, int lost, bool along_x, int nt, int &tp_out, int &ts_out)
+{
+    long long best = -1;
+    tp_out = 1;
+    ts_out = lost + 1;
+    const int tp0 = along_x || npen < 3 ? 1 : 3;
+    for (int tp = tp0; tp <= nt / (lost + 1) && (tp <= npen || tp == tp0); tp++) {
+        const int k = (span + nt / tp - lost - 1) / (nt / tp - lost);
+        const int out = (span + k - 1) / k;
+        const long long wgs = (long long)((span + out - 1) / out) * ((npen + tp - 1) / tp);
+        if (best < 0 || wgs < best || (wgs == best && !along_x && tp_out < 4)) {
+            best = wgs;
+            tp_out = tp;
+            ts_out = out + lost;
+        }
+    }
+    return best;
+}
+
+// Default tile: 256 lanes (MHD 64^3, z: 256 lanes 47 us, 512 lanes 56; the
+// register budget of the kernels holds two or three 4-wave workgroups per CU,
+// which hide each other's barriers, but one 8-wave workgroup), fewer where
+// that leaves some of the 256 CUs without a workgroup (HD 32^3: 4x40 in 256
+// workgroups 12.4 us, 6x40 in 171 13.3; HD 16^3: 2x24 in 128 11.3 us, 10x24 in
+// 26 12.3 - 13.5).  Against a fixed 3 x 72, which leaves the last chunk of
+// most lengths nearly empty: MHD 131x98x77 206, 179, 212 us along x, y, z there,
+// 147, 140, 125 here; HD 96^3 82, 77, 82 there, 65, 62, 65 here.
+inline void full_tile(int span, long long npen, int lost, bool along_x, int &tp, int &ts)
+{
+    for (int nt = 256; nt >= 64; nt -= 64)
+        if (even_tile(span, npen, lost, along_x, nt, tp, ts) >= 256) return;
+}
 
 hipError_t launch_sweep(int dir, bool mhd, bool fused, const SweepArgs &a, hipStream_t st);
 // Workgroup size that selects the stream form of the list sweep

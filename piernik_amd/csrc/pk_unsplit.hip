@@ -29,11 +29,14 @@
 #include <hip/hip_runtime.h>
 #include "pk_math.hpp"
 #include "pk_mass.hpp"
+#include "pk_kernels.hpp"
 #include "pk_unsplit.hpp"
 
 namespace PK_KNS {
 
 using pk::UnsplitArgs;
+
+#include "pk_tile.hpp"
 
 namespace {
 
@@ -64,19 +67,16 @@ __global__ __launch_bounds__(256) void k_unsplit_flux_tile(const UnsplitArgs a, 
     double *B = lds + NV * blockDim.x; // left face states
     const int nt = blockDim.x;
     const int t = threadIdx.x;
-    // XCD-aware order: each XCD gets a contiguous range of tiles
-    int bid = blockIdx.x;
-    const int nfull = (int)(gridDim.x / 8u) * 8;
-    if (bid < nfull) bid = (bid % 8) * (nfull / 8) + bid / 8;
+    const int bid = (int)pk::xcd_order();
     int p, sl, tm, tp;
     if (DIR == 0) {
-        sl = t % TS;
-        p = t / TS;
+        p = small_div(t, TS);
+        sl = t - p * TS;
         tm = t - 1;
         tp = t + 1;
     } else {
-        p = t % TP;
-        sl = t / TP;
+        sl = small_div(t, TP);
+        p = t - sl * TP;
         tm = t - TP;
         tp = t + TP;
     }
@@ -96,32 +96,44 @@ __global__ __launch_bounds__(256) void k_unsplit_flux_tile(const UnsplitArgs a, 
     const int csc = cs < 0 ? 0 : (cs >= ng ? ng - 1 : cs);
     int xyz[3];
     xyz[DIR] = csc;
-    xyz[d1] = a.g[d1] + pfc % n1;
-    xyz[d2] = a.g[d2] + pfc / n1;
+    const int e0 = (ptile * TP) / n1;  // the tile's first pencil: uniform, the lanes step on from it
+    int e1 = ptile * TP - e0 * n1 + (pfc - ptile * TP), e2 = e0;
+    if (n1 >= TP) {
+        if (e1 >= n1) e1 -= n1, e2++;
+    } else {
+        e2 += e1 / n1;
+        e1 = e1 % n1;
+    }
+    xyz[d1] = a.g[d1] + e1;
+    xyz[d2] = a.g[d2] + e2;
     const long long idx = (long long)xyz[0] + (long long)a.sy * xyz[1] + (long long)a.sz * xyz[2];
 
     double W[NV], q[NV];
 #pragma unroll
     for (int k = 0; k < NV; k++) W[k] = a.src[(long long)uplane(DIR, k) * a.sv + idx];
     prim<P>(W, a.gam_1, q);
-#pragma unroll
-    for (int v = 0; v < NV; v++) A[v * nt + t] = q[v];
+    lds_put<NV>(A, t, q);
     __syncthreads();
     double fp[NV];
+    {
+        double qm[NV], qp[NV], fm[NV];
+        lds_get<NV>(A, tm, qm);
+        lds_get<NV>(A, tp, qp);
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-        const int lim = (LIM >= 0) ? LIM : ((v < 5) ? a.lim : a.limb);
-        const double h = 0.5 * limit(lim, q[v] - A[v * nt + tm], A[v * nt + tp] - q[v]);
-        fp[v] = q[v] + h;          // right face of this cell
-        B[v * nt + t] = q[v] - h;  // left face of this cell
+        for (int v = 0; v < NV; v++) {
+            const int lim = (LIM >= 0) ? LIM : ((v < 5) ? a.lim : a.limb);
+            const double h = 0.5 * limit(lim, q[v] - qm[v], qp[v] - q[v]);
+            fp[v] = q[v] + h;  // right face of this cell
+            fm[v] = q[v] - h;  // left face of this cell
+        }
+        lds_put<NV>(B, t, fm);
     }
     __syncthreads();
     // the flux at cs+1/2, row cs+1, for interfaces g-1/2 .. g+n-1/2
     const bool own = pvalid && sl >= 1 && sl < 1 + out && cs >= a.g[DIR] - 1 && cs <= a.g[DIR] + a.n[DIR] - 1;
     if (!own) return;
     double fr[NV], f[NV];
-#pragma unroll
-    for (int v = 0; v < NV; v++) fr[v] = B[v * nt + tp];
+    lds_get<NV>(B, tp, fr);
     if constexpr (P::MAG)
         flux_hlld(fp, fr, a.gam, a.ch, f);
     else
@@ -139,13 +151,16 @@ __global__ __launch_bounds__(256) void k_unsplit_flux_tile(const UnsplitArgs a, 
 // flux from its neighbour through LDS, to the cell's running sum.  The sum
 // starts from base at the first active direction and waits in dst between
 // directions, each cell read and written by its own lane only; after the
-// last active direction the source passes run, dst holds the stage's
-// result and the pass also writes each cell's periodic ghost images (the
-// stage's ghost refresh).  The operands and their order are those of
+// last active direction the source passes run and dst holds the stage's
+// result (interior cells; its ghosts are left as they are, and read through
+// their pre-images: a.wrap).  The operands and their order are those of
 // k_unsplit_update, so the result is the same bit for bit, without the flux
 // arrays.
-// Three waves per SIMD: the relaxed build needs 172 VGPRs unconstrained (two
-// waves); held to 168 it spills 7 and runs 10 % faster.
+// Bound by memory where it adds to dst (read src and dst, write dst: 90 us at
+// the copy rate for 128^3 MHD), by FP64 issue and memory both along x.  Lane-
+// major LDS (pk_tile.hpp), chunks of equal length and no images: the passes of
+// a 128^3 MHD block along x, y, z took 134, 141, 157 us with 4 x 64 and 8 x 32
+// tiles, images and [variable][lane] LDS; 101, 116, 129 us now.
 template <int DIR, class P, int LIM>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k_unsplit_fused_tile(const UnsplitArgs a, int TP, int TS, int chunks,
                                                             int first, int last)
@@ -158,18 +173,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     double *B = lds + NV * blockDim.x;  // left face states
     const int nt = blockDim.x;
     const int t = threadIdx.x;
-    int bid = blockIdx.x;
-    const int nfull = (int)(gridDim.x / 8u) * 8;
-    if (bid < nfull) bid = (bid % 8) * (nfull / 8) + bid / 8;
+    const int bid = (int)pk::xcd_order();
     int p, sl, tm, tp;
     if (DIR == 0) {
-        sl = t % TS;
-        p = t / TS;
+        p = small_div(t, TS);
+        sl = t - p * TS;
         tm = t - 1;
         tp = t + 1;
     } else {
-        p = t % TP;
-        sl = t / TP;
+        sl = small_div(t, TP);
+        p = t - sl * TP;
         tm = t - TP;
         tp = t + TP;
     }
@@ -186,34 +199,48 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     const int c0 = a.g[DIR] + chunk * out;  // the tile's first updated cell
     const int cs = c0 - 2 + sl;             // this lane's cell
     const int ng = a.ng[DIR];
-    const int csc = cs < 0 ? 0 : (cs >= ng ? ng - 1 : cs);
+    int csc = cs < 0 ? 0 : (cs >= ng ? ng - 1 : cs);
+    if (a.wrap) csc = wrap_cell(csc, a.g[DIR], a.n[DIR]);
     int xyz[3];
     xyz[DIR] = csc;
-    xyz[d1] = a.g[d1] + pfc % n1;
-    xyz[d2] = a.g[d2] + pfc / n1;
+    const int e0 = (ptile * TP) / n1;  // the tile's first pencil: uniform, the lanes step on from it
+    int e1 = ptile * TP - e0 * n1 + (pfc - ptile * TP), e2 = e0;
+    if (n1 >= TP) {
+        if (e1 >= n1) e1 -= n1, e2++;
+    } else {
+        e2 += e1 / n1;
+        e1 = e1 % n1;
+    }
+    xyz[d1] = a.g[d1] + e1;
+    xyz[d2] = a.g[d2] + e2;
     const long long idx = (long long)xyz[0] + (long long)a.sy * xyz[1] + (long long)a.sz * xyz[2];
 
     double W[NV], q[NV];
 #pragma unroll
     for (int k = 0; k < NV; k++) W[k] = a.src[(long long)uplane(DIR, k) * a.sv + idx];
+    if constexpr (P::MAG) W[8] = W[8] * a.src_fac;
     prim<P>(W, a.gam_1, q);
-#pragma unroll
-    for (int v = 0; v < NV; v++) A[v * nt + t] = q[v];
+    lds_put<NV>(A, t, q);
     __syncthreads();
     double fp[NV];
+    {
+        double qm[NV], qp[NV], fm[NV];
+        lds_get<NV>(A, tm, qm);
+        lds_get<NV>(A, tp, qp);
 #pragma unroll
-    for (int v = 0; v < NV; v++) {
-        const int lim = (LIM >= 0) ? LIM : ((v < 5) ? a.lim : a.limb);
-        const double h = 0.5 * limit(lim, q[v] - A[v * nt + tm], A[v * nt + tp] - q[v]);
-        fp[v] = q[v] + h;
-        B[v * nt + t] = q[v] - h;
+        for (int v = 0; v < NV; v++) {
+            const int lim = (LIM >= 0) ? LIM : ((v < 5) ? a.lim : a.limb);
+            const double h = 0.5 * limit(lim, q[v] - qm[v], qp[v] - q[v]);
+            fp[v] = q[v] + h;
+            fm[v] = q[v] - h;
+        }
+        lds_put<NV>(B, t, fm);
     }
     __syncthreads();
     double f[NV];
     if (sl >= 1 && sl < TS - 2) {
         double fr[NV];
-#pragma unroll
-        for (int v = 0; v < NV; v++) fr[v] = B[v * nt + tp];
+        lds_get<NV>(B, tp, fr);
         if constexpr (P::MAG)
             flux_hlld(fp, fr, a.gam, a.ch, f);
         else
@@ -222,24 +249,30 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 #pragma unroll
         for (int v = 0; v < NV; v++) f[v] = 0.0;
     }
-    // every read of A (the primitives) came before the last barrier
-#pragma unroll
-    for (int v = 0; v < NV; v++) A[v * nt + t] = f[v];
-    __syncthreads();
     const bool upd = pvalid && sl >= 2 && sl < 2 + out && cs < a.g[DIR] + a.n[DIR];
     const long long ci = idx;  // an interior cell when upd: csc == cs
     double T[NV];
-    unsigned flags = 0u;
-    double dmass = 0.0;
     if (upd) {
         const double *S = first ? a.base : a.dst;
 #pragma unroll
         for (int v = 0; v < NV; v++) T[v] = S[(long long)v * a.sv + ci];
+    }
+    // every read of A (the primitives) came before the last barrier
+    lds_put<NV>(A, t, f);
+    __syncthreads();
+    unsigned flags = 0u;
+    double dmass = 0.0;
+    if (upd) {
+        if constexpr (P::MAG) {
+            if (first) T[8] = T[8] * a.base_fac;
+        }
         const double coef = (a.dt / a.dl[DIR]) * a.rk;
+        double fl[NV];
+        lds_get<NV>(A, tm, fl);
 #pragma unroll
         for (int k = 0; k < NV; k++) {
             const int v = uplane(DIR, k);
-            T[v] = T[v] + coef * (A[k * nt + tm] - f[k]);
+            T[v] = T[v] + coef * (fl[k] - f[k]);
         }
         if (last) {
             for (int d = 0; d < 3; d++) {
@@ -264,32 +297,15 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 #pragma unroll
         for (int v = 0; v < NV; v++) a.dst[(long long)v * a.sv + ci] = T[v];
     }
-    // last and a.last are the same for every lane: the whole wave takes part
+    // last, a.last and a.dtslots are the same for every lane: the whole wave takes part
     if (last && a.last) pk::mass_add(a.dmass, dmass);
-    if (!upd) return;
-    if (flags) atomicOr(a.flags, flags);
-    if (!last) return;
-    // periodic images of the finished cell (the stage's ghost refresh): every
-    // ghost has exactly one interior pre-image, since n >= nb
-    int off[3][3], cnt[3];
-#pragma unroll
-    for (int d = 0; d < 3; d++) {
-        const int ic = xyz[d] - a.g[d];
-        cnt[d] = 1;
-        off[d][0] = 0;
-        if (a.g[d] > 0) {
-            if (ic < a.g[d]) off[d][cnt[d]++] = a.n[d];
-            if (ic >= a.n[d] - a.g[d]) off[d][cnt[d]++] = -a.n[d];
-        }
+    if (last && a.dtslots) {  // timestep_fluid of the cells of the finished state
+        const double huge = 1.7976931348623157e308;
+        double mn[3] = {huge, huge, huge}, cmax = 0.0;
+        if (upd) dt_cell<0, P>(a, T, mn, cmax);
+        dt_reduce(a, mn, cmax, blockIdx.x);
     }
-    for (int i0 = 0; i0 < cnt[0]; i0++)
-        for (int i1 = 0; i1 < cnt[1]; i1++)
-            for (int i2 = 0; i2 < cnt[2]; i2++) {
-                if ((i0 | i1 | i2) == 0) continue;
-                const long long j = ci + off[0][i0] + (long long)a.sy * off[1][i1] + (long long)a.sz * off[2][i2];
-#pragma unroll
-                for (int v = 0; v < NV; v++) a.dst[(long long)v * a.sv + j] = T[v];
-            }
+    if (upd && flags) atomicOr(a.flags, flags);
 }
 
 template <class P>
@@ -344,22 +360,37 @@ __global__ __launch_bounds__(256) void k_unsplit_update(const UnsplitArgs a, con
     if (flags) atomicOr(a.flags, flags);
 }
 
-// Tile shapes of the flux kernel, pencils x cells: along x one wave per
-// pencil; along y and z 8 x-consecutive pencils (64 B rows) x 32 cells
-// (measured at 256^3 MHD against 4 x 64, 16 x 16 and 32 x 8).
-constexpr int kTile[3][2] = {{4, 64}, {8, 32}, {8, 32}};
+// Tile of the flux kernels for npen pencils of span rows, ts - lost finished per
+// tile.  Along x the fewest workgroups (full_tile); along y and z 8 x-consecutive
+// pencils, 64 bytes a row, in equal chunks of at most 32 cells: these passes
+// wait for memory, and other widths leave part of every line to another
+// workgroup (three steps of a 128^3 MHD block with 7 x 36 in y and z 2550 us,
+// with 8 x 30 in y 2454 - 2330, in both 2230; hydro 1034, 1008).
+template <int DIR>
+void unsplit_tile(int span, long long npen, int lost, int &TP, int &TS)
+{
+    if (DIR == 0) {
+        pk::full_tile(span, npen, lost, true, TP, TS);
+        return;
+    }
+    TP = 8;
+    const int k = (span + 32 - lost - 1) / (32 - lost);
+    TS = (span + k - 1) / k + lost;
+}
 
 template <int DIR, class P, int LIM>
 hipError_t fused_tile(const UnsplitArgs &a, int first, int last, hipStream_t st)
 {
     const int d1 = (DIR == 0) ? 1 : 0, d2 = (DIR == 2) ? 1 : 2;
     const long long npen = (long long)a.n[d1] * a.n[d2];
-    const int TP = kTile[DIR][0], TS = kTile[DIR][1];
+    int TP, TS;
+    unsplit_tile<DIR>(a.n[DIR], npen, 4, TP, TS);
     const int chunks = (a.n[DIR] + (TS - 4) - 1) / (TS - 4);
+    const int nt = (TP * TS + 63) / 64 * 64;
     const long long tiles = (npen + TP - 1) / TP * chunks;
     if (tiles < 1 || tiles > 0x7fffffffll) return hipErrorInvalidValue;
-    const size_t shm = sizeof(double) * 2 * P::NV * TP * TS;
-    hipLaunchKernelGGL((k_unsplit_fused_tile<DIR, P, LIM>), dim3((unsigned)tiles), dim3(TP * TS), shm, st, a, TP,
+    const size_t shm = sizeof(double) * 2 * P::NV * nt;
+    hipLaunchKernelGGL((k_unsplit_fused_tile<DIR, P, LIM>), dim3((unsigned)tiles), dim3(nt), shm, st, a, TP,
                        TS, chunks, first, last);
     return hipGetLastError();
 }
@@ -384,12 +415,14 @@ hipError_t flux_tile(const UnsplitArgs &a, double *F, hipStream_t st)
 {
     const int d1 = (DIR == 0) ? 1 : 0, d2 = (DIR == 2) ? 1 : 2;
     const long long npen = (long long)a.n[d1] * a.n[d2];
-    const int TP = kTile[DIR][0], TS = kTile[DIR][1];
+    int TP, TS;
+    unsplit_tile<DIR>(a.n[DIR] + 1, npen, 3, TP, TS);
     const int chunks = (a.n[DIR] + 1 + (TS - 3) - 1) / (TS - 3);
+    const int nt = (TP * TS + 63) / 64 * 64;
     const long long tiles = (npen + TP - 1) / TP * chunks;
     if (tiles < 1 || tiles > 0x7fffffffll) return hipErrorInvalidValue;
-    const size_t shm = sizeof(double) * 2 * P::NV * TP * TS;
-    hipLaunchKernelGGL((k_unsplit_flux_tile<DIR, P, LIM>), dim3((unsigned)tiles), dim3(TP * TS), shm, st, a, F, TP,
+    const size_t shm = sizeof(double) * 2 * P::NV * nt;
+    hipLaunchKernelGGL((k_unsplit_flux_tile<DIR, P, LIM>), dim3((unsigned)tiles), dim3(nt), shm, st, a, F, TP,
                        TS, chunks);
     return hipGetLastError();
 }

@@ -18,6 +18,11 @@ struct UnsplitArgs {
     double gam, gam_1;
     double ch;           // GLM cleaning speed
     double dt, rk;       // dt and rk_coef of the stage
+    // fused passes only:
+    int wrap;            // 1: src's ghosts are read from their pre-images (a block periodic on itself)
+    double src_fac, base_fac;  // psi of src and of base times these when read (glmdamping before the stages)
+    unsigned long long *dtslots;  // if set: the last direction's pass folds timestep_fluid of the finished
+    int nslots;                   // state into these slots (as SweepArgs)
     double psi_fac;      // fused passes: psi of the finished state times this (glmdamping after the stages)
     int last;            // last stage: care_for_positives runs
     double smalld, smallei;
@@ -36,9 +41,8 @@ hipError_t launch_unsplit_flux(int dir, bool mhd, const UnsplitArgs &a, double *
 hipError_t launch_unsplit_update(bool mhd, const UnsplitArgs &a, const double *const F[3], hipStream_t st);
 // Flux along dir and its difference added in one pass (src != dst): the
 // running sum starts from base when `first`, is kept in dst between
-// directions, and gets the source passes and the periodic ghost images when
-// `last` (first and last active direction of the stage).  Same result as the
-// two launchers above followed by the ghost refresh.
+// directions, and gets the source passes when `last` (first and last active
+// direction of the stage).  Same interior as the two launchers above.
 hipError_t launch_unsplit_fused(int dir, bool mhd, const UnsplitArgs &a, int first, int last, hipStream_t st);
 
 }  // namespace pk

@@ -1,0 +1,79 @@
+"""Unsplit tiles at their edges: pencils shorter than the halo needs, lengths
+either side of a chunk (28 cells along y and z), pencils that leave the last
+tile partly empty, ghosts read from their pre-images, and the timestep and psi
+factors folded into the passes.  Bit for bit against the oracle, through
+whole runs and through single steps from ghosts that are not periodic images
+(a step reads the ghosts it is given)."""
+import numpy as np
+import pytest
+
+import piernik_amd as pk
+from piernik_amd import setups
+
+pytestmark = pytest.mark.gpu
+
+CASES = [((4, 4, 4), (True, True, True)), ((5, 29, 7), (True, True, True)), ((61, 6, 28), (True, True, True)),
+         ((9, 57, 1), (True, True, False)), ((253, 1, 1), (True, False, False))]
+
+
+def assert_same(cg, ob, where):
+    for name in ("u", "b", "psi"):
+        a, o = getattr(cg, name), getattr(ob, name)
+        if a is None:
+            continue
+        bad = np.argwhere(~(a == o))
+        assert bad.size == 0, f"{where} {name}: {len(bad)} differ, first at {tuple(bad[0])}"
+
+
+@pytest.mark.parametrize("mag", [False, True])
+@pytest.mark.parametrize("n,has_dir", CASES)
+def test_run_bit_exact(oracle, n, has_dir, mag):
+    cfg = pk.Config(magnetized=mag, limiter="vanleer", cfl=0.3, smalld=1e-10, smallei=1e-10, has_dir=has_dir)
+    cg = setups.smooth_random(n, seed=sum(n), magnetized=mag, has_dir=has_dir)
+    if mag:
+        cg.psi[...] = np.random.default_rng(4).normal(0, 0.01, cg.psi.shape)
+    setups.fill_ghosts_periodic(cg)
+    print(f"unsplit {n} magnetized {mag}", flush=True)
+    pk.load_library()
+    pk.finalize()
+    pk.init(cfg)
+    ob = oracle.OBlock.from_cg(cg)
+    p = oracle.params_from_config(cfg)
+    cg.upload()
+    t_g, n_g = pk.run_unsplit(cg, 1.0, nmax=3)
+    t_o, n_o = oracle.run_unsplit(p, ob, 1.0, nmax=3)
+    cg.download()
+    assert (t_g, n_g) == (t_o, n_o)
+    assert_same(cg, ob, f"{n}")
+    # the timestep the last pass reduced is that of the state it left
+    pending = pk.timestep_fluid(cg)
+    cg.upload()
+    assert pk.timestep_fluid(cg) == pending
+    pk.finalize()
+
+
+def test_step_reads_the_ghosts_it_is_given(oracle):
+    """One step from ghosts that are not the periodic images of the interior:
+    the first stage reads them as they are (the oracle's driver refreshes
+    them, so the step is compared with itself on a block whose ghosts were
+    refreshed, and must differ)."""
+    cfg = pk.Config(magnetized=True, limiter="vanleer", smalld=1e-10, smallei=1e-10)
+    out = []
+    for scale in (1.0, 1.5):
+        cg = setups.smooth_random((12, 9, 8), seed=3, magnetized=True)
+        setups.fill_ghosts_periodic(cg)
+        cg.u[0, :4] *= scale
+        pk.load_library()
+        pk.finalize()
+        pk.init(cfg)
+        cg.upload()
+        pk.fluid_update_unsplit(cg, 1e-3)
+        cg.download()
+        out.append(cg.u.copy())
+        # the step leaves refreshed ghosts
+        ref = cg.u.copy(order="F")
+        setups.fill_ghosts_periodic(cg)
+        assert np.array_equal(ref, cg.u)
+        pk.finalize()
+    inner = (0, slice(4, -4), slice(4, -4), slice(4, -4))
+    assert not np.array_equal(out[0][inner], out[1][inner])
