@@ -221,91 +221,85 @@ __global__ __launch_bounds__(256) void k_dtslots_final(unsigned long long *__res
 
 // ---- ghosts ------------------------------------------------------------------------
 
-// Copies of the planes of one cell, kPl at a time so that the loads of a
-// group are in flight together.
-constexpr int kPl = 5;
-__device__ __forceinline__ void copy_planes(const double *s, long long ssv, double *d, long long dsv, int np)
+// The planes of one cell in as few groups of loads as they fit (a block has 5
+// or 9 planes with one fluid, 10 or 14 with two).
+__device__ __forceinline__ void copy_cell(const double *s, long long ssv, double *d, long long dsv, int np)
 {
-    for (int v0 = 0; v0 < np; v0 += kPl) {
-        double x[kPl];
-#pragma unroll
-        for (int v = 0; v < kPl; v++) x[v] = s[(long long)min(v0 + v, np - 1) * ssv];
-#pragma unroll
-        for (int v = 0; v < kPl; v++)
-            if (v0 + v < np) d[(long long)(v0 + v) * dsv] = x[v];
-    }
+    if (np == 9)
+        copy_planes<9>(s, ssv, d, dsv, np);
+    else if (np == 14)
+        copy_planes<14>(s, ssv, d, dsv, np);
+    else
+        copy_planes<5>(s, ssv, d, dsv, np);
 }
 
 // Ghost exchange between blocks (internal_boundaries_local,
 // cg_list_bnd.F90:269-322): one job per face, cut into chunks of kFaceCells
 // cells, one workgroup per chunk (wgjob names its job); cells run x fastest,
 // so rows of y and z faces are coalesced, and a lane finds its cell once for
-// all planes (one value at a time the index divisions were 90 % of the
-// instructions: 1484 per wave for 16 values, 20 us per exchange of twelve
-// 40x40x40-like MHD blocks).
+// all planes.  The time is latency, so a lane has one cell and its planes'
+// loads are in flight together: an exchange of twelve 40x48x40 MHD blocks took
+// 20 us a value at a time (1484 instructions per wave, 90 % of them index
+// divisions), 17 with two cells a lane in groups of five planes, 14.6 so.
 __global__ __launch_bounds__(256) void k_exchange_faces(const FaceJob *__restrict__ jobs, const int *__restrict__ wgjob)
 {
     const FaceJob &J = jobs[wgjob[blockIdx.x]];
     const int e0 = J.ext[0], e01 = e0 * J.ext[1], ncell = e01 * J.ext[2];
-    const int base = ((int)blockIdx.x - J.wg0) * kFaceCells;
-    const int end = min(base + kFaceCells, ncell);
-    for (int c = base + (int)threadIdx.x; c < end; c += 256) {
-        const int k = c / e01, r = c - k * e01;
-        const int j = r / e0, i = r - j * e0;
-        const double *s = J.src + (J.sorg[0] + i) + (long long)J.ssy * (J.sorg[1] + j) + (long long)J.ssz * (J.sorg[2] + k);
-        double *d = J.dst + (J.dorg[0] + i) + (long long)J.dsy * (J.dorg[1] + j) + (long long)J.dsz * (J.dorg[2] + k);
-        copy_planes(s, J.ssv, d, J.dsv, J.nplanes);
-    }
+    const int c = ((int)blockIdx.x - J.wg0) * kFaceCells + (int)threadIdx.x;
+    if (c >= ncell) return;
+    const int k = c / e01, r = c - k * e01;
+    const int j = r / e0, i = r - j * e0;
+    const double *s = J.src + (J.sorg[0] + i) + (long long)J.ssy * (J.sorg[1] + j) + (long long)J.ssz * (J.sorg[2] + k);
+    double *d = J.dst + (J.dorg[0] + i) + (long long)J.dsy * (J.dorg[1] + j) + (long long)J.dsz * (J.dorg[2] + k);
+    copy_cell(s, J.ssv, d, J.dsv, J.nplanes);
 }
+static_assert(kFaceCells == 256, "k_exchange_faces: a cell per lane");
 
 // Periodic refresh of every ghost cell of a block in one launch: each ghost
 // is a copy of the interior cell its coordinates wrap to, which is what
-// refreshes along x, y and z in turn leave (n >= g).  The ghosts are
-// numbered z slabs (whole planes), then y slabs (interior z), then x slabs.
+// refreshes along x, y and z in turn leave (n >= g).
 __global__ __launch_bounds__(256) void k_fill_periodic(const GhostArgs a)
 {
-    const unsigned nx = (unsigned)a.ng[0], ny = (unsigned)a.ng[1];
-    const unsigned ix = (unsigned)a.n[0], iy = (unsigned)a.n[1], iz = (unsigned)a.n[2];
-    const unsigned gx = (unsigned)a.g[0], gy = (unsigned)a.g[1], gz = (unsigned)a.g[2];
-    const unsigned rz = 2u * gz * nx * ny, ry = 2u * gy * iz * nx, rx = 2u * gx * iz * iy;  // < 2^32 (launcher)
-    unsigned t = blockIdx.x * 256u + threadIdx.x;
-    unsigned x, y, z;
-    if (t < rz) {
-        const unsigned pl = nx * ny, l = t / pl, r = t - l * pl;
-        z = l < gz ? l : iz + l;
-        y = r / nx;
-        x = r - y * nx;
-    } else if (t < rz + ry) {
-        t -= rz;
-        const unsigned pl = 2u * gy * nx, l = t / pl, r = t - l * pl;
-        z = gz + l;
-        const unsigned q = r / nx;
-        y = q < gy ? q : iy + q;
-        x = r - q * nx;
-    } else if (t < rz + ry + rx) {
-        t -= rz + ry;
-        const unsigned pl = 2u * gx * iy, l = t / pl, r = t - l * pl;
-        z = gz + l;
-        const unsigned q = r / (2u * gx), e = r - q * 2u * gx;
-        y = gy + q;
-        x = e < gx ? e : ix + e;
-    } else {
-        return;
-    }
-    const unsigned sx = x < gx ? x + ix : (x >= gx + ix ? x - ix : x);
-    const unsigned sy = y < gy ? y + iy : (y >= gy + iy ? y - iy : y);
-    const unsigned sz = z < gz ? z + iz : (z >= gz + iz ? z - iz : z);
+    const unsigned n[3] = {(unsigned)a.n[0], (unsigned)a.n[1], (unsigned)a.n[2]};
+    const unsigned g[3] = {(unsigned)a.g[0], (unsigned)a.g[1], (unsigned)a.g[2]};
+    unsigned c[3], f[3];
+    if (!ghost_cell(blockIdx.x * 256u + threadIdx.x, n, g, c)) return;
+#pragma unroll
+    for (int d = 0; d < 3; d++) f[d] = c[d] < g[d] ? c[d] + n[d] : (c[d] >= g[d] + n[d] ? c[d] - n[d] : c[d]);
     double *base = a.u + (long long)a.plane0 * a.sv;
-    copy_planes(base + sx + (long long)a.sy * sy + (long long)a.sz * sz, a.sv,
-                base + x + (long long)a.sy * y + (long long)a.sz * z, a.sv, a.nplanes);
+    copy_cell(base + f[0] + (long long)a.sy * f[1] + (long long)a.sz * f[2], a.sv,
+              base + c[0] + (long long)a.sy * c[1] + (long long)a.sz * c[2], a.sv, a.nplanes);
 }
 
 // ---- layout conversion ---------------------------------------------------------------
 // Arrays of the reference layout (variable fastest; up to three of them, for
 // u, B and psi) <-> device planes, a cell per lane and every array in one
 // launch: grid (cells of a z plane / 256, nz).  Bound by memory: 5.6 TB/s of
-// 16 B per value at 256^3 (the strided accesses of a wave share cache lines);
-// small blocks pay for the launch only.
+// 16 B per value at 256^3 (the strided accesses of a wave share cache lines).
+// On small blocks the time is the latency of one lane's accesses, so the
+// values of a cell are read in groups of up to kPl before they are written:
+// one after another, 14 values of a cell of two fluids took 22 us to the planes'
+// arrays and 14 us back on blocks of 85000 cells (a launch is 3 us).
+
+// One array of a cell.
+constexpr int kPl = 5;
+template <bool IN>
+__device__ __forceinline__ void planes_array(const PlaneMap &m, double *q, double *s, long long sv)
+{
+    for (int c0 = 0; c0 < m.nc; c0 += kPl) {
+        double x[kPl];
+#pragma unroll
+        for (int c = 0; c < kPl; c++) {
+            const int cc = min(c0 + c, m.nc - 1);
+            x[c] = IN ? q[cc] : s[(long long)m.planes[cc] * sv];
+        }
+#pragma unroll
+        for (int c = 0; c < kPl; c++) {
+            if (c0 + c >= m.nc) break;
+            (IN ? s[(long long)m.planes[c0 + c] * sv] : q[c0 + c]) = x[c];
+        }
+    }
+}
 
 template <bool IN>
 __global__ __launch_bounds__(256) void k_planes(const PlanesArgs a)
@@ -317,32 +311,31 @@ __global__ __launch_bounds__(256) void k_planes(const PlanesArgs a)
     for (unsigned z = blockIdx.y; z < nz; z += gridDim.y) {
         const long long i = (long long)e + (long long)z * nx * ny;
         double *s = a.soa + x + (long long)a.sy * y + (long long)a.sz * z;
+        // u of one fluid with B and psi: all nine values in flight
+        if (a.aos[0] && a.aos[1] && a.aos[2] && a.map[0].nc == 5 && a.map[1].nc == 3 && a.map[2].nc == 1) {
+            double *q[9], *p[9], v[9];
 #pragma unroll
-        for (int k = 0; k < 3; k++) {
-            if (!a.aos[k]) continue;
-            const int nc = a.map[k].nc;
-            double *q = a.aos[k] + i * nc;
-            if (nc == 5) {
-                double v[5];
-#pragma unroll
-                for (int c = 0; c < 5; c++) v[c] = IN ? q[c] : s[(long long)a.map[k].planes[c] * a.sv];
-#pragma unroll
-                for (int c = 0; c < 5; c++) (IN ? s[(long long)a.map[k].planes[c] * a.sv] : q[c]) = v[c];
-            } else {
-                for (int c = 0; c < nc; c++) {
-                    if (IN)
-                        s[(long long)a.map[k].planes[c] * a.sv] = q[c];
-                    else
-                        q[c] = s[(long long)a.map[k].planes[c] * a.sv];
-                }
+            for (int c = 0; c < 9; c++) {
+                const int k = c < 5 ? 0 : (c < 8 ? 1 : 2), cc = c < 5 ? c : (c < 8 ? c - 5 : 0);
+                q[c] = a.aos[k] + i * (k == 0 ? 5 : (k == 1 ? 3 : 1)) + cc;
+                p[c] = s + (long long)a.map[k].planes[cc] * a.sv;
             }
+#pragma unroll
+            for (int c = 0; c < 9; c++) v[c] = IN ? *q[c] : *p[c];
+#pragma unroll
+            for (int c = 0; c < 9; c++) (IN ? *p[c] : *q[c]) = v[c];
+            continue;
         }
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            if (a.aos[k]) planes_array<IN>(a.map[k], a.aos[k] + i * a.map[k].nc, s, a.sv);
     }
 }
 
 // The adjoint of the periodic ghost refresh while converting: an interior
 // cell's adjoint is its own plus those of the ghosts that copy it (folded
-// along z, then y, then x, low ghost before high), a ghost's is 0.
+// along z, then y, then x, low ghost before high), a ghost's is 0.  Values in
+// groups of kPl, as k_planes.
 __global__ __launch_bounds__(256) void k_planes_fold(const PlanesArgs a, int g0, int g1, int g2)
 {
     const int nx = a.nx, ny = a.ny;
@@ -351,15 +344,13 @@ __global__ __launch_bounds__(256) void k_planes_fold(const PlanesArgs a, int g0,
     const int y = (int)(e / (unsigned)nx), x = (int)(e - (unsigned)y * (unsigned)nx);
     for (int z = (int)blockIdx.y; z < a.nz; z += (int)gridDim.y) {
         const int g[3] = {g0, g1, g2}, ng[3] = {nx, ny, a.nz}, p[3] = {x, y, z};
-        int at[3][3], cnt[3];
+        int lo[3], hi[3];  // the low and the high ghost that copy the cell, or -1
         bool inner = true;
 #pragma unroll
         for (int d = 0; d < 3; d++) {
             const int n = ng[d] - 2 * g[d], i = p[d] - g[d];
-            at[d][0] = p[d];
-            at[d][1] = (g[d] > 0 && i >= n - g[d]) ? i - (n - g[d]) : -1;  // the low ghost that copies it
-            at[d][2] = (g[d] > 0 && i < g[d]) ? g[d] + n + i : -1;          // the high one
-            cnt[d] = (at[d][1] >= 0 || at[d][2] >= 0) ? 3 : 1;
+            lo[d] = (g[d] > 0 && i >= n - g[d]) ? i - (n - g[d]) : -1;
+            hi[d] = (g[d] > 0 && i < g[d]) ? g[d] + n + i : -1;
             inner = inner && i >= 0 && i < n;
         }
         double *s = a.soa + x + (long long)a.sy * y + (long long)a.sz * z;
@@ -367,26 +358,41 @@ __global__ __launch_bounds__(256) void k_planes_fold(const PlanesArgs a, int g0,
         for (int k = 0; k < 3; k++) {
             if (!a.aos[k]) continue;
             const int nc = a.map[k].nc;
-            for (int c = 0; c < nc; c++) {
-                double fx = 0.0;
+            for (int c0 = 0; c0 < nc; c0 += kPl) {
+                double fx[kPl];
+#pragma unroll
+                for (int c = 0; c < kPl; c++) fx[c] = 0.0;
                 if (inner) {
-                    for (int i0 = 0; i0 < cnt[0]; i0++) {
-                        if (at[0][i0] < 0) continue;
-                        double fy = 0.0;
-                        for (int i1 = 0; i1 < cnt[1]; i1++) {
-                            if (at[1][i1] < 0) continue;
-                            double fz = 0.0;
-                            for (int i2 = 0; i2 < cnt[2]; i2++) {
-                                if (at[2][i2] < 0) continue;
-                                const double v = a.aos[k][(at[0][i0] + (long long)nx * (at[1][i1] + (long long)ny * at[2][i2])) * nc + c];
-                                fz = i2 == 0 ? v : fz + v;
+                    for (int i0 = 0; i0 < 3; i0++) {
+                        const int cx = i0 == 0 ? x : (i0 == 1 ? lo[0] : hi[0]);
+                        if (cx < 0) continue;
+                        double fy[kPl];
+                        for (int i1 = 0; i1 < 3; i1++) {
+                            const int cy = i1 == 0 ? y : (i1 == 1 ? lo[1] : hi[1]);
+                            if (cy < 0) continue;
+                            double fz[kPl];
+                            for (int i2 = 0; i2 < 3; i2++) {
+                                const int cz = i2 == 0 ? z : (i2 == 1 ? lo[2] : hi[2]);
+                                if (cz < 0) continue;
+                                const double *q = a.aos[k] + (cx + (long long)nx * (cy + (long long)ny * cz)) * nc;
+                                double v[kPl];
+#pragma unroll
+                                for (int c = 0; c < kPl; c++) v[c] = q[min(c0 + c, nc - 1)];
+#pragma unroll
+                                for (int c = 0; c < kPl; c++) fz[c] = i2 == 0 ? v[c] : fz[c] + v[c];
                             }
-                            fy = i1 == 0 ? fz : fy + fz;
+#pragma unroll
+                            for (int c = 0; c < kPl; c++) fy[c] = i1 == 0 ? fz[c] : fy[c] + fz[c];
                         }
-                        fx = i0 == 0 ? fy : fx + fy;
+#pragma unroll
+                        for (int c = 0; c < kPl; c++) fx[c] = i0 == 0 ? fy[c] : fx[c] + fy[c];
                     }
                 }
-                s[(long long)a.map[k].planes[c] * a.sv] = fx;
+#pragma unroll
+                for (int c = 0; c < kPl; c++) {
+                    if (c0 + c >= nc) break;
+                    s[(long long)a.map[k].planes[c0 + c] * a.sv] = fx[c];
+                }
             }
         }
     }

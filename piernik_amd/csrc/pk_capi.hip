@@ -465,43 +465,6 @@ int launch_timed(int d, double bytes, const std::function<hipError_t()> &go)
     return PK_OK;
 }
 
-// Copy the cells outside the transverse interior (for sweep direction d)
-// from src to dst, so that a one-stage call leaves them as the reference
-// does (it only writes transverse-interior pencils).
-__global__ void k_copy_transverse_ghosts(const double *__restrict__ src, double *__restrict__ dst, long long sv,
-                                         int nplanes, int sy, int sz, int d, int nx, int ny, int nz, int gx, int gy,
-                                         int gz, int ix, int iy, int iz)
-{
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long ncell = (long long)nx * ny * nz;
-    if (i >= ncell) return;
-    const int x = (int)(i % nx);
-    const long long r = i / nx;
-    const int y = (int)(r % ny);
-    const int z = (int)(r / ny);
-    const bool inx = x >= gx && x < gx + ix, iny = y >= gy && y < gy + iy, inz = z >= gz && z < gz + iz;
-    bool interior;
-    if (d == 0)
-        interior = iny && inz;
-    else if (d == 1)
-        interior = inx && inz;
-    else
-        interior = inx && iny;
-    if (interior) return;
-    const long long idx = (long long)x + (long long)sy * y + (long long)sz * z;
-    for (int v = 0; v < nplanes; v++) dst[(long long)v * sv + idx] = src[(long long)v * sv + idx];
-}
-
-int copy_transverse_ghosts(Block *b, int d, const double *src, double *dst)
-{
-    const long long ncell = (long long)b->ng[0] * b->ng[1] * b->ng[2];
-    hipLaunchKernelGGL(k_copy_transverse_ghosts, dim3((unsigned)((ncell + 255) / 256)), dim3(256), 0, g_stream, src,
-                       dst, b->sv, g_nplanes, b->sy, b->sz, d, b->ng[0], b->ng[1], b->ng[2], b->g[0], b->g[1],
-                       b->g[2], b->n[0], b->n[1], b->n[2]);
-    HIPCHK(hipGetLastError());
-    return PK_OK;
-}
-
 // ---- fine/coarse flux points (set_fluxpointers / save_outfluxes,
 // grid_container_fcflx.F90:148-235) ------------------------------------
 
@@ -689,7 +652,6 @@ int do_stage(Block *b, int ddim, int istep, double dt, double ch)
         if (fc) fc_args(b, ddim, f, a);
         RCCHK(launch(ddim, false, a, b, f));
     }
-    RCCHK(copy_transverse_ghosts(b, ddim, state(b, src_i), state(b, dst_i)));
     if (fc) RCCHK(fc_end(b, ddim));
     if (first) {
         b->uh = b->cur;

@@ -41,6 +41,9 @@ struct SweepArgs {
     int nslots;
     int has_dir[3];
     double dl[3];
+    // stage mode only:
+    int gwgs;            // the launch's first gwgs workgroups (a multiple of 8) copy the cells outside the
+                         // transverse interior from src to dst (set by the launcher)
     // stage mode only: fine/coarse flux points of the pencils (null when none)
     const int *fc_at;    // [4][fc_npen]: the cell whose right-face flux is replaced (li, ri) or saved (lo, ro);
                          // kFcNone (below every lane's cell) where absent
@@ -93,10 +96,59 @@ struct StepScalars {
 // This workgroup's place in an XCD-aware order: workgroup i runs on XCD i % 8,
 // so each XCD gets a contiguous range of places, and tiles that share halo
 // cells or cache lines share an L2.
-__device__ __forceinline__ unsigned xcd_order()
+__device__ __forceinline__ unsigned xcd_order(unsigned w, unsigned n)
 {
-    const unsigned full = gridDim.x / 8u * 8u, w = blockIdx.x;
+    const unsigned full = n / 8u * 8u;
     return w < full ? (w % 8u) * (full / 8u) + w / 8u : w;
+}
+__device__ __forceinline__ unsigned xcd_order() { return xcd_order(blockIdx.x, gridDim.x); }
+
+// The t-th ghost cell of a block of i (interior) cells and g ghost layers on
+// each side per direction: z slabs (whole planes), then y slabs (interior z),
+// then x slabs.  False past the last one.
+__device__ __forceinline__ bool ghost_cell(unsigned t, const unsigned (&i)[3], const unsigned (&g)[3], unsigned (&c)[3])
+{
+    const unsigned nx = i[0] + 2u * g[0], ny = i[1] + 2u * g[1];
+    const unsigned rz = 2u * g[2] * nx * ny, ry = 2u * g[1] * i[2] * nx, rx = 2u * g[0] * i[2] * i[1];  // < 2^32 (launchers)
+    if (t < rz) {
+        const unsigned pl = nx * ny, l = t / pl, r = t - l * pl;
+        c[2] = l < g[2] ? l : i[2] + l;
+        c[1] = r / nx;
+        c[0] = r - c[1] * nx;
+        return true;
+    }
+    t -= rz;
+    if (t < ry) {
+        const unsigned pl = 2u * g[1] * nx, l = t / pl, r = t - l * pl;
+        const unsigned q = r / nx;
+        c[2] = g[2] + l;
+        c[1] = q < g[1] ? q : i[1] + q;
+        c[0] = r - q * nx;
+        return true;
+    }
+    t -= ry;
+    if (t >= rx) return false;
+    const unsigned pl = 2u * g[0] * i[1], l = t / pl, r = t - l * pl;
+    const unsigned q = r / (2u * g[0]), e = r - q * 2u * g[0];
+    c[2] = g[2] + l;
+    c[1] = g[1] + q;
+    c[0] = e < g[0] ? e : i[0] + e;
+    return true;
+}
+
+// Copies of the planes of one cell, G at a time so that the loads of a group
+// are in flight together.
+template <int G>
+__device__ __forceinline__ void copy_planes(const double *s, long long ssv, double *d, long long dsv, int np)
+{
+    for (int v0 = 0; v0 < np; v0 += G) {
+        double x[G];
+#pragma unroll
+        for (int v = 0; v < G; v++) x[v] = s[(long long)(v0 + v < np ? v0 + v : np - 1) * ssv];
+#pragma unroll
+        for (int v = 0; v < G; v++)
+            if (v0 + v < np) d[(long long)(v0 + v) * dsv] = x[v];
+    }
 }
 #endif
 
@@ -150,8 +202,8 @@ struct FaceJob {
     int nplanes;
     int wg0;             // the job's first workgroup in its launch (kFaceCells cells each)
 };
-// Cells one workgroup of k_exchange_faces copies (every plane of each).
-constexpr int kFaceCells = 512;
+// Cells one workgroup of k_exchange_faces copies (every plane of each), one per lane.
+constexpr int kFaceCells = 256;
 
 // Arrays of the reference layout and the planes of a state (k_planes):
 // aos[k] holds map[k].nc components per cell, null: not converted.
