@@ -333,12 +333,10 @@ class GridContainer:
         shape (nzg, nyg, nxg, nvar), (nzg, nyg, nxg, 3), (nzg, nyg, nxg),
         float64, contiguous, on this GPU) without host staging."""
         self.register()
-        ptr = lambda t: None if t is None else ctypes.c_void_p(_device_ptr(t))
-        _call("pk_upload_device", self.cg_id, ptr(u), ptr(b), ptr(psi))
+        _call("pk_upload_device", self.cg_id, *_device_ptrs(u, b, psi))
 
     def download_device(self, u, b=None, psi=None):
-        ptr = lambda t: None if t is None else ctypes.c_void_p(_device_ptr(t))
-        _call("pk_download_device", self.cg_id, ptr(u), ptr(b), ptr(psi))
+        _call("pk_download_device", self.cg_id, *_device_ptrs(u, b, psi))
 
     def unregister(self):
         if self.registered:
@@ -346,15 +344,30 @@ class GridContainer:
             self.registered = False
 
 
-def _device_ptr(t):
-    """Device address of a torch tensor handed to the library.  The library
-    works on its own stream: torch's queued work on the tensor is finished
-    first (the library's calls return with their own work finished)."""
-    if not (t.is_cuda and t.is_contiguous() and str(t.dtype) == "torch.float64"):
-        raise PiernikError("device arrays must be contiguous float64 tensors on the GPU")
+def _device_ptrs(*ts):
+    """Device addresses (ctypes; None where t is None) of torch tensors handed
+    to the library.  The library works on its own stream: torch's queued work
+    on the tensors is finished first, once for all of them on a device (the
+    library's calls return with their own work finished)."""
     import torch
-    torch.cuda.synchronize(t.device)
-    return t.data_ptr()
+
+    out, dev = [], None
+    for t in ts:
+        if t is None:
+            out.append(None)
+            continue
+        if not (t.is_cuda and t.dtype == torch.float64 and t.is_contiguous()):
+            raise PiernikError("device arrays must be contiguous float64 tensors on the GPU")
+        if t.device != dev:
+            dev = t.device
+            torch.cuda.synchronize(dev)
+        out.append(ctypes.c_void_p(t.data_ptr()))
+    return out
+
+
+def _device_ptr(t):
+    """The device address of one tensor, as _device_ptrs."""
+    return _device_ptrs(t)[0].value
 
 
 _cfg = None

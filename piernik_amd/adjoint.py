@@ -29,7 +29,7 @@ import ctypes
 
 import torch
 
-from . import PiernikError, _call, _device_ptr, timestep_fluid, fluid_update, update_boundaries
+from . import PiernikError, _call, _device_ptrs, timestep_fluid, fluid_update, update_boundaries
 from .setups import _DeviceBlock
 
 
@@ -103,7 +103,8 @@ class RolloutPlan:
         cg = self.cg
         single = torch.is_tensor(g)
         g = (g,) if single else tuple(g)
-        ptrs = [ctypes.c_void_p(_device_ptr(t.contiguous())) for t in g] + [None] * (3 - len(g))
+        g = [t.contiguous() for t in g]
+        ptrs = _device_ptrs(*g) + [None] * (3 - len(g))
         _call("pk_adjoint_set", cg.cg_id, *ptrs)
         carry = 0.0
         for seg in reversed(range(self.nck)):
@@ -124,7 +125,7 @@ class RolloutPlan:
                     carry = 0.0
         self.last_recorded = False  # the recomputed segments have overwritten the slots
         out = self._empty(g[0].device)
-        ptrs = [ctypes.c_void_p(_device_ptr(t)) for t in out] + [None] * (3 - len(out))
+        ptrs = _device_ptrs(*out) + [None] * (3 - len(out))
         _call("pk_adjoint_get", cg.cg_id, *ptrs)
         return out[0] if single else out
 
@@ -222,7 +223,8 @@ class EnsemblePlan:
         """dL/d(initial states) for dL/d(final states) = grads."""
         n = len(self.blocks)
         for cg, g in zip(self.blocks, grads):
-            ptrs = [ctypes.c_void_p(_device_ptr(t.contiguous())) for t in g] + [None] * (3 - len(g))
+            g = [t.contiguous() for t in g]
+            ptrs = _device_ptrs(*g) + [None] * (3 - len(g))
             _call("pk_adjoint_set", cg.cg_id, *ptrs)
         carry = [0.0] * n
         for seg in reversed(range(self.nck)):
@@ -246,7 +248,7 @@ class EnsemblePlan:
         out = []
         for cg, g in zip(self.blocks, grads):
             o = self._empty(cg, g[0].device)
-            ptrs = [ctypes.c_void_p(_device_ptr(t)) for t in o] + [None] * (3 - len(o))
+            ptrs = _device_ptrs(*o) + [None] * (3 - len(o))
             _call("pk_adjoint_get", cg.cg_id, *ptrs)
             out.append(o)
         return out
