@@ -473,49 +473,40 @@ __device__ double wg_range_sum(const double *__restrict__ part, long long lo, lo
 
 __device__ __forceinline__ long long range_lo(long long n, int g) { return n * g / kRedParts; }
 
-// grid (kRedParts, jobs): range g of a job, into part[n + g].  (One workgroup
+// range g of job j into part[n + g]: a workgroup per range.  (One workgroup
 // per job walked its 64 ranges one after the other, ten barriers each: 61 us
 // for the 40 sums of 20 instances.)
-__global__ __launch_bounds__(256) void k_sum_ranges_jobs(const SumJob *__restrict__ jobs)
+__device__ __forceinline__ void sum_range(const SumJob &j, int g)
 {
     __shared__ double red[256];
-    const SumJob j = jobs[blockIdx.y];
-    const int g = blockIdx.x;
     const double r = wg_range_sum(j.part, range_lo(j.n, g), range_lo(j.n, g + 1), red);
     if (threadIdx.x == 0) j.part[j.n + g] = r;
 }
 
-// the range sums of each job in order, a job per lane
-__global__ void k_sum_final_jobs(const SumJob *__restrict__ jobs, int njobs)
+// the range sums of job j in order: a wave fetches them, one lane adds
+__device__ __forceinline__ void sum_final(const SumJob &j)
 {
-    const int jb = blockIdx.x * blockDim.x + threadIdx.x;
-    if (jb >= njobs) return;
-    const SumJob j = jobs[jb];
+    static_assert(kRedParts == 64, "a range sum per lane");
+    __shared__ double v[kRedParts];
+    v[threadIdx.x] = j.part[j.n + threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x != 0) return;
     double tot = 0.0;
-    for (int g = 0; g < kRedParts; g++) tot += j.part[j.n + g];
+#pragma unroll
+    for (int g = 0; g < kRedParts; g++) tot += v[g];
     j.out[0] = tot;
 }
 
-// grid (kRedParts, 2): range g of partial array y, into part_y[n + g]
-__global__ __launch_bounds__(256) void k_sum_ranges(double *__restrict__ p0, double *__restrict__ p1, long long n)
+// The sums of all sweeps of a step (and of all instances) in two launches.
+// After every sweep they were two launches of 5 us each, which nothing
+// overlaps: 172 of the 1590 us of a 3-step gradient of a 45x40x34 MHD block.
+__global__ __launch_bounds__(256) void k_sum_ranges_jobs(const SumJob *__restrict__ jobs)
 {
-    __shared__ double red[256];
-    double *p = blockIdx.y ? p1 : p0;
-    const int g = blockIdx.x;
-    const double r = wg_range_sum(p, range_lo(n, g), range_lo(n, g + 1), red);
-    if (threadIdx.x == 0) p[n + g] = r;
+    sum_range(jobs[blockIdx.y], blockIdx.x);
 }
-
-// grid 2: the range sums in order
-__global__ void k_sum_final(const double *__restrict__ p0, const double *__restrict__ p1, long long n,
-                            double *__restrict__ out)
-{
-    if (threadIdx.x != 0) return;
-    const double *p = blockIdx.x ? p1 : p0;
-    double tot = 0.0;
-    for (int g = 0; g < kRedParts; g++) tot += p[n + g];
-    out[blockIdx.x] = tot;
-}
+__global__ __launch_bounds__(64) void k_sum_final_jobs(const SumJob *__restrict__ jobs) { sum_final(jobs[blockIdx.x]); }
+__global__ __launch_bounds__(256) void k_sum_ranges(const SweepSums s) { sum_range(s.job[blockIdx.y], blockIdx.x); }
+__global__ __launch_bounds__(64) void k_sum_final(const SweepSums s) { sum_final(s.job[blockIdx.x]); }
 
 __global__ void k_zero_best(unsigned long long *best)
 {
@@ -770,7 +761,15 @@ hipError_t launch_sum_parts_jobs(const SumJob *jobs, int njobs, hipStream_t st)
         const int n = njobs - j0 < 32768 ? njobs - j0 : 32768;
         hipLaunchKernelGGL(k_sum_ranges_jobs, dim3(kRedParts, (unsigned)n), dim3(256), 0, st, jobs + j0);
     }
-    hipLaunchKernelGGL(k_sum_final_jobs, dim3((unsigned)((njobs + 63) / 64)), dim3(64), 0, st, jobs, njobs);
+    hipLaunchKernelGGL(k_sum_final_jobs, dim3((unsigned)njobs), dim3(64), 0, st, jobs);
+    return hipGetLastError();
+}
+
+hipError_t launch_sweep_sums(const SweepSums &s, int njobs, hipStream_t st)
+{
+    if (njobs < 1 || njobs > 2 * kStepSweeps) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_sum_ranges, dim3(kRedParts, (unsigned)njobs), dim3(256), 0, st, s);
+    hipLaunchKernelGGL(k_sum_final, dim3((unsigned)njobs), dim3(64), 0, st, s);
     return hipGetLastError();
 }
 
@@ -788,17 +787,12 @@ static hipError_t adj_dir(int dir, const AdjArgs &a, int nt, long long nblk, hip
 // their sums of the same partials agree bit for bit.
 long long sweep_adjoint_parts(const AdjArgs &a) { return (long long)a.chunks * a.ptiles * 4; }
 
-hipError_t launch_sweep_adjoint(int dir, bool mhd, const AdjArgs &a, double *dtb_out, hipStream_t st)
+hipError_t launch_sweep_adjoint(int dir, bool mhd, const AdjArgs &a, hipStream_t st)
 {
     const int nt = 256;
     if (a.TP * a.TS < 1 || a.TP * a.TS > nt || a.out < 1 || a.out != a.TS - 16) return hipErrorInvalidValue;
     const long long nblk = (long long)a.chunks * a.ptiles;
-    hipError_t e = mhd ? adj_dir<MHD>(dir, a, nt, nblk, st) : adj_dir<HD>(dir, a, nt, nblk, st);
-    if (e != hipSuccess) return e;
-    const long long n = sweep_adjoint_parts(a);
-    hipLaunchKernelGGL(k_sum_ranges, dim3(kRedParts, 2), dim3(256), 0, st, a.dtb_part, a.chb_part, n);
-    hipLaunchKernelGGL(k_sum_final, dim3(2), dim3(64), 0, st, a.dtb_part, a.chb_part, n, dtb_out);
-    return hipGetLastError();
+    return mhd ? adj_dir<MHD>(dir, a, nt, nblk, st) : adj_dir<HD>(dir, a, nt, nblk, st);
 }
 
 hipError_t launch_dt_adjoint_batch(const DtBatchJob *jobs, int njobs, hipStream_t st)

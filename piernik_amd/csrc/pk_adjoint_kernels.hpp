@@ -60,7 +60,13 @@ struct AdjListArgs {
 struct SumJob {
     double *part;
     long long n;
-    double *out;
+    double *out;  // device or pinned host memory
+};
+
+// The sums of one block's sweeps of a step (dL/d(dt) and dL/d(ch) of each).
+constexpr int kStepSweeps = 6;
+struct SweepSums {
+    SumJob job[2 * kStepSweeps];
 };
 
 // Batched timestep adjoint over independent instances: per job the minimum
@@ -81,8 +87,9 @@ long long sweep_adjoint_parts(const AdjArgs &a);
 hipError_t launch_dt_adjoint_batch(const DtBatchJob *jobs, int njobs, hipStream_t st);
 hipError_t launch_sweep_adjoint_list(int dir, bool mhd, int lim, int limb, const AdjListArgs &L, hipStream_t st);
 hipError_t launch_sum_parts_jobs(const SumJob *jobs, int njobs, hipStream_t st);
-// dtb_out[0] = dL/d(dt) at fixed ch, dtb_out[1] = dL/d(ch)
-hipError_t launch_sweep_adjoint(int dir, bool mhd, const AdjArgs &a, double *dtb_out, hipStream_t st);
+hipError_t launch_sweep_sums(const SweepSums &s, int njobs, hipStream_t st);
+// leaves the partial sums of dL/d(dt) at fixed ch and of dL/d(ch) in a.dtb_part, a.chb_part
+hipError_t launch_sweep_adjoint(int dir, bool mhd, const AdjArgs &a, hipStream_t st);
 hipError_t launch_dt_adjoint(const DtAdjArgs &a, unsigned long long *best, double *lam, hipStream_t st);
 
 }  // namespace pk

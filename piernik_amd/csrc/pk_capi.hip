@@ -57,10 +57,9 @@ struct Block {
     std::vector<char> slot_stale;  // the slot's ghosts are old (periodic images of its interior replace them)
     double *lam[2] = {nullptr, nullptr};
     int lcur = 0;
-    double *d_dtb_part = nullptr;
+    double *d_dtb_part = nullptr;             // per sweep of a step: dtb_parts partials and kRedParts range sums
     double *d_chb_part = nullptr;
     long long dtb_parts = 0;
-    double *d_dtb = nullptr;
     unsigned long long *d_best = nullptr;
     // the block whose interior adjoins each ghost face (pk_set_neighbour):
     // nbr[d][0] low side, nbr[d][1] high side; the block's own id when it is
@@ -873,11 +872,9 @@ void free_adjoint(Block *b)
     }
     if (b->d_dtb_part) (void)hipFree(b->d_dtb_part);
     if (b->d_chb_part) (void)hipFree(b->d_chb_part);
-    if (b->d_dtb) (void)hipFree(b->d_dtb);
     if (b->d_best) (void)hipFree(b->d_best);
     b->d_dtb_part = nullptr;
     b->d_chb_part = nullptr;
-    b->d_dtb = nullptr;
     b->d_best = nullptr;
     b->dtb_parts = 0;
 }
@@ -1078,25 +1075,28 @@ void adj_tile(const Block *b, int d, int &TP, int &TS, int &out, int &chunks, in
     ptiles = (int)((npen + TP - 1) / TP);
 }
 
+// the partial sums of a step's k-th sweep
+double *sweep_part(double *parts, const Block *b, int k) { return parts + (b->dtb_parts + pk::kRedParts) * k; }
+
 // lam <- adjoint of the fused sweep along d linearised at state u (a slot).
-// dL/d(dt) at fixed ch and dL/d(ch) land in d_dtb[2*out_slot ..]; with dtb
-// set they are also read back and added to *dtb, *chb.
-int do_sweep_adjoint(Block *b, const double *u, int d, double dt, double ch, double psi_fac, double *dtb,
-                     double *chb, int out_slot = 0)
+// sums gets the two jobs that add up dL/d(dt) at fixed ch and dL/d(ch)
+// of the step's k-th sweep, into g_pinned[2 k] and [2 k + 1].
+int do_sweep_adjoint(Block *b, const double *u, int d, double dt, double ch, double psi_fac, pk::SweepSums *sums,
+                     int k)
 {
     pk::AdjArgs a{};
     a.u = u + b->xo;
     a.lam_out = b->lam[b->lcur] + b->xo;
     a.lam_in = b->lam[1 - b->lcur] + b->xo;
-    a.dtb_part = b->d_dtb_part;
-    a.chb_part = b->d_chb_part;
+    a.dtb_part = sweep_part(b->d_dtb_part, b, k);
+    a.chb_part = sweep_part(b->d_chb_part, b, k);
     a.sv = b->sv;
     a.sy = b->sy;
     a.sz = b->sz;
-    for (int k = 0; k < 3; k++) {
-        a.ng[k] = b->ng[k];
-        a.g[k] = b->g[k];
-        a.n[k] = b->n[k];
+    for (int q = 0; q < 3; q++) {
+        a.ng[q] = b->ng[q];
+        a.g[q] = b->g[q];
+        a.n[q] = b->n[q];
     }
     adj_tile(b, d, a.TP, a.TS, a.out, a.chunks, a.ptiles);
     if (pk::sweep_adjoint_parts(a) > b->dtb_parts) return fail(PK_EINVAL, "adjoint partial-sum buffer too small");
@@ -1116,15 +1116,11 @@ int do_sweep_adjoint(Block *b, const double *u, int d, double dt, double ch, dou
     a.smallei = g_cfg.smallei;
     a.use_smalld = g_cfg.use_smalld;
     a.use_smallei = g_cfg.use_smallei;
-    HIPCHK(pk::launch_sweep_adjoint(d, g_mhd, a, b->d_dtb + 2 * out_slot, g_stream));
+    HIPCHK(pk::launch_sweep_adjoint(d, g_mhd, a, g_stream));
     b->lcur = 1 - b->lcur;
-    if (dtb) {
-        HIPCHK(hipMemcpyAsync(g_pinned, b->d_dtb + 2 * out_slot, 2 * sizeof(double), hipMemcpyDeviceToHost,
-                              g_stream));
-        HIPCHK(hipStreamSynchronize(g_stream));
-        *dtb += g_pinned[0];
-        *chb += g_pinned[1];
-    }
+    const long long n = pk::sweep_adjoint_parts(a);
+    sums->job[2 * k] = pk::SumJob{a.dtb_part, n, g_pinned + 2 * k};
+    sums->job[2 * k + 1] = pk::SumJob{a.chb_part, n, g_pinned + 2 * k + 1};
     return PK_OK;
 }
 
@@ -1257,8 +1253,7 @@ struct ListState {
     bool fresh = false;  // ghosts current and dtout holds the timestep of the current state
     bool filled = false; // the ghosts were refreshed since the state last changed
     // blocks connected to other blocks (pk_set_neighbour): ghost faces come from
-    // the neighbours through an exchange before every sweep instead of the
-    // sweep's periodic images
+    // the neighbours through an exchange before every sweep
     bool linked = false;
     bool ghosts_stale = false;  // linked list after a step: the ghosts other than the swept faces are old
     FaceTab ex[3][2];           // per direction and buffer parity
@@ -1286,7 +1281,7 @@ struct EnsembleState {
     pk::CopyJob *d_jobs = nullptr;
     std::vector<pk::CopyJob> h_jobs;
     // reverse mode
-    pk::AdjArgs *d_adj = nullptr, *h_adj = nullptr;  // per block (pinned host copy)
+    pk::AdjArgs *d_adj = nullptr, *h_adj = nullptr;  // per sweep of a step and block (pinned host copy)
     unsigned *d_afirst[3] = {nullptr, nullptr, nullptr}, *d_aitems[3] = {nullptr, nullptr, nullptr};
     unsigned anitems[3] = {0, 0, 0};
     bool adj_built = false;
@@ -1296,7 +1291,7 @@ struct EnsembleState {
     std::vector<pk::DtBatchJob> h_dtj;
     double *d_mn = nullptr;
     unsigned long long *d_best = nullptr;
-    double *d_sums = nullptr, *h_sums = nullptr;  // per block, per sweep: dtb, chb
+    double *h_sums = nullptr;                        // pinned; per sweep and block: dtb, chb
 };
 EnsembleState g_ens;
 
@@ -1355,7 +1350,6 @@ void ens_free()
     if (g_ens.d_dtj) (void)hipFree(g_ens.d_dtj);
     if (g_ens.d_mn) (void)hipFree(g_ens.d_mn);
     if (g_ens.d_best) (void)hipFree(g_ens.d_best);
-    if (g_ens.d_sums) (void)hipFree(g_ens.d_sums);
     if (g_ens.h_sums) (void)hipHostFree(g_ens.h_sums);
     g_ens = EnsembleState();
 }
@@ -1983,12 +1977,11 @@ int ens_adj_build()
 {
     if (g_ens.adj_built) return PK_OK;
     const size_t n = g_ens.nblk;
-    HIPCHK(hipMalloc((void **)&g_ens.d_adj, sizeof(pk::AdjArgs) * n));
-    HIPCHK(hipHostMalloc((void **)&g_ens.h_adj, sizeof(pk::AdjArgs) * n, hipHostMallocDefault));
-    HIPCHK(hipMalloc((void **)&g_ens.d_sum, sizeof(pk::SumJob) * 2 * n));
-    HIPCHK(hipMalloc((void **)&g_ens.d_sums, sizeof(double) * 12 * n));
-    HIPCHK(hipHostMalloc((void **)&g_ens.h_sums, sizeof(double) * 12 * n, hipHostMallocDefault));
-    g_ens.h_sum.resize(2 * n);
+    HIPCHK(hipMalloc((void **)&g_ens.d_adj, sizeof(pk::AdjArgs) * pk::kStepSweeps * n));
+    HIPCHK(hipHostMalloc((void **)&g_ens.h_adj, sizeof(pk::AdjArgs) * pk::kStepSweeps * n, hipHostMallocDefault));
+    HIPCHK(hipMalloc((void **)&g_ens.d_sum, sizeof(pk::SumJob) * 2 * pk::kStepSweeps * n));
+    HIPCHK(hipHostMalloc((void **)&g_ens.h_sums, sizeof(double) * 2 * pk::kStepSweeps * n, hipHostMallocDefault));
+    g_ens.h_sum.resize(2 * pk::kStepSweeps * n);
     for (int d = 0; d < 3; d++) {
         if (!g_cfg.has_dir[d]) continue;
         std::vector<unsigned> first(n + 1);
@@ -3392,10 +3385,9 @@ int pk_adjoint_setup(int64_t cg_id, int32_t nslots)
         const long long p = (long long)chunks * ptiles * 4;  // 4 waves per tile: 256-lane list workgroups too
         if (p > parts) parts = p;
     }
-    HIPCHK(hipMalloc((void **)&b->d_dtb_part, sizeof(double) * (parts + pk::kRedParts)));
-    HIPCHK(hipMalloc((void **)&b->d_chb_part, sizeof(double) * (parts + pk::kRedParts)));
+    HIPCHK(hipMalloc((void **)&b->d_dtb_part, sizeof(double) * pk::kStepSweeps * (parts + pk::kRedParts)));
+    HIPCHK(hipMalloc((void **)&b->d_chb_part, sizeof(double) * pk::kStepSweeps * (parts + pk::kRedParts)));
     b->dtb_parts = parts;
-    HIPCHK(hipMalloc((void **)&b->d_dtb, 2 * 6 * sizeof(double)));
     HIPCHK(hipMalloc((void **)&b->d_best, sizeof(unsigned long long)));
     b->lcur = 0;
     HIPCHK(hipStreamSynchronize(g_stream));
@@ -3462,10 +3454,12 @@ int pk_sweep_adjoint(int64_t cg_id, int32_t slot, int32_t ddim, double dt, doubl
     RCCHK(slot_ptr(b, slot, &p));
     if (ddim < 0 || ddim > 2 || !g_cfg.has_dir[ddim]) return fail(PK_EINVAL, "inactive or bad direction %d", ddim);
     if (!(dt > 0.0)) return fail(PK_EINVAL, "dt must be positive");
-    double dtb = 0.0, chb = 0.0;
-    RCCHK(do_sweep_adjoint(b, p, ddim, dt, chspeed, psi_fac, &dtb, &chb));
-    if (dt_bar) *dt_bar += dtb;
-    if (ch_bar) *ch_bar += chb;
+    pk::SweepSums sums;
+    RCCHK(do_sweep_adjoint(b, p, ddim, dt, chspeed, psi_fac, &sums, 0));
+    HIPCHK(pk::launch_sweep_sums(sums, 2, g_stream));
+    HIPCHK(hipStreamSynchronize(g_stream));
+    if (dt_bar) *dt_bar += g_pinned[0];
+    if (ch_bar) *ch_bar += g_pinned[1];
     return PK_OK;
 }
 
@@ -3514,10 +3508,10 @@ int pk_fluid_update_adjoint(int64_t cg_id, int32_t slot0, double dt, double *dt_
     double ch, fac;
     block_glm(b, dt, &ch, &fac);
     double dtb = 0.0, chb = 0.0;
+    pk::SweepSums sums;
     for (int i = (int)dirs.size() - 1; i >= 0; i--)
-        RCCHK(do_sweep_adjoint(b, b->slots[slot0 + i], dirs[i], dt, ch, damp[i] ? fac : 1.0, nullptr, nullptr, i));
-    // the sweeps' sums, read back once
-    HIPCHK(hipMemcpyAsync(g_pinned, b->d_dtb, 2 * dirs.size() * sizeof(double), hipMemcpyDeviceToHost, g_stream));
+        RCCHK(do_sweep_adjoint(b, b->slots[slot0 + i], dirs[i], dt, ch, damp[i] ? fac : 1.0, &sums, i));
+    HIPCHK(pk::launch_sweep_sums(sums, 2 * (int)dirs.size(), g_stream));
     HIPCHK(hipStreamSynchronize(g_stream));
     for (size_t i = 0; i < dirs.size(); i++) {
         dtb += g_pinned[2 * i];
@@ -3723,18 +3717,26 @@ int pk_ensemble_step_adjoint(const double *dts, int32_t slot0, double *dt_bar)
     std::vector<double> ch(n, 0.0), fac(n, 1.0);
     for (size_t i = 0; i < n; i++)
         if (g_mhd) glm_scalars({g_list.mdl[i]}, dts[i], &ch[i], &fac[i]);
-    for (int k = (int)dirs.size() - 1; k >= 0; k--) {
+    // the tables of every sweep in one copy each, then the sweeps back to back
+    // (a synchronisation and two copies before each one left the device idle
+    // for as long as a table took to fill)
+    const int nsw = (int)dirs.size();
+    for (int k = 0; k < nsw; k++)
+        if (slot0 + k >= (int)g_list.blocks[0]->slots.size())
+            return fail(PK_EINVAL, "slot %d does not exist", slot0 + k);
+    HIPCHK(hipStreamSynchronize(g_stream));  // the pinned tables may still feed the previous copy
+    for (int k = nsw - 1; k >= 0; k--) {
         const int d = dirs[k];
-        HIPCHK(hipStreamSynchronize(g_stream));  // the pinned tables may still feed the previous copy
+        const int cur = (nsw - 1 - k) % 2 == 0 ? lc : 1 - lc;  // the adjoint buffer this sweep reads is lam[cur]
         for (size_t i = 0; i < n; i++) {
             Block *b = g_list.blocks[i];
             if (slot0 + k >= (int)b->slots.size()) return fail(PK_EINVAL, "slot %d does not exist", slot0 + k);
             pk::AdjArgs a{};
             a.u = b->slots[slot0 + k] + b->xo;
-            a.lam_out = b->lam[b->lcur] + b->xo;
-            a.lam_in = b->lam[1 - b->lcur] + b->xo;
-            a.dtb_part = b->d_dtb_part;
-            a.chb_part = b->d_chb_part;
+            a.lam_out = b->lam[cur] + b->xo;
+            a.lam_in = b->lam[1 - cur] + b->xo;
+            a.dtb_part = sweep_part(b->d_dtb_part, b, k);
+            a.chb_part = sweep_part(b->d_chb_part, b, k);
             a.sv = b->sv;
             a.sy = b->sy;
             a.sz = b->sz;
@@ -3760,30 +3762,33 @@ int pk_ensemble_step_adjoint(const double *dts, int32_t slot0, double *dt_bar)
             a.smallei = g_cfg.smallei;
             a.use_smalld = g_cfg.use_smalld;
             a.use_smallei = g_cfg.use_smallei;
-            g_ens.h_adj[i] = a;
-            const long long parts = (long long)a.chunks * a.ptiles * 4;
-            g_ens.h_sum[2 * i] = pk::SumJob{b->d_dtb_part, parts, g_ens.d_sums + 12 * i + 2 * k};
-            g_ens.h_sum[2 * i + 1] = pk::SumJob{b->d_chb_part, parts, g_ens.d_sums + 12 * i + 2 * k + 1};
+            const size_t at = (size_t)k * n + i;
+            g_ens.h_adj[at] = a;
+            const long long parts = pk::sweep_adjoint_parts(a);
+            g_ens.h_sum[2 * at] = pk::SumJob{a.dtb_part, parts, g_ens.h_sums + 2 * at};
+            g_ens.h_sum[2 * at + 1] = pk::SumJob{a.chb_part, parts, g_ens.h_sums + 2 * at + 1};
         }
-        HIPCHK(hipMemcpyAsync(g_ens.d_adj, g_ens.h_adj, sizeof(pk::AdjArgs) * n, hipMemcpyHostToDevice, g_stream));
-        HIPCHK(hipMemcpyAsync(g_ens.d_sum, g_ens.h_sum.data(), sizeof(pk::SumJob) * 2 * n, hipMemcpyHostToDevice,
-                              g_stream));
+    }
+    HIPCHK(hipMemcpyAsync(g_ens.d_adj, g_ens.h_adj, sizeof(pk::AdjArgs) * nsw * n, hipMemcpyHostToDevice, g_stream));
+    HIPCHK(hipMemcpyAsync(g_ens.d_sum, g_ens.h_sum.data(), sizeof(pk::SumJob) * 2 * nsw * n, hipMemcpyHostToDevice,
+                          g_stream));
+    for (int k = nsw - 1; k >= 0; k--) {
+        const int d = dirs[k];
         pk::AdjListArgs L{};
-        L.args = g_ens.d_adj;
+        L.args = g_ens.d_adj + (size_t)k * n;
         L.first = g_ens.d_afirst[d];
         L.items = g_ens.d_aitems[d];
         L.nitems = g_ens.anitems[d];
         HIPCHK(pk::launch_sweep_adjoint_list(d, g_mhd, g_cfg.limiter, g_cfg.limiter_b, L, g_stream));
-        HIPCHK(pk::launch_sum_parts_jobs(g_ens.d_sum, (int)(2 * n), g_stream));
         for (Block *b : g_list.blocks) b->lcur = 1 - b->lcur;
     }
-    HIPCHK(hipMemcpyAsync(g_ens.h_sums, g_ens.d_sums, sizeof(double) * 12 * n, hipMemcpyDeviceToHost, g_stream));
+    HIPCHK(pk::launch_sum_parts_jobs(g_ens.d_sum, (int)(2 * nsw * n), g_stream));
     HIPCHK(hipStreamSynchronize(g_stream));
     for (size_t i = 0; i < n; i++) {
         double dtb = 0.0, chb = 0.0;
         for (size_t k = 0; k < dirs.size(); k++) {
-            dtb += g_ens.h_sums[12 * i + 2 * k];
-            chb += g_ens.h_sums[12 * i + 2 * k + 1];
+            dtb += g_ens.h_sums[2 * (k * n + i)];
+            chb += g_ens.h_sums[2 * (k * n + i) + 1];
         }
         // ch = cfl_glm*min(dl)/dt (hdc.F90:122)
         if (g_mhd) dtb += chb * (-(ch[i] / dts[i]));

@@ -1,6 +1,6 @@
 // pk_stream.hpp -- the fused RK2 sweep as a stream (included by
-// pk_kernels.hip inside its namespace; uses plane_of, tile helpers, floors,
-// the timestep fold and the periodic images defined there).
+// pk_kernels.hip inside its namespace; uses the helpers of pk_tile.hpp, the
+// floors and the timestep fold).
 //
 // One wave per workgroup walks a stream of positions along the sweep.  TP
 // pencils (consecutive along the first transverse direction: x for y and z
