@@ -807,9 +807,11 @@ void glm_scalars(const std::vector<double> &mdls, double dt, double *ch_out, dou
     *fac_out = std::exp(-f);
 }
 
-// One step of fluid_update.  The RK2 sweeps leave the periodic ghosts old
+// One step of fluid_update.  wrap: the block's ghosts are its periodic images
+// (or old), so that the first sweep need not read them; the later sweeps
+// always read their pre-images.  The RK2 sweeps leave the ghosts old
 // (b->ghosts_stale): the caller refills them with do_fill before they are read.
-int do_fluid_update(Block *b, double dt)
+int do_fluid_update(Block *b, double dt, bool wrap)
 {
     double ch = 0.0, fac = 1.0;
     if (g_mhd) glm_scalars({min_dl(b)}, dt, &ch, &fac);
@@ -824,7 +826,8 @@ int do_fluid_update(Block *b, double dt)
             if (!g_cfg.has_dir[d]) continue;
             if (g_cfg.integration_order == 2) {
                 // the last sweep of the step also reduces the next step's timestep
-                RCCHK(do_sweep(b, d, dt, ch, (d == last) ? fac : 1.0, true, half == 1 && d == last));
+                RCCHK(do_sweep(b, d, dt, ch, (d == last) ? fac : 1.0, wrap, half == 1 && d == last));
+                wrap = true;
             } else {
                 RCCHK(do_sweep(b, d, dt, ch, (d == last) ? fac : 1.0));
                 RCCHK(do_fill(b));
@@ -1473,6 +1476,14 @@ int build_tab(LaunchTab &t, const std::vector<Block *> &blks, int d, int f, int 
                           g_stream));
     HIPCHK(pk::launch_fill_items(t.d_first, (int)blks.size(), t.d_items, g_stream));
     t.grid = list_resident(d, g_fmag[f], nt);
+    // stream: whole rounds of the workgroups the device holds, about 8 items
+    // each, so that the workgroups in flight walk a window that moves over the
+    // list.  In one round each walks far from the others: 4096 two-fluid blocks
+    // (240000 items, 54 GB) took 308 ms a step so, 225 in rounds (223 with one
+    // item a workgroup, 226 with 4; queues 220); lists up to 12 M cells stay at
+    // one round, which starts the stream least often.
+    const long long round = 8ll * t.grid;
+    if (t.grid > 0 && t.nitems > round) t.grid *= (int)((t.nitems + round / 2) / round);
     if (t.grid > 0 && t.nitems < (unsigned)t.grid) t.grid = (int)t.nitems;
     if (t.grid <= 0) return fail(PK_EHIP, "no resident workgroups for the list sweep (nt = %d)", nt);
     HIPCHK(hipStreamSynchronize(g_stream));
@@ -1722,11 +1733,27 @@ std::vector<SweepStep> step_sweeps()
     return v;
 }
 
+// Makes the tables of the sweeps along d read ghosts as they are (wrap 0) or
+// their pre-images (1, as built).
+int list_set_wrap(int d, int wrap)
+{
+    for (int f = 0; f < g_nfl; f++)
+        for (LaunchTab *t : {&g_list.tab[d][f], &g_list.stab[d][f]}) {
+            if (t->nitems == 0) continue;
+            for (pk::SweepArgs &a : t->h_args) a.wrap = wrap;
+            HIPCHK(hipMemcpyAsync(t->d_args, t->h_args.data(), sizeof(pk::SweepArgs) * t->h_args.size(),
+                                  hipMemcpyHostToDevice, g_stream));
+        }
+    HIPCHK(hipStreamSynchronize(g_stream));
+    return PK_OK;
+}
+
 // Enqueue the launches of one step on g_stream.  mode PK_BATCH_PER_BLOCK
 // launches the single-block sweep once per block with the same tile shapes
 // (for items of the stream form, the block's single-block shape); the
 // list modes launch the list sweep once per sweep and fluid.
-int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
+// given: the first sweep reads the ghosts as they are (not in a captured step).
+int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false, bool given = false)
 {
     const std::vector<SweepStep> sw = step_sweeps();
     const bool persistent = mode != PK_BATCH_PER_BLOCK;
@@ -1737,6 +1764,7 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
         const int d = sw[k].d;
         const int parity = (int)(k % 2);
         if (g_list.linked && !ens) RCCHK(exchange(d, parity));
+        if (given && k == 0) RCCHK(list_set_wrap(d, 0));
         for (int f = 0; f < g_nfl; f++) {
             for (LaunchTab *tp : {&g_list.tab[d][f], &g_list.stab[d][f]}) {
                 LaunchTab &t = *tp;
@@ -1788,6 +1816,7 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
                 }
             }
         }
+        if (given && k == 0) RCCHK(list_set_wrap(d, 1));
     }
     if (ens)
         HIPCHK(pk::launch_dtslots_final(g_ens.d_dtslots, kEnsSlots, (int)g_ens.nblk, g_ens.dtout, g_stream));
@@ -2845,7 +2874,7 @@ int pk_fluid_update(int64_t cg_id, double dt)
     RCCHK(solo(b));
     if (!(dt > 0.0)) return fail(PK_EINVAL, "dt must be positive");
     list_touch();
-    RCCHK(do_fluid_update(b, dt));
+    RCCHK(do_fluid_update(b, dt, false));
     if (b->ghosts_stale) RCCHK(do_fill(b));
     return PK_OK;
 }
@@ -2862,7 +2891,7 @@ int pk_run(int64_t cg_id, int32_t nsteps, double *t_out, double *dt_out)
     StepLoop L;
     L.blocks = {b};
     L.timestep = [b](double *dt, double *c) { return do_timestep(b, dt, c); };
-    L.update = [b](double dt) { return do_fluid_update(b, dt); };
+    L.update = [b](double dt) { return do_fluid_update(b, dt, true); };
     RCCHK(run_loop(L, nsteps, t_out, dt_out, &g_last_redone));
     if (b->ghosts_stale) RCCHK(do_fill(b));
     return PK_OK;
@@ -3482,10 +3511,10 @@ int pk_fluid_update_record(int64_t cg_id, int32_t slot0, double dt)
     for (size_t i = 0; i < dirs.size(); i++) b->slot_stale[slot0 + i] = i > 0;
     HIPCHK(hipMemcpyAsync(b->slots[slot0], b->buf[b->cur], state_bytes(b), hipMemcpyDeviceToDevice, g_stream));
     for (size_t i = 0; i + 1 < dirs.size(); i++)
-        RCCHK(do_sweep(b, dirs[i], dt, ch, damp[i] ? fac : 1.0, true, false, b->slots[slot0 + i],
+        RCCHK(do_sweep(b, dirs[i], dt, ch, damp[i] ? fac : 1.0, i > 0, false, b->slots[slot0 + i],
                        b->slots[slot0 + i + 1]));
     const size_t l = dirs.size() - 1;
-    RCCHK(do_sweep(b, dirs[l], dt, ch, damp[l] ? fac : 1.0, true, true, b->slots[slot0 + l], b->buf[1 - b->cur]));
+    RCCHK(do_sweep(b, dirs[l], dt, ch, damp[l] ? fac : 1.0, l > 0, true, b->slots[slot0 + l], b->buf[1 - b->cur]));
     b->cur = 1 - b->cur;
     b->uh = -1;
     b->dt_pending = false;
@@ -3599,12 +3628,13 @@ int pk_ensemble_step(int32_t mode, int32_t first, double *dt_out, int32_t *cappe
         g_ens.dt_old[i] = dt[i];
     }
     RCCHK(ens_set_step(dt.data()));
-    if (mode == PK_BATCH_GRAPH) {
+    const bool given = !g_list.wrap_stale;  // ghosts a caller may have set: the first sweep reads them
+    if (mode == PK_BATCH_GRAPH && !given) {
         RCCHK(ens_graph());
         HIPCHK(hipGraphLaunch(g_ens.exec, g_stream));
     } else {
         pk::StepScalars sc{};
-        RCCHK(enqueue_step(mode, sc, true));
+        RCCHK(enqueue_step(mode == PK_BATCH_GRAPH ? PK_BATCH_PERSISTENT : mode, sc, true, given));
     }
     for (Block *b : g_list.blocks) {
         b->uh = -1;
@@ -3670,6 +3700,8 @@ int pk_ensemble_record_step(const double *dts, int32_t slot0)
     for (size_t k = 0; k < dirs.size(); k++) {
         RCCHK(ens_copy_slots(slot0 + (int)k, true, (int)(k % 2)));
         const int d = dirs[k];
+        const bool given = !g_list.wrap_stale;  // the first sweep of a state whose ghosts are current
+        if (given) RCCHK(list_set_wrap(d, 0));
         for (int f = 0; f < g_nfl; f++) {
             for (int part = 0; part < 2; part++) {
                 LaunchTab &t = part ? g_list.stab[d][f] : g_list.tab[d][f];
@@ -3689,9 +3721,10 @@ int pk_ensemble_record_step(const double *dts, int32_t slot0)
                 HIPCHK(list_kernel(d, g_fmag[f], L, t.nt, t.grid));
             }
         }
+        if (given) RCCHK(list_set_wrap(d, 1));
+        g_list.wrap_stale = true;  // from here on: the later slots' ghosts are old too
     }
     list_touch();
-    g_list.wrap_stale = true;
     for (Block *b : g_list.blocks) {
         b->dt_pending = false;
         b->uh = -1;

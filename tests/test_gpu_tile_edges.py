@@ -7,6 +7,8 @@ partly empty, and lists whose launches have fewer items than CUs.
 Bit for bit against the oracle, as the rest of the exact build.  A pinned
 tile runs beside the default: a tile changes who computes a cell, never how.
 """
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -78,3 +80,55 @@ def test_list_items_bit_exact(oracle, shapes, lanes, ts):
         cg.download()
         assert_same(cg, ob, f"list {cg.n}")
     pk.finalize()
+
+
+@pytest.mark.parametrize("n", [(12, 9, 8), (5, 4, 33)])
+def test_step_reads_the_ghosts_it_is_given(n):
+    """A single step from ghosts that are not periodic images: its first sweep
+    reads them as they are, the later ones see refreshed ghosts; sweep by
+    sweep with refreshes in between gives the same bits."""
+    cfg = pk.Config(limiter="vanleer", smalld=1e-3, smallei=1e-4)
+    out = []
+    for whole in (True, False):
+        pk.load_library()
+        pk.finalize()
+        pk.init(cfg)
+        cg = setups.smooth_random(n, nb=4, seed=7, gamma=cfg.gamma)
+        cg.u[:, :4] *= 1.25
+        cg.upload()
+        if whole:
+            pk.fluid_update(cg, 1e-3)
+        else:
+            for d in (0, 1, 2, 2, 1, 0):
+                pk.sweep(cg, d, 1e-3)
+                pk.update_boundaries(cg)
+        cg.download()
+        out.append(cg.u.copy())
+        pk.finalize()
+    assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("mode", [pk.BATCH_GRAPH, pk.BATCH_PERSISTENT, pk.BATCH_PER_BLOCK])
+def test_ensemble_step_reads_the_ghosts_it_is_given(mode):
+    """As above for an ensemble of one: its steps equal fluid_update's with
+    the same dt, from ghosts that are not periodic images and after."""
+    cfg = pk.Config(limiter="vanleer", smalld=1e-3, smallei=1e-4)
+    out, dts = [], []
+    for ens in (True, False):
+        pk.load_library()
+        pk.finalize()
+        pk.init(cfg)
+        cg = setups.smooth_random((12, 9, 8), nb=4, seed=7, gamma=cfg.gamma)
+        cg.u[:, :4] *= 1.25
+        cg.upload()
+        for s in range(2):
+            if ens:
+                dt, cap = (ctypes.c_double * 1)(), (ctypes.c_int32 * 1)()
+                pk._call("pk_ensemble_step", int(mode), int(s == 0), dt, cap)
+                dts.append(dt[0])
+            else:
+                pk.fluid_update(cg, dts[s])
+        cg.download()
+        out.append(cg.u.copy())
+        pk.finalize()
+    assert np.array_equal(out[0], out[1])
