@@ -96,7 +96,7 @@ typedef struct pk_stage_report {
 } pk_stage_report;
 
 /* Execution of the block-list entry points (pk_*_all). */
-#define PK_BATCH_GRAPH 0       /* one persistent launch per sweep and fluid, the step captured in a HIP graph */
+#define PK_BATCH_GRAPH 0       /* one launch per sweep and fluid, the step captured in a HIP graph */
 #define PK_BATCH_PERSISTENT 1  /* the same launches issued directly on the stream */
 #define PK_BATCH_PER_BLOCK 2   /* one launch per block, sweep and fluid, same tile shapes */
 
@@ -270,7 +270,7 @@ int pk_run_all(int32_t mode, int32_t nsteps, double *t_out, double *dt_out);
 /* ---- ensembles of independent instances (no counterpart in the reference) -- */
 /* The registered blocks (ascending cg_id; pk_ensemble_ids lists them) as
  * independent problems: each takes its own time_step (its own dt, caps, ch
- * and GLM damping), all advanced by the same persistent launches as the list
+ * and GLM damping), all advanced by the same launches as the list
  * entry points.  Arrays below have one entry per block in that order. */
 int pk_ensemble_ids(int64_t *ids, int32_t n);
 /* One main-loop iteration of every block; first != 0: no growth cap (the
@@ -284,7 +284,7 @@ int pk_ensemble_state_load(int32_t slot);
 /* one step of every block with the given dts, keeping the state before each
  * sweep in slots slot0, slot0+1, ... */
 int pk_ensemble_record_step(const double *dts, int32_t slot0);
-/* the recorded step of every block in reverse (one persistent adjoint launch
+/* the recorded step of every block in reverse (one adjoint launch
  * per sweep); dt_bar[i] += dL/d(dt_i), the dependence of ch on dt included */
 int pk_ensemble_step_adjoint(const double *dts, int32_t slot0, double *dt_bar);
 /* lam_i += dt_bar[i] * d(dt_i)/du_i at the state in slot (timestep_fluid) */
@@ -365,7 +365,7 @@ int pk_run_unsplit(int64_t cg_id, double tend, int32_t nmax, double *t_out, int3
  * overrides the tuned one. */
 int pk_autotune(int64_t cg_id, double dt, double chspeed, int32_t tiles_out[6]);
 
-/* Tile shapes of the persistent list sweep: per direction and fluid kind the
+/* Tile shapes of the list sweep: per direction and fluid kind the
  * workgroup size (64 lanes: the stream form, one-wave workgroups walking
  * ranges of a block's pencils; 128, 256 or 512 lanes: tiles) and, per block
  * shape, the tile length (stream: iterations per item), timed on the

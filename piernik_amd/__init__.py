@@ -597,7 +597,7 @@ def fluid_update_all(dt, mode=BATCH_GRAPH):
 
 def run_all(nsteps, mode=BATCH_GRAPH):
     """nsteps main-loop iterations over every registered block with one dt;
-    returns (t, last dt).  mode: BATCH_GRAPH (persistent launches replayed
+    returns (t, last dt).  mode: BATCH_GRAPH (list launches replayed
     from a HIP graph), BATCH_PERSISTENT, or BATCH_PER_BLOCK (one launch per
     block); all give identical results."""
     t, dt = ctypes.c_double(), ctypes.c_double()

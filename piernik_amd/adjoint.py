@@ -159,8 +159,8 @@ class EnsemblePlan:
     """Independent problems, one block each, advanced together.
 
     Every instance takes its own time_step (own dt, caps, ch, damping); the
-    forward steps are the library's persistent list launches, the backward
-    pass runs the adjoint of all instances in one persistent launch per
+    forward steps are the library's list launches, the backward
+    pass runs the adjoint of all instances in one launch per
     sweep (pk_ensemble_*).  States are tuples (u, b, psi) for MHD or (u,)
     for hydro, per instance, in the reference layout (see RolloutPlan)."""
 
