@@ -1476,14 +1476,14 @@ int build_tab(LaunchTab &t, const std::vector<Block *> &blks, int d, int f, int 
                           g_stream));
     HIPCHK(pk::launch_fill_items(t.d_first, (int)blks.size(), t.d_items, g_stream));
     t.grid = list_resident(d, g_fmag[f], nt);
-    // stream: whole rounds of the workgroups the device holds, about 8 items
+    // stream: whole rounds of the workgroups the device holds, about an item
     // each, so that the workgroups in flight walk a window that moves over the
-    // list.  In one round each walks far from the others: 4096 two-fluid blocks
-    // (240000 items, 54 GB) took 308 ms a step so, 225 in rounds (223 with one
-    // item a workgroup, 226 with 4; queues 220); lists up to 12 M cells stay at
-    // one round, which starts the stream least often.
-    const long long round = 8ll * t.grid;
-    if (t.grid > 0 && t.nitems > round) t.grid *= (int)((t.nitems + round / 2) / round);
+    // list; in one round each walks far from the others.  Items of 8
+    // iterations, ms a step: 1000 two-fluid blocks 67.6 in one round, 55.7 at 8
+    // items a workgroup, 54.5 at one (queues 55.6); 200 blocks 11.0, 10.7, 10.0
+    // (10.6).
+    if (t.grid > 0 && t.nitems > (unsigned)t.grid)
+        t.grid *= (int)(((long long)t.nitems + t.grid / 2) / t.grid);
     if (t.grid > 0 && t.nitems < (unsigned)t.grid) t.grid = (int)t.nitems;
     if (t.grid <= 0) return fail(PK_EHIP, "no resident workgroups for the list sweep (nt = %d)", nt);
     HIPCHK(hipStreamSynchronize(g_stream));
