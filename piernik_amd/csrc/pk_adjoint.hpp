@@ -91,11 +91,11 @@ PK_HD void limit_vjp(int lim, double dl, double dr, double dqb, double &dlb, dou
     if (lim == LIM_VANLEER) {
         const double dcen = dl * dr;
         if (dcen > 0.0) {
-            // 2*dl*dr/(dl+dr)
-            const double rs = nrcp(dl + dr);
-            const double g = dqb * (rs * rs);
-            dlb = g * (2.0 * dr * dr);
-            drb = g * (2.0 * dl * dl);
+            // 2*dl*dr/(dl+dr); the quotients are at most 1 each, where the square
+            // of the reciprocal overflows for slopes below 1e-154
+            const double rs = nrcp(dl + dr), x = dr * rs, y = dl * rs, g = 2.0 * dqb;
+            dlb = g * (x * x);
+            drb = g * (y * y);
         }
         return;
     }

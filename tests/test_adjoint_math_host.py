@@ -85,6 +85,27 @@ def test_limiter_vjp(hm, lim):
         assert close(out, fd_vjp(f, np.array([dl, dr]), np.array([1.0]))), (lim, dl, dr, out)
 
 
+def test_vanleer_vjp_ends_of_the_range(hm):
+    """d/d(dl) of 2*dl*dr/(dl+dr) is 2*(dr/(dl+dr))**2 <= 2 whatever the size
+    of the slopes, wherever dl*dr > 0: checked against exact fractions, down
+    to slopes whose square underflows and up to ones whose square overflows.
+    Two quotients, a square and a product: within 8 roundings."""
+    from fractions import Fraction
+
+    out = np.zeros(2)
+    for scale in (1e-161, 1e-160, 1e-158, 1e-155, 1e-154, 1e-150, 1e-100, 1.0, 1e100, 1e154, 1e300):
+        for ratio in (1.0, 0.5, 2.0, 0.3):
+            for sign in (1.0, -1.0):
+                dl, dr = sign * scale, sign * scale * ratio
+                if not dl * dr > 0.0:
+                    continue
+                s = Fraction(dl) + Fraction(dr)
+                for dqb in (0.0, 1e-3, 1.0, -7.5):
+                    hm.hm_limit_vjp(0, dl, dr, dqb, dp(out))
+                    ref = [float(2 * Fraction(dqb) * (Fraction(x) / s) ** 2) for x in (dr, dl)]
+                    assert np.all(np.abs(out - ref) <= 8 * 2.0 ** -53 * np.abs(ref)), (dl, dr, dqb, out, ref)
+
+
 def hllc(hm, l, r):
     f = np.zeros((1, 5), order="F")
     hm.hm_hllc(1, dp(np.asfortranarray(l.reshape(1, 5))), dp(np.asfortranarray(r.reshape(1, 5))), GAM, dp(f))
