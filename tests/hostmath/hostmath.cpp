@@ -22,6 +22,11 @@ double hm_mass_sum(int n, const double *x)
     return pk::mass_value(acc);
 }
 
+// the reverse mode's division and square root
+double hm_nrcp(double b) { return pk::nrcp(b); }
+double hm_ndiv(double a, double b) { return pk::ndiv(a, b, pk::nrcp(b)); }
+double hm_nsqrt(double x) { return pk::nsqrt(x); }
+
 double hm_limit(int lim, double dl, double dr) { return pk::limit(lim, dl, dr); }
 
 // u: (m, 5) or (m, 9) column-major conserved states -> q (same shape)

@@ -32,6 +32,9 @@ def load():
     L.hm_spacing.restype = d
     L.hm_mass_sum.argtypes = [i, P]
     L.hm_mass_sum.restype = d
+    for f, n in ((L.hm_nrcp, 1), (L.hm_ndiv, 2), (L.hm_nsqrt, 1)):
+        f.argtypes = [d] * n
+        f.restype = d
     L.hm_limit.argtypes = [i, d, d]
     L.hm_limit.restype = d
     L.hm_prim.argtypes = [i, i, d, P, P]

@@ -106,6 +106,41 @@ def test_vanleer_vjp_ends_of_the_range(hm):
                     assert np.all(np.abs(out - ref) <= 8 * 2.0 ** -53 * np.abs(ref)), (dl, dr, dqb, out, ref)
 
 
+ENDS = [0.0, 5e-324, 1e-310, 2.0 ** -1024, 2.0 ** -1022, 1e-300, 1e-200, 0.3, 1.0, 7.0, 1e200, 1e300, 2.0 ** 1023,
+        np.finfo(np.float64).max, np.inf]
+
+
+def test_reverse_mode_division_and_sqrt_at_the_ends_of_the_range(hm):
+    """The reverse mode's reciprocal, division and square root (their steps,
+    from rounded starting values): a division's results for zeros, infinities
+    and NaN, the same bits where nothing leaves the normal range, within two
+    units of the last place where a residual does, and NaN where the quotient of
+    finite numbers or the divisor's reciprocal overflows."""
+    same = lambda x, y: (np.isnan(x) and np.isnan(y)) or x == y
+    ulp = lambda x: 2.0 ** -1074 if x == 0.0 else np.spacing(abs(x))
+    values = ENDS + [-x for x in ENDS] + [np.nan]
+    with np.errstate(all="ignore"):
+        for b in values:
+            one = np.float64(1.0) / np.float64(b)
+            r = hm.hm_nrcp(b)
+            over = b != 0.0 and np.isinf(one)
+            assert np.isnan(r) if over else (same(r, one) or abs(r - one) <= ulp(one)), (b, r, one)
+            for a in values:
+                q = hm.hm_ndiv(a, b)
+                ref = np.float64(a) / np.float64(b)
+                if b != 0.0 and np.isfinite(a) and a != 0.0 and (over or np.isinf(ref)):
+                    ref = np.float64(np.nan)
+                near = (0.0 < abs(a) < 2.0 ** -960) or abs(ref) < 2.0 ** -960 or abs(b) > 2.0 ** 1020
+                assert same(q, ref) or (near and abs(q - ref) <= 2 * ulp(ref)), (a, b, q, ref)
+        for x in values:
+            got, ref = hm.hm_nsqrt(x), np.sqrt(np.float64(x))
+            assert same(got, ref) or (0.0 < x < 2.0 ** -767 and abs(got - ref) <= ulp(ref)), (x, got, ref)
+            assert x != 0.0 or np.signbit(got) == np.signbit(x)
+        rng = np.random.default_rng(0)
+        for a, b in rng.normal(0, 1, (2000, 2)) * 10.0 ** rng.uniform(-140, 140, (2000, 2)):
+            assert hm.hm_ndiv(a, b) == a / b and hm.hm_nsqrt(abs(a)) == np.sqrt(abs(a))
+
+
 def hllc(hm, l, r):
     f = np.zeros((1, 5), order="F")
     hm.hm_hllc(1, dp(np.asfortranarray(l.reshape(1, 5))), dp(np.asfortranarray(r.reshape(1, 5))), GAM, dp(f))
