@@ -733,6 +733,19 @@ int do_fill(Block *b)
     return PK_OK;
 }
 
+// The way out of a stepping call, its return code passed through: ghosts that
+// the sweeps left old are refreshed whether the call succeeded or not, and a
+// failed call keeps its message.
+int settle_block(Block *b, int rc)
+{
+    if (!b->ghosts_stale) return rc;
+    const std::string msg = g_err;
+    const int rf = do_fill(b);
+    if (!rc) return rf;
+    g_err = msg;
+    return rc;
+}
+
 // timestep_fluid of every fluid of one block, min over fluids; with
 // cfl > 0 the min commutes with the multiplication by cfl, so one combined
 // reduction over all fluids' cells gives the same dt.
@@ -2874,9 +2887,7 @@ int pk_fluid_update(int64_t cg_id, double dt)
     RCCHK(solo(b));
     if (!(dt > 0.0)) return fail(PK_EINVAL, "dt must be positive");
     list_touch();
-    RCCHK(do_fluid_update(b, dt, false));
-    if (b->ghosts_stale) RCCHK(do_fill(b));
-    return PK_OK;
+    return settle_block(b, do_fluid_update(b, dt, false));
 }
 
 int pk_run(int64_t cg_id, int32_t nsteps, double *t_out, double *dt_out)
@@ -2886,15 +2897,16 @@ int pk_run(int64_t cg_id, int32_t nsteps, double *t_out, double *dt_out)
     RCCHK(solo(b));
     if (nsteps < 0) return fail(PK_EINVAL, "nsteps < 0");
     list_touch();
-    // the RK2 sweeps read the periodic interior; the ghosts are refreshed after the steps
-    if (nsteps == 0 || g_cfg.integration_order != 2) RCCHK(do_fill(b));
+    // the RK2 sweeps read the periodic interior; the ghosts are refreshed on the way out
+    if (g_cfg.integration_order == 2)
+        b->ghosts_stale = true;
+    else
+        RCCHK(do_fill(b));
     StepLoop L;
     L.blocks = {b};
     L.timestep = [b](double *dt, double *c) { return do_timestep(b, dt, c); };
     L.update = [b](double dt) { return do_fluid_update(b, dt, true); };
-    RCCHK(run_loop(L, nsteps, t_out, dt_out, &g_last_redone));
-    if (b->ghosts_stale) RCCHK(do_fill(b));
-    return PK_OK;
+    return settle_block(b, run_loop(L, nsteps, t_out, dt_out, &g_last_redone));
 }
 
 int pk_set_cfl_control(int32_t mode, double cfl_max, double dt_shrink, int32_t max_attempts,
@@ -2954,9 +2966,7 @@ int pk_fluid_update_unsplit(int64_t cg_id, double dt)
     if (!(dt > 0.0)) return fail(PK_EINVAL, "dt must be positive");
     RCCHK(solo(b));
     list_touch();
-    RCCHK(fluid_update_unsplit(b, dt, false));
-    if (b->ghosts_stale) RCCHK(do_fill(b));
-    return PK_OK;
+    return settle_block(b, fluid_update_unsplit(b, dt, false));
 }
 
 int pk_run_unsplit(int64_t cg_id, double tend, int32_t nmax, double *t_out, int32_t *nsteps_out)
@@ -2967,11 +2977,11 @@ int pk_run_unsplit(int64_t cg_id, double tend, int32_t nmax, double *t_out, int3
     if (nmax < 0) return fail(PK_EINVAL, "nmax < 0");
     list_touch();
     double t = 0.0, dt = -1.0, dt_old = -1.0;
-    int s = 0;
+    int s = 0, rc = PK_OK;
     RCCHK(do_fill(b));
     while (t < tend && s < nmax) {
         double c;
-        RCCHK(do_timestep(b, &dt, &c));
+        if ((rc = do_timestep(b, &dt, &c))) break;
         // time_step caps (timestep.F90:198-207), then the unsplit clamp to tend (:221-222)
         if (s >= 1 && dt_old > 0.0) {
             const double cap = dt_old * 2.0;
@@ -2980,12 +2990,12 @@ int pk_run_unsplit(int64_t cg_id, double tend, int32_t nmax, double *t_out, int3
         const double rem = tend - t;
         const double cl = rem + (2.0 * DBL_EPSILON) * rem;
         if (cl < dt) dt = cl;
-        RCCHK(fluid_update_unsplit(b, dt, true));
+        if ((rc = fluid_update_unsplit(b, dt, true))) break;
         t = t + dt;
         dt_old = dt;
         s++;
     }
-    if (b->ghosts_stale) RCCHK(do_fill(b));
+    RCCHK(settle_block(b, rc));
     HIPCHK(hipStreamSynchronize(g_stream));
     if (t_out) *t_out = t;
     if (nsteps_out) *nsteps_out = s;
@@ -3163,7 +3173,15 @@ int pk_run_all(int32_t mode, int32_t nsteps, double *t_out, double *dt_out)
     L.blocks = g_list.blocks;
     L.timestep = [](double *dt, double *c) { return list_dt(dt, c); };
     L.update = [mode](double dt) { return list_step(mode, dt); };
-    return run_loop(L, nsteps, t_out, dt_out, &g_last_redone);  // ghosts left old are refilled when read
+    const int rc = run_loop(L, nsteps, t_out, dt_out, &g_last_redone);
+    if (rc && !g_list.fresh && !g_list.filled) {
+        // a call that fails before its first step leaves refreshed ghosts (a
+        // step's are refilled when read)
+        const std::string msg = g_err;
+        (void)list_fill();
+        g_err = msg;
+    }
+    return rc;
 }
 
 int pk_autotune_all(double dt, double chspeed)
