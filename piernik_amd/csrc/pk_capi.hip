@@ -1765,8 +1765,7 @@ int list_set_wrap(int d, int wrap)
 // launches the single-block sweep once per block with the same tile shapes
 // (for items of the stream form, the block's single-block shape); the
 // list modes launch the list sweep once per sweep and fluid.
-// given: the first sweep reads the ghosts as they are (not in a captured step).
-int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false, bool given = false)
+int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
 {
     const std::vector<SweepStep> sw = step_sweeps();
     const bool persistent = mode != PK_BATCH_PER_BLOCK;
@@ -1777,7 +1776,6 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false, bool giv
         const int d = sw[k].d;
         const int parity = (int)(k % 2);
         if (g_list.linked && !ens) RCCHK(exchange(d, parity));
-        if (given && k == 0) RCCHK(list_set_wrap(d, 0));
         for (int f = 0; f < g_nfl; f++) {
             for (LaunchTab *tp : {&g_list.tab[d][f], &g_list.stab[d][f]}) {
                 LaunchTab &t = *tp;
@@ -1829,7 +1827,6 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false, bool giv
                 }
             }
         }
-        if (given && k == 0) RCCHK(list_set_wrap(d, 1));
     }
     if (ens)
         HIPCHK(pk::launch_dtslots_final(g_ens.d_dtslots, kEnsSlots, (int)g_ens.nblk, g_ens.dtout, g_stream));
@@ -3646,13 +3643,12 @@ int pk_ensemble_step(int32_t mode, int32_t first, double *dt_out, int32_t *cappe
         g_ens.dt_old[i] = dt[i];
     }
     RCCHK(ens_set_step(dt.data()));
-    const bool given = !g_list.wrap_stale;  // ghosts a caller may have set: the first sweep reads them
-    if (mode == PK_BATCH_GRAPH && !given) {
+    if (mode == PK_BATCH_GRAPH) {
         RCCHK(ens_graph());
         HIPCHK(hipGraphLaunch(g_ens.exec, g_stream));
     } else {
         pk::StepScalars sc{};
-        RCCHK(enqueue_step(mode == PK_BATCH_GRAPH ? PK_BATCH_PERSISTENT : mode, sc, true, given));
+        RCCHK(enqueue_step(mode, sc, true));
     }
     for (Block *b : g_list.blocks) {
         b->uh = -1;

@@ -109,9 +109,11 @@ def test_step_reads_the_ghosts_it_is_given(n):
 
 
 @pytest.mark.parametrize("mode", [pk.BATCH_GRAPH, pk.BATCH_PERSISTENT, pk.BATCH_PER_BLOCK])
-def test_ensemble_step_reads_the_ghosts_it_is_given(mode):
-    """As above for an ensemble of one: its steps equal fluid_update's with
-    the same dt, from ghosts that are not periodic images and after."""
+def test_ensemble_steps_refresh_the_ghosts(mode):
+    """An ensemble's steps take each block as periodic, whatever its ghosts
+    hold: an ensemble of one from ghosts that are not periodic images equals
+    fluid_update with the same dt from refreshed ones, at the first step and
+    after it."""
     cfg = pk.Config(limiter="vanleer", smalld=1e-3, smallei=1e-4)
     out, dts = [], []
     for ens in (True, False):
@@ -121,6 +123,8 @@ def test_ensemble_step_reads_the_ghosts_it_is_given(mode):
         cg = setups.smooth_random((12, 9, 8), nb=4, seed=7, gamma=cfg.gamma)
         cg.u[:, :4] *= 1.25
         cg.upload()
+        if not ens:
+            pk.update_boundaries(cg)
         for s in range(2):
             if ens:
                 dt, cap = (ctypes.c_double * 1)(), (ctypes.c_int32 * 1)()
