@@ -1746,21 +1746,6 @@ std::vector<SweepStep> step_sweeps()
     return v;
 }
 
-// Makes the tables of the sweeps along d read ghosts as they are (wrap 0) or
-// their pre-images (1, as built).
-int list_set_wrap(int d, int wrap)
-{
-    for (int f = 0; f < g_nfl; f++)
-        for (LaunchTab *t : {&g_list.tab[d][f], &g_list.stab[d][f]}) {
-            if (t->nitems == 0) continue;
-            for (pk::SweepArgs &a : t->h_args) a.wrap = wrap;
-            HIPCHK(hipMemcpyAsync(t->d_args, t->h_args.data(), sizeof(pk::SweepArgs) * t->h_args.size(),
-                                  hipMemcpyHostToDevice, g_stream));
-        }
-    HIPCHK(hipStreamSynchronize(g_stream));
-    return PK_OK;
-}
-
 // Enqueue the launches of one step on g_stream.  mode PK_BATCH_PER_BLOCK
 // launches the single-block sweep once per block with the same tile shapes
 // (for items of the stream form, the block's single-block shape); the
@@ -1771,7 +1756,6 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
     const bool persistent = mode != PK_BATCH_PER_BLOCK;
     unsigned long long *slots = ens ? g_ens.d_dtslots : g_list.d_dtslots;
     const int nslots = ens ? kEnsSlots : kDtSlots;
-    int q = 0;
     for (size_t k = 0; k < sw.size(); k++) {
         const int d = sw[k].d;
         const int parity = (int)(k % 2);
@@ -1986,15 +1970,24 @@ int ens_set_step(const double *dts)
     return PK_OK;
 }
 
+// every block has the slots slot0 .. slot0 + n - 1
+int ens_check_slots(int slot0, int n)
+{
+    for (Block *b : g_list.blocks)
+        for (int slot = slot0; slot < slot0 + n; slot++)
+            if (b->lam[0] == nullptr || slot < 0 || slot >= (int)b->slots.size())
+                return fail(PK_EINVAL, "block %lld has no slot %d (pk_adjoint_setup)", (long long)b->id, slot);
+    return PK_OK;
+}
+
 // every block's current buffer <-> its slot; parity 1: the data sits in the
 // block's other buffer (between the sweeps of a step)
 int ens_copy_slots(int slot, bool save, int parity = 0)
 {
+    RCCHK(ens_check_slots(slot, 1));
     bool stale = false;
     for (size_t i = 0; i < g_ens.nblk; i++) {
         Block *b = g_list.blocks[i];
-        if (b->lam[0] == nullptr || slot < 0 || slot >= (int)b->slots.size())
-            return fail(PK_EINVAL, "block %lld has no slot %d (pk_adjoint_setup)", (long long)b->id, slot);
         pk::CopyJob j{};
         j.src = save ? b->buf[b->cur ^ parity] : b->slots[slot];
         j.dst = save ? b->slots[slot] : b->buf[b->cur ^ parity];
@@ -3710,12 +3703,12 @@ int pk_ensemble_record_step(const double *dts, int32_t slot0)
     RCCHK(ens_build());
     std::vector<bool> damp;
     const std::vector<int> dirs = step_dirs(&damp);
+    RCCHK(ens_check_slots(slot0, (int)dirs.size()));
     RCCHK(ens_set_step(dts));
     for (size_t k = 0; k < dirs.size(); k++) {
         RCCHK(ens_copy_slots(slot0 + (int)k, true, (int)(k % 2)));
         const int d = dirs[k];
         const bool given = !g_list.wrap_stale;  // the first sweep of a state whose ghosts are current
-        if (given) RCCHK(list_set_wrap(d, 0));
         for (int f = 0; f < g_nfl; f++) {
             for (int part = 0; part < 2; part++) {
                 LaunchTab &t = part ? g_list.stab[d][f] : g_list.tab[d][f];
@@ -3727,6 +3720,7 @@ int pk_ensemble_record_step(const double *dts, int32_t slot0)
                 L.nitems = t.nitems;
                 L.parity = (int)(k % 2);
                 L.apply_fac = damp[k] && g_fmag[f];
+                L.given = given;
                 L.step = g_ens.d_step;
                 L.dtslots = nullptr;
                 L.nslots = kEnsSlots;
@@ -3735,7 +3729,6 @@ int pk_ensemble_record_step(const double *dts, int32_t slot0)
                 HIPCHK(list_kernel(d, g_fmag[f], L, t.nt, t.grid));
             }
         }
-        if (given) RCCHK(list_set_wrap(d, 1));
         g_list.wrap_stale = true;  // from here on: the later slots' ghosts are old too
     }
     list_touch();

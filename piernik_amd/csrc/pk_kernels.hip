@@ -431,6 +431,7 @@ __device__ __forceinline__ unsigned load_list_args(const ListArgs &L, unsigned i
     }
     const unsigned first = ((cu32 *)L.first)[blk];
     next = ((cu32 *)L.first)[blk + 1];
+    if (L.given) a.wrap = 0;
     if (L.parity) {
         const double *s0 = a.src;
         a.src = a.dst;

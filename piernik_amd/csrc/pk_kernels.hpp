@@ -174,6 +174,7 @@ struct ListArgs {
     unsigned item0;          // first item of the launch
     int parity;              // 1: read buffer 1, write buffer 0
     int apply_fac;           // multiply psi by step->psi_fac
+    int given;               // 1: the ghosts are read as they are, whatever the blocks' wrap
     const StepScalars *step;      // one for the whole list, or one per block (per_block)
     unsigned long long *dtslots;  // if set: fold timestep_fluid of the cells written into these slots
     int nslots;                   // slots (per block when per_block)
