@@ -662,6 +662,14 @@ int do_stage(Block *b, int ddim, int istep, double dt, double ch)
     return PK_OK;
 }
 
+// Timestep slots are clean between steps: launch_dtslots_final leaves them so,
+// and this does after a step that failed (rc) before it.
+int clean_slots(int rc, unsigned long long *slots, int nslots)
+{
+    if (rc) (void)pk::launch_dtslots_init(slots, nslots, g_stream);
+    return rc;
+}
+
 // One directional sweep, both RK2 stages, every fluid.  wrap: the block is
 // periodic on itself and the sweep reads its interior in place of the ghosts,
 // which it leaves old (b->ghosts_stale); want_dt: reduce the next step's
@@ -693,7 +701,8 @@ int do_sweep(Block *b, int ddim, double dt, double ch, double psi_fac, bool wrap
         a.dst = dst ? dst + b->xo + (long long)g_fplane[f] * b->sv : fluid_state(b, 1 - b->cur, f);
         a.wrap = wrap ? 1 : 0;
         a.dtslots = want_dt ? b->d_dtslots : nullptr;
-        RCCHK(launch(ddim, true, a, b, f));
+        const int rc = launch(ddim, true, a, b, f);
+        if (rc) return want_dt ? clean_slots(rc, b->d_dtslots, kDtSlots) : rc;
     }
     if (src || dst) return PK_OK;
     if (wrap) b->ghosts_stale = true;
@@ -1819,6 +1828,8 @@ int enqueue_step(int mode, const pk::StepScalars &sc, bool ens = false)
     return PK_OK;
 }
 
+int ens_graph();
+
 int ensure_graph()
 {
     if (g_list.exec) return PK_OK;
@@ -1859,6 +1870,15 @@ int list_dt(double *dt_out, double *c_out)
     return list_prepare(dt_out, c_out);
 }
 
+// One step of the list or the ensemble: the captured launches or the launches.
+int run_step(int mode, const pk::StepScalars &sc, bool ens)
+{
+    if (mode != PK_BATCH_GRAPH) return enqueue_step(mode, sc, ens);
+    RCCHK(ens ? ens_graph() : ensure_graph());
+    HIPCHK(hipGraphLaunch(ens ? g_ens.exec : g_list.exec, g_stream));
+    return PK_OK;
+}
+
 int list_step(int mode, double dt)
 {
     pk::StepScalars sc{};
@@ -1870,21 +1890,16 @@ int list_step(int mode, double dt)
     HIPCHK(hipStreamSynchronize(g_stream));
     *g_list.h_step = sc;
     HIPCHK(hipMemcpyAsync(g_list.d_step, g_list.h_step, sizeof sc, hipMemcpyHostToDevice, g_stream));
-    if (mode == PK_BATCH_GRAPH) {
-        RCCHK(ensure_graph());
-        HIPCHK(hipGraphLaunch(g_list.exec, g_stream));
-    } else {
-        RCCHK(enqueue_step(mode, sc));
-    }
+    // from here on, whether or not every launch succeeds
+    list_touch();
+    g_list.ghosts_stale = g_list.linked;
+    if (!g_list.linked) g_list.wrap_stale = true;
     for (Block *b : g_list.blocks) {
         b->uh = -1;
         b->dt_pending = false;
     }
+    RCCHK(clean_slots(run_step(mode, sc, false), g_list.d_dtslots, kDtSlots));
     g_list.fresh = true;
-    g_list.filled = false;
-    g_list.ghosts_stale = g_list.linked;
-    if (!g_list.linked) g_list.wrap_stale = true;
-    g_ens.fresh = false;
     return PK_OK;
 }
 
@@ -3636,20 +3651,13 @@ int pk_ensemble_step(int32_t mode, int32_t first, double *dt_out, int32_t *cappe
         g_ens.dt_old[i] = dt[i];
     }
     RCCHK(ens_set_step(dt.data()));
-    if (mode == PK_BATCH_GRAPH) {
-        RCCHK(ens_graph());
-        HIPCHK(hipGraphLaunch(g_ens.exec, g_stream));
-    } else {
-        pk::StepScalars sc{};
-        RCCHK(enqueue_step(mode, sc, true));
-    }
+    list_touch();
+    g_list.wrap_stale = true;
     for (Block *b : g_list.blocks) {
         b->uh = -1;
         b->dt_pending = false;
     }
-    g_list.fresh = false;
-    g_list.filled = false;
-    g_list.wrap_stale = true;
+    RCCHK(clean_slots(run_step(mode, pk::StepScalars{}, true), g_ens.d_dtslots, kEnsSlots * (int)g_ens.nblk));
     g_ens.fresh = true;
     return PK_OK;
 }
