@@ -299,12 +299,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
     }
     // last, a.last and a.dtslots are the same for every lane: the whole wave takes part
     if (last && a.last) pk::mass_add(a.dmass, dmass);
+#if !PK_RELAXED
     if (last && a.dtslots) {  // timestep_fluid of the cells of the finished state
         const double huge = 1.7976931348623157e308;
         double mn[3] = {huge, huge, huge}, cmax = 0.0;
         if (upd) dt_cell<0, P>(a, T, mn, cmax);
         dt_reduce(a, mn, cmax, blockIdx.x);
     }
+#endif
     if (upd && flags) atomicOr(a.flags, flags);
 }
 

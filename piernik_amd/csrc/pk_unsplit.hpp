@@ -21,7 +21,7 @@ struct UnsplitArgs {
     // fused passes only:
     int wrap;            // 1: src's ghosts are read from their pre-images (a block periodic on itself)
     double src_fac, base_fac;  // psi of src and of base times these when read (glmdamping before the stages)
-    unsigned long long *dtslots;  // if set: the last direction's pass folds timestep_fluid of the finished
+    unsigned long long *dtslots;  // if set (exact build only): the last direction's pass folds timestep_fluid of the finished
     int nslots;                   // state into these slots (as SweepArgs)
     double psi_fac;      // fused passes: psi of the finished state times this (glmdamping after the stages)
     int last;            // last stage: care_for_positives runs
