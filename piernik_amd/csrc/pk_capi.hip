@@ -1497,17 +1497,18 @@ int build_tab(LaunchTab &t, const std::vector<Block *> &blks, int d, int f, int 
     HIPCHK(hipMemcpyAsync(t.d_first, t.h_first.data(), sizeof(unsigned) * (2 * blks.size() + 1), hipMemcpyHostToDevice,
                           g_stream));
     HIPCHK(pk::launch_fill_items(t.d_first, (int)blks.size(), t.d_items, g_stream));
-    t.grid = list_resident(d, g_fmag[f], nt);
+    t.grid = list_resident(d, g_fmag[f], nt);  // (also sets the kernel's attributes, outside any capture)
+    if (t.grid <= 0) return fail(PK_EHIP, "no resident workgroups for the list sweep (nt = %d)", nt);
     // stream: whole rounds of the workgroups the device holds, about an item
     // each, so that the workgroups in flight walk a window that moves over the
     // list; in one round each walks far from the others.  Items of 8
     // iterations, ms a step: 1000 two-fluid blocks 67.6 in one round, 55.7 at 8
     // items a workgroup, 54.5 at one (queues 55.6); 200 blocks 11.0, 10.7, 10.0
     // (10.6).
-    if (t.grid > 0 && t.nitems > (unsigned)t.grid)
-        t.grid *= (int)(((long long)t.nitems + t.grid / 2) / t.grid);
-    if (t.grid > 0 && t.nitems < (unsigned)t.grid) t.grid = (int)t.nitems;
-    if (t.grid <= 0) return fail(PK_EHIP, "no resident workgroups for the list sweep (nt = %d)", nt);
+    if (nt == pk::kStreamListNt) {
+        const long long g = t.grid, rounds = std::max(1ll, (t.nitems + g / 2) / g);
+        t.grid = (int)std::min({g * std::min(rounds, std::max(1ll, pk::kListPiece / g)), (long long)t.nitems});
+    }
     HIPCHK(hipStreamSynchronize(g_stream));
     return PK_OK;
 }
