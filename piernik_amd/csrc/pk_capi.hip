@@ -3223,8 +3223,29 @@ int pk_autotune_all(double dt, double chspeed)
     // the stream form stores through buffer ranges of 24 sv bytes: every block's planes must fit
     bool streams_fit = true;
     for (Block *b : g_list.blocks) streams_fit = streams_fit && pk::stream_stores_fit(b->sv);
-    LaunchTab tmp;
+    LaunchTab tmp, tmp2;
     int rc = PK_OK;
+    // ms of a launch of each table (the second may be empty): a warm-up, then timed
+    auto time_tabs = [&](int d, int f, LaunchTab *const (&tabs)[2], float &ms) -> int {
+        for (int rep = 0; rep < 2; rep++) {
+            HIPCHK(hipEventRecord(e0, g_stream));
+            for (LaunchTab *t : tabs) {
+                if (t->nitems == 0) continue;
+                pk::ListArgs L{};
+                L.args = t->d_args;
+                L.first = t->d_first;
+                L.items = t->d_items;
+                L.nitems = t->nitems;
+                L.step = g_list.d_step;
+                L.nslots = kDtSlots;
+                HIPCHK(list_kernel(d, g_fmag[f], L, t->nt, t->grid));
+            }
+            HIPCHK(hipEventRecord(e1, g_stream));
+            HIPCHK(hipEventSynchronize(e1));
+            HIPCHK(hipEventElapsedTime(&ms, e0, e1));
+        }
+        return PK_OK;
+    };
     const int nt_list[] = {pk::kStreamListNt, 128, 256, 512};
     for (int d = 0; d < 3 && !rc; d++) {
         if (!g_cfg.has_dir[d]) continue;
@@ -3251,24 +3272,9 @@ int pk_autotune_all(double dt, double chspeed)
                     for (int ts : cand) {
                         std::vector<int> tsv(cl.second.size(), ts);
                         if ((rc = build_tab(tmp, cl.second, d, f, nt, &tsv))) break;
-                        pk::ListArgs L{};
-                        L.args = tmp.d_args;
-                        L.first = tmp.d_first;
-                        L.items = tmp.d_items;
-                        L.nitems = tmp.nitems;
-                        L.parity = 0;
-                        L.apply_fac = 0;
-                        L.step = g_list.d_step;
-                        L.dtslots = nullptr;
-                        L.nslots = kDtSlots;
+                        tmp2.nitems = 0;
                         float ms = 0.0f;
-                        for (int rep = 0; rep < 2; rep++) {  // warm-up, then timed
-                            HIPCHK(hipEventRecord(e0, g_stream));
-                            HIPCHK(list_kernel(d, g_fmag[f], L, nt, tmp.grid));
-                            HIPCHK(hipEventRecord(e1, g_stream));
-                            HIPCHK(hipEventSynchronize(e1));
-                            HIPCHK(hipEventElapsedTime(&ms, e0, e1));
-                        }
+                        if ((rc = time_tabs(d, f, {&tmp, &tmp2}, ms))) break;
                         if (ms < best) {
                             best = ms;
                             best_ts = ts;
@@ -3310,6 +3316,47 @@ int pk_autotune_all(double dt, double chspeed)
                     }
                 }
             }
+            // A shape's time alone counts the drain of a short launch, which the
+            // list pays once: the choice is checked over the whole list against
+            // the stream form for every block and against its own workgroup size
+            // unsplit (4096 two-fluid blocks: 221 ms a step as chosen from the
+            // times alone, 220 checked, 215 in streams of 8 iterations throughout).
+            {
+                const std::pair<int, bool> choices[3] = {{best_nt, best_split}, {pk::kStreamListNt, false}, {best_nt, false}};
+                float best_ms = 1e30f;
+                for (int c = 0; c < 3; c++) {
+                    const int nt = choices[c].first;
+                    const bool sp = choices[c].second;
+                    if (c && std::find(choices, choices + c, choices[c]) != choices + c) continue;
+                    std::vector<Block *> main, str;
+                    std::vector<int> main_ts, str_ts;
+                    bool ok = true;
+                    for (Block *b : g_list.blocks) {
+                        auto &tm = timed[{b->n[0], b->n[1], b->n[2]}];
+                        const auto it = tm.find(nt), is = tm.find(pk::kStreamListNt);
+                        const bool s = sp && is != tm.end() && (it == tm.end() || is->second.second < it->second.second);
+                        const auto use = s ? is : it;
+                        if (use == tm.end()) {
+                            ok = false;
+                            break;
+                        }
+                        (s ? str : main).push_back(b);
+                        (s ? str_ts : main_ts).push_back(use->second.first);
+                    }
+                    if (!ok) continue;
+                    float ms = 0.0f;
+                    if ((rc = build_tab(tmp, main, d, f, nt, &main_ts)) ||
+                        (rc = build_tab(tmp2, str, d, f, pk::kStreamListNt, &str_ts)) ||
+                        (rc = time_tabs(d, f, {&tmp, &tmp2}, ms)))
+                        break;
+                    if (ms < best_ms) {
+                        best_ms = ms;
+                        best_nt = nt;
+                        best_split = sp;
+                    }
+                }
+            }
+            if (rc) break;
             g_list.nt_pref[d][g_fmag[f]] = best_nt;
             g_list.ts_force[d][g_fmag[f]] = 0;
             g_list.split_cls[d][g_fmag[f]].clear();
@@ -3332,6 +3379,7 @@ int pk_autotune_all(double dt, double chspeed)
         }
     }
     free_tab(tmp);
+    free_tab(tmp2);
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
     if (rc) return rc;
