@@ -146,14 +146,20 @@ PK_HD void limit_vjp(int lim, double dl, double dr, double dqb, double &dlb, dou
 // side the contact speed points to -- and the average of the two sides when
 // sm == 0.  The reverse pass is written once, for side A = the selected side
 // and side O = the other one, with sg = +1 when A is the left side; the two
-// sides' formulas are mirror images.  The averaged case runs it twice with
-// weight 1/2 (it is linear in the flux adjoint given the branch).
+// sides' formulas are mirror images.  In the averaged case O's own part runs
+// too, both with weight 1/2 (the pass is linear in the flux adjoint given the
+// branch).
 
 // The flux of side A and its reverse, shared by both solvers: with
 // dn = q0*(s - q1) and ds = dn/(s - sm) the side's star flux F + s*(U* - U) is
 //   [s*ds - dn, pt - dn*q1 + s*ds*sm, s*ds*vy - dn*q2, s*ds*vz - dn*q3,
 //    pt*q1 - x*en + s*us4], x = s - q1
 // (B terms apart), which needs neither F nor U.
+
+// Adjoints of what a side's star flux takes from the interface.
+struct HllcSide {
+    double ssm, x, p, prt, sm, dn, s;
+};
 
 // f = flux_hllc(l, r); given fb, add dL/dl to lb and dL/dr to rb.
 // rg1 = 1/(gam - 1).
@@ -194,115 +200,102 @@ PK_HD void hllc_vjp_r(const double *l, const double *r, double gam, double rg1, 
     const double sm = degen ? (sl + sr) / 2.0
                             : ndiv((auxr * r[1] - r[4]) - (auxl * l[1] - l[4]), auxr - auxl, rden);
     const double prt = 0.5 * ((l[4] + auxl * (sm - l[1])) + (r[4] + auxr * (sm - r[1])));
-    const bool both = sm == 0.0;
-    bool left = sm > 0.0;
+    const bool both = sm == 0.0, left = sm > 0.0;
     const double w = both ? 0.5 : 1.0;
     double a[5], o[5], ab[5], ob[5];
-    volatile double first[10];  // the first pass of an averaged interface (rare: kept out of registers)
 #pragma unroll
     for (int v = 0; v < 5; v++) {
         a[v] = left ? l[v] : r[v];
         o[v] = left ? r[v] : l[v];
     }
-    double s = left ? sl : sr, so = left ? sr : sl;
-    double ca2 = left ? cl2 : cr2, co2 = left ? cr2 : cl2;
-    double rdo = left ? rden : -rden;  // 1/(dno - dn)
-    for (int pass = 0;; pass++) {
-        const double x = s - a[1], xo = so - o[1];
-        const double dn = a[0] * x, dno = o[0] * xo;
-        const double K = (a[1] * a[1] + a[2] * a[2]) + a[3] * a[3];
-        const double en = (a[4] * rg1) + (0.5 * a[0]) * K;
-        const double rs = nrcp(s - sm);
-        const double d = dn * rs;
-        const double us4 = (((x * en) - (a[4] * a[1])) + (prt * sm)) * rs;
+    const double s = left ? sl : sr, so = left ? sr : sl;
+    const double ca2 = left ? cl2 : cr2, co2 = left ? cr2 : cl2;
+    const double rdo = left ? rden : -rden;  // 1/(dno - dn)
+    const double x = s - a[1], xo = so - o[1];
+    const double dn = a[0] * x, dno = o[0] * xo;
+    // the side's own part: from the flux adjoint to those of its state and of
+    // what both sides share (x = s - q1, dn, en, prt, sm, s - sm)
+    auto side = [&](const double (&q)[5], double s_, double x_, double dn_, double (&qb)[5], HllcSide &y) {
+        const double K = (q[1] * q[1] + q[2] * q[2]) + q[3] * q[3];
+        const double en = (q[4] * rg1) + (0.5 * q[0]) * K;
+        const double rs = nrcp(s_ - sm);
+        const double d = dn_ * rs;
+        const double us4 = (((x_ * en) - (q[4] * q[1])) + (prt * sm)) * rs;
         const double g0 = w * fb[0], g1 = w * fb[1], g2 = w * fb[2], g3 = w * fb[3], g4 = w * fb[4];
-        const double sd = s * d, W = sd - dn;
-        const double Wb = (g0 + g2 * a[2]) + g3 * a[3];
+        const double sd = s_ * d, W = sd - dn_;
+        const double Wb = (g0 + g2 * q[2]) + g3 * q[3];
         const double sdb = Wb + g1 * sm;
-        const double db = sdb * s;
-        const double nb = (g4 * s) * rs;
-        const double dr = db * rs;
-        double sb = sdb * d + g4 * us4;
-        const double ssmb = -(nb * us4) - dr * d;
-        double xb = nb * en - g4 * en;
-        const double enb = nb * x - g4 * x;
+        const double nb = (g4 * s_) * rs;
+        const double dr = (sdb * s_) * rs;
+        y.ssm = -(nb * us4) - dr * d;
+        y.x = nb * en - g4 * en;
+        const double enb = nb * x_ - g4 * x_;
         const double pf = g4 - nb;  // pt*q1 - (pt*q1 in the star energy)
-        double pb = g1 + pf * a[1];
-        const double prtb = nb * sm;
-        const double h = 0.5 * prtb;
-        double smb = g1 * sd + nb * prt + h * (dn + dno) - ssmb;
-        double dnb = dr - Wb - g1 * a[1] + h * (sm - a[1]);
-        double dnob = h * (sm - o[1]);
-        const double kb = enb * a[0];
-        ab[1] = kb * a[1] - g1 * dn + pf * a[4] - h * dn;
-        ab[2] = g2 * W + kb * a[2];
-        ab[3] = g3 * W + kb * a[3];
-        ob[1] = -(h * dno);
-        pb += h;
-        double pob = h;
-        double sob = 0.0;
-        sb += ssmb;
-        // sm = ((dno*o1 - po) - (dn*a1 - pa)) / (dno - dn), or the mirror image of it
-        if (degen) {
-            sb += 0.5 * smb;
-            sob += 0.5 * smb;
-        } else {
-            const double q = smb * rdo;
-            dnob += q * (o[1] - sm);
-            dnb -= q * (a[1] - sm);
-            ob[1] += q * dno;
-            ab[1] -= q * dn;
-            pob -= q;
-            pb += q;
-        }
-        // dn = q0*x, x = s - q1
-        ab[0] = (0.5 * enb) * K + dnb * x;
-        xb += dnb * a[0];
-        ob[0] = dnob * xo;
-        const double xob = dnob * o[0];
-        sb += xb;
-        ab[1] -= xb;
-        sob += xob;
-        ob[1] -= xob;
-        ab[4] = pb + enb * rg1;
-        ob[4] = pob;
-        // sl = min(l1, r1) - c, sr = max(l1, r1) + c, c = sqrt(max(cl2, cr2))
-        const double lowb = left ? sb : sob, highb = left ? sob : sb;
-        double wa, wo;
-        dmin(a[1], o[1], wa, wo);
-        ab[1] += lowb * wa;
-        ob[1] += lowb * wo;
-        dmax(a[1], o[1], wa, wo);
-        ab[1] += highb * wa;
-        ob[1] += highb * wo;
-        const double cmb = (highb - lowb) * (0.5 * nrcp(c));
-        dmax(ca2, co2, wa, wo);
-        const double ga = (cmb * wa) * nrcp(a[0]), go = (cmb * wo) * nrcp(o[0]);
-        ab[4] += ga * gam;
-        ab[0] -= ga * ca2;
-        ob[4] += go * gam;
-        ob[0] -= go * co2;
-        ob[2] = ob[3] = 0.0;
-        if (!both || pass) break;
-        // sm == 0: once more with the sides exchanged
-        left = !left;
+        y.p = g1 + pf * q[1];
+        y.prt = nb * sm;
+        y.sm = g1 * sd + nb * prt;
+        y.dn = dr - Wb - g1 * q[1];
+        const double kb = enb * q[0];
+        qb[0] = (0.5 * enb) * K;
+        qb[1] = kb * q[1] - g1 * dn_ + pf * q[4];
+        qb[2] = g2 * W + kb * q[2];
+        qb[3] = g3 * W + kb * q[3];
+        qb[4] = enb * rg1;
+        y.s = sdb * d + g4 * us4 + y.ssm;
+    };
+    HllcSide y, yo;
+    side(a, s, x, dn, ab, y);
+    yo.ssm = yo.x = yo.p = yo.prt = yo.sm = yo.dn = yo.s = 0.0;
 #pragma unroll
-        for (int v = 0; v < 5; v++) {
-            first[v] = ab[v];
-            first[5 + v] = ob[v];
-            swap_(a[v], o[v]);
-        }
-        swap_(s, so);
-        swap_(ca2, co2);
-        rdo = -rdo;
+    for (int v = 0; v < 5; v++) ob[v] = 0.0;
+    if (both) side(o, so, xo, dno, ob, yo);
+    const double h = 0.5 * (y.prt + yo.prt);
+    const double smb = (y.sm + yo.sm) + h * (dn + dno) - y.ssm - yo.ssm;
+    double dnb = y.dn + h * (sm - a[1]), dnob = yo.dn + h * (sm - o[1]);
+    double sb = y.s, sob = yo.s;
+    ab[1] -= h * dn;
+    ob[1] -= h * dno;
+    double pb = y.p + h, pob = yo.p + h;
+    // sm = ((dno*o1 - po) - (dn*a1 - pa)) / (dno - dn), or the mirror image of it
+    if (degen) {
+        sb += 0.5 * smb;
+        sob += 0.5 * smb;
+    } else {
+        const double q = smb * rdo;
+        dnob += q * (o[1] - sm);
+        dnb -= q * (a[1] - sm);
+        ob[1] += q * dno;
+        ab[1] -= q * dn;
+        pob -= q;
+        pb += q;
     }
-    if (both) {
-#pragma unroll
-        for (int v = 0; v < 5; v++) {
-            ab[v] += first[5 + v];
-            ob[v] += first[v];
-        }
-    }
+    // dn = q0*x, x = s - q1
+    ab[0] += dnb * x;
+    const double xb = y.x + dnb * a[0];
+    ob[0] += dnob * xo;
+    const double xob = yo.x + dnob * o[0];
+    sb += xb;
+    ab[1] -= xb;
+    sob += xob;
+    ob[1] -= xob;
+    ab[4] += pb;
+    ob[4] += pob;
+    // sl = min(l1, r1) - c, sr = max(l1, r1) + c, c = sqrt(max(cl2, cr2))
+    const double lowb = left ? sb : sob, highb = left ? sob : sb;
+    double wa, wo;
+    dmin(a[1], o[1], wa, wo);
+    ab[1] += lowb * wa;
+    ob[1] += lowb * wo;
+    dmax(a[1], o[1], wa, wo);
+    ab[1] += highb * wa;
+    ob[1] += highb * wo;
+    const double cmb = (highb - lowb) * (0.5 * nrcp(c));
+    dmax(ca2, co2, wa, wo);
+    const double ga = (cmb * wa) * nrcp(a[0]), go = (cmb * wo) * nrcp(o[0]);
+    ab[4] += ga * gam;
+    ab[0] -= ga * ca2;
+    ob[4] += go * gam;
+    ob[0] -= go * co2;
 #pragma unroll
     for (int v = 0; v < 5; v++) {
         lb[v] += left ? ab[v] : ob[v];
