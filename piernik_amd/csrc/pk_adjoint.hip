@@ -426,10 +426,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2))) void k
     extern __shared__ double lds[];
     // XCD-aware order, as k_sweep: tiles whose cells share cache lines (the
     // pencils of a y or z tile are a fraction of a line wide) share an L2
-    int bid = blockIdx.x;
-    const int nfull = (int)(gridDim.x / 8u) * 8;
-    if (bid < nfull) bid = (bid % 8) * (nfull / 8) + bid / 8;
-    adjoint_tile<DIR, P, LIM>(a, bid, lds);
+    adjoint_tile<DIR, P, LIM>(a, (int)xcd_order(), lds);
 }
 
 // Adjoint sweep over a block list (independent instances): as k_sweep_list, a

@@ -415,9 +415,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) void k_
     // XCD-aware order: workgroup i runs on XCD i % 8, so each XCD gets a
     // contiguous range of the stream; neighbouring pencil groups of a y or z
     // sweep, which share cache lines, then share an L2
-    int bid = blockIdx.x;
-    const int nfull = (int)(gridDim.x / 8u) * 8;
-    if (bid < nfull) bid = (bid % 8) * (nfull / 8) + bid / 8;
+    const int bid = (int)pk::xcd_order();
     const int L = a.n[DIR] + 8;
     const int g0 = (int)((long long)bid * ngroups / gridDim.x), g1 = (int)((long long)(bid + 1) * ngroups / gridDim.x);
     stream_range<DIR, P, LIM, TP>(a, g0 * L, (g1 - g0) * L, blockIdx.x, AK, U);
