@@ -82,6 +82,73 @@ def test_list_items_bit_exact(oracle, shapes, lanes, ts):
     pk.finalize()
 
 
+# Pencils of two blocks, in stream items of one pencil group each: a group is a
+# pencil along x and eight along y and z.
+STREAM_LISTS = {2900: ((44, 41), (33, 33)), 4300: ((60, 45), (40, 40)), 5700: ((75, 48), (50, 42))}
+
+
+@pytest.mark.parametrize("items", sorted(STREAM_LISTS))
+@pytest.mark.parametrize("d", [0, 1, 2])
+def test_stream_ranges_of_several_items_bit_exact(oracle, d, items):
+    """More items than workgroups the device holds (2048 at two waves per SIMD,
+    3072 at three, 4096 at four), by less than half: the launch has one round of
+    workgroups, whose ranges hold one or two items, join items of a block, and
+    cross from one block to the next."""
+    cfg = setups.batch_config(fluids=((5.0 / 3.0, True), (1.4, False)))
+    shapes = []
+    for (a, b), length in zip(STREAM_LISTS[items], (125, 121) if d == 0 else (5, 7)):
+        n = [a, b] if d == 0 else [4 * a, 2 * b]
+        n.insert(d, length)
+        shapes.append(tuple(n))
+    shapes.append((4, 4, 4))
+    print(f"stream list of {items} items along {'xyz'[d]}: {shapes}", flush=True)
+    cgs = setups.batch_blocks(shapes, cfg, seed=5)
+    obs = [oracle.OBlock.from_cg(c) for c in cgs]
+    pk.load_library()
+    pk.finalize()
+    pk.init(cfg)
+    for cg in cgs:
+        cg.registered = False
+        cg.upload()
+    for f in range(2):
+        pk.set_list_tiles(d, f, 64, -2)
+    t_g, _ = pk.run_all(1)
+    assert t_g == oracle.run_list(oracle.params_from_config(cfg), obs, 1)
+    for cg, ob in zip(cgs, obs):
+        cg.download()
+        assert_same(cg, ob, f"list {cg.n}")
+    pk.finalize()
+
+
+def test_list_of_several_launches():
+    """More tiles than one launch takes (2^22): one cell and 14 pencils a tile
+    against the default tiles, the same bits."""
+    torch = pytest.importorskip("torch")
+    n = 400
+    print(f"list of {n}^3 cells in tiles of 14", flush=True)
+    cfg = pk.Config(limiter="vanleer", gamma=1.4)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    u = torch.empty((n + 8, n + 8, n + 8, 5), dtype=torch.float64, device="cuda")
+    u.uniform_(-0.3, 0.3, generator=gen)
+    u[..., 0] += 1.0
+    u[..., 4] += 3.0
+    out = []
+    for ts in (0, 9):
+        pk.load_library()
+        pk.finalize()
+        pk.init(cfg)
+        cg = setups._DeviceBlock((n, n, n), 4, cfg, 1)
+        cg.upload_device(u)
+        if ts:
+            for d in range(3):
+                pk.set_list_tiles(d, 0, 128, ts)
+        pk.run_all(1)
+        out.append(torch.empty_like(u))
+        cg.download_device(out[-1])
+        pk.finalize()
+    assert torch.equal(out[0], out[1]) and bool(torch.isfinite(out[0]).all())
+
+
 @pytest.mark.parametrize("n", [(12, 9, 8), (5, 4, 33)])
 def test_step_reads_the_ghosts_it_is_given(n):
     """A single step from ghosts that are not periodic images: its first sweep
