@@ -206,6 +206,26 @@ def test_hllc_vjp_mirror_state_averages_the_two_sides(hm):
         assert close(np.concatenate([lb, rb]), g, 1e-6)
 
 
+def test_hllc_vjp_contact_at_rest(hm):
+    """Isobaric gas at rest normal to the interface, different densities and
+    transverse velocities: the contact speed is exactly 0 and both sides
+    contribute, each with its own sound speed and star state."""
+    rng = np.random.default_rng(9)
+    for _ in range(50):
+        l, r = random_face(rng), random_face(rng)
+        l[1] = r[1] = 0.0
+        r[4] = l[4]
+        if abs(GAM * l[4] / l[0] - GAM * r[4] / r[0]) < 1e-3:
+            continue
+        assert speeds(l, r)[2] == 0.0
+        fb = rng.normal(0, 1, 5)
+        lb, rb = np.zeros(5), np.zeros(5)
+        hm.hm_hllc_vjp(dp(l), dp(r), GAM, dp(fb), dp(lb), dp(rb))
+        # across the kinks (sm = 0, equal normal velocities) a central difference errs by O(h)
+        g = fd_vjp(lambda y: hllc(hm, y[:5], y[5:]), np.concatenate([l, r]), fb, rel=1e-7)
+        assert close(np.concatenate([lb, rb]), g, 1e-6), (l, r, lb, rb, g)
+
+
 @pytest.mark.parametrize("case", ["none", "density", "energy", "both"])
 def test_floors_vjp(hm, case):
     rng = np.random.default_rng(11)
