@@ -242,7 +242,8 @@ int pk_fluid_update(int64_t cg_id, double dt);
 
 /* nsteps iterations of the main loop (piernik.F90:124-170) with
  * cflcontrol='warn': time_step, then fluid_update.  *t_out = simulated time,
- * *dt_out = the last dt. */
+ * *dt_out = the last dt.  The block's ghosts are refreshed on return, also
+ * where a step fails (dt below dt_min, a step redone too often). */
 int pk_run(int64_t cg_id, int32_t nsteps, double *t_out, double *dt_out);
 
 /* Floor bookkeeping of one block since the last reset. */
@@ -273,8 +274,9 @@ int pk_run_all(int32_t mode, int32_t nsteps, double *t_out, double *dt_out);
  * and GLM damping), all advanced by the same launches as the list
  * entry points.  Arrays below have one entry per block in that order. */
 int pk_ensemble_ids(int64_t *ids, int32_t n);
-/* One main-loop iteration of every block; first != 0: no growth cap (the
- * first step of a run).  dt_out, capped_out (may be NULL): each block's dt
+/* One main-loop iteration of every block, taken as periodic whatever its
+ * ghosts hold (pk_ensemble_record_step reads the ghosts as they are at its
+ * first sweep); first != 0: no growth cap (the first step of a run).  dt_out, capped_out (may be NULL): each block's dt
  * and whether dt_max_grow capped it. */
 int pk_ensemble_step(int32_t mode, int32_t first, double *dt_out, int32_t *capped_out);
 int pk_ensemble_run(int32_t mode, int32_t nsteps, double *t_out, double *dt_out);

@@ -152,13 +152,15 @@ __device__ __forceinline__ void prim_vjp(const AdjArgs &a, const double (&u)[P::
 // another lane.  U and the stage-1 primitives are formed again where they are
 // needed instead of being held across the flux VJPs.
 //
-// Bound by FP64 VALU issue (hydro: four waves per SIMD, each issuing 23-24 %
-// of its cycles; MHD: two waves at 31 %, the rest LDS and scratch waits).
+// Bound by FP64 VALU issue (hydro: four waves per SIMD, the VALU 86 - 90 %
+// busy at 128^3) and, for MHD, by waits (two waves per SIMD, the VALU 41 - 48 %
+// busy, half the waves' cycles at s_waitcnt for LDS and scratch).
 // Against both-sided flux VJPs with IEEE divisions, eight (hydro five) arrays
 // and tiles in launch order: VALU instructions per wave 3143 -> 2136 (hydro)
 // and 9508 -> 5000 (MHD), waves per SIMD 2 -> 4 and 1 -> 2; the list sweeps of
 // 20 Orszag-Tang instances (64^2 .. 256^2) 527 and 633 us -> 297 and 325 us
-// (x, y), a 96^3 hydro rollout with its gradient 7.18 -> 5.3-5.8 ms.  The
+// (x, y), a 96^3 hydro rollout with its gradient 7.18 -> 5.3-5.8 ms.  (The
+// special values of division cost 1.5 % of a gradient since.)  The
 // XCD-aware order is worth 1.4x of that rollout: in launch order the tiles of
 // one cache line of a y or z sweep ran on eight L2s (110e6 busy CU cycles per
 // y sweep against 49e6 along x; in XCD order 50e6).

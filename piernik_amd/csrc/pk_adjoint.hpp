@@ -13,7 +13,7 @@
 // speeds and their signs, the star-state tests, limiter cases, min/max
 // choices, floors) in the forward's order with the forward's bits (ndiv and
 // nsqrt: those of the exact division and square root for operands away from
-// the ends of the exponent range), and then runs the chain rule backwards
+// the ends of the exponent range, and their special values), and then runs the chain rule backwards
 // through the branch the forward took.  Quotients that only scale adjoints
 // are formed with one reciprocal per divisor: they differ from a division by
 // at most an ulp, far below the derivative's own truncation, and an IEEE
@@ -146,9 +146,13 @@ PK_HD void limit_vjp(int lim, double dl, double dr, double dqb, double &dlb, dou
 // side the contact speed points to -- and the average of the two sides when
 // sm == 0.  The reverse pass is written once, for side A = the selected side
 // and side O = the other one, with sg = +1 when A is the left side; the two
-// sides' formulas are mirror images.  In the averaged case O's own part runs
-// too, both with weight 1/2 (the pass is linear in the flux adjoint given the
-// branch).
+// sides' formulas are mirror images.  In the averaged case both sides count
+// with weight 1/2 (the pass is linear in the flux adjoint given the branch):
+// HLLC adds O's own part to A's and runs what they share (sm, the star
+// pressure, the wave speeds) once, HLLD runs its pass twice.  Isobaric gas at
+// rest averages at every interface: a 128^3 hydro reverse sweep along x, y, z
+// takes 222, 211, 209 us there and 229, 226, 225 in moving gas; with HLLC's
+// pass run twice, its first result in scratch memory, 345, 388, 390 at rest.
 
 // The flux of side A and its reverse, shared by both solvers: with
 // dn = q0*(s - q1) and ds = dn/(s - sm) the side's star flux F + s*(U* - U) is

@@ -51,7 +51,7 @@ struct Block {
     double *dtout = nullptr;                  // timestep results (4 per fluid), pinned host memory
     unsigned long long *d_dtslots = nullptr;  // timestep reduction written by the last sweep of a step
     bool dt_pending = false;                  // dtout holds timestep_fluid of the current state
-    bool ghosts_stale = false;                // stream sweeps read the periodic interior and left the ghosts old
+    bool ghosts_stale = false;                // sweeps read the periodic interior and left the ghosts old
     // reverse mode (pk_adjoint_setup): saved states and the adjoint state
     std::vector<double *> slots;
     std::vector<char> slot_stale;  // the slot's ghosts are old (periodic images of its interior replace them)
@@ -206,7 +206,7 @@ void list_touch();
 int settle_ghosts();
 
 // Every entry point that takes a block reads or replaces its state, so the
-// ghosts a list's stream sweeps left old are refilled first.
+// ghosts a list's sweeps left old are refilled first.
 int get_block(int64_t id, Block **b)
 {
     if (!g_init) return fail(PK_ESTATE, "pk_init has not been called");
@@ -1654,7 +1654,7 @@ int list_fill()
     return PK_OK;
 }
 
-// The ghosts the list's stream sweeps left old (every block of the list, as
+// The ghosts the list's sweeps left old (every block of the list, as
 // its sweeps read them), before anything reads them.
 int settle_ghosts()
 {

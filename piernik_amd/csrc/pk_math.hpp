@@ -126,8 +126,8 @@ PK_HD double nsqrt(double x)
 // uses the correctly rounded operations, as the reference does.  The reverse
 // mode (PK_NORMAL_RANGE) uses ndiv and nsqrt: the same bits as the exact
 // build wherever its expansions apply no range scaling (operands and
-// quotients well inside 2^-767 .. 2^767), in fewer instructions and with
-// one reciprocal for all quotients of a divisor.
+// quotients well inside 2^-767 .. 2^767), and its special values, in fewer
+// instructions and with one reciprocal for all quotients of a divisor.
 PK_HD double qdiv(double a, double b)
 {
 #if PK_RELAXED && defined(__HIP_DEVICE_COMPILE__)
