@@ -40,12 +40,10 @@ using pk::UnsplitArgs;
 
 namespace {
 
-// sweep-order variable k -> xyz plane (fluidtypes.F90:318-320, fluidindex.F90:190-192)
+// plane_of for a direction that is a loop's variable
 __device__ __forceinline__ int uplane(int dir, int k)
 {
-    if (dir == 0 || k == 0 || k == 4 || k == 8) return k;
-    if (dir == 1) return (k == 1 || k == 2) ? 3 - k : ((k == 5 || k == 6) ? 11 - k : k);
-    return (k == 1 || k == 3) ? 4 - k : ((k == 5 || k == 7) ? 12 - k : k);
+    return dir == 0 ? plane_of<0>(k) : (dir == 1 ? plane_of<1>(k) : plane_of<2>(k));
 }
 
 // Tile of TP pencils x TS cells along DIR, lanes x fastest.  The lane of
@@ -110,7 +108,7 @@ __global__ __launch_bounds__(256) void k_unsplit_flux_tile(const UnsplitArgs a, 
 
     double W[NV], q[NV];
 #pragma unroll
-    for (int k = 0; k < NV; k++) W[k] = a.src[(long long)uplane(DIR, k) * a.sv + idx];
+    for (int k = 0; k < NV; k++) W[k] = a.src[(long long)plane_of<DIR>(k) * a.sv + idx];
     prim<P>(W, a.gam_1, q);
     lds_put<NV>(A, t, q);
     __syncthreads();
@@ -141,7 +139,7 @@ __global__ __launch_bounds__(256) void k_unsplit_flux_tile(const UnsplitArgs a, 
     const long long st = (DIR == 0) ? 1ll : ((DIR == 1) ? (long long)a.sy : (long long)a.sz);
     const long long row = idx + st;
 #pragma unroll
-    for (int k = 0; k < NV; k++) F[(long long)uplane(DIR, k) * a.sv + row] = f[k];
+    for (int k = 0; k < NV; k++) F[(long long)plane_of<DIR>(k) * a.sv + row] = f[k];
 }
 
 // Flux along DIR and its difference in one tile (dst != src).  The tile
@@ -217,7 +215,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
 
     double W[NV], q[NV];
 #pragma unroll
-    for (int k = 0; k < NV; k++) W[k] = a.src[(long long)uplane(DIR, k) * a.sv + idx];
+    for (int k = 0; k < NV; k++) W[k] = a.src[(long long)plane_of<DIR>(k) * a.sv + idx];
     if constexpr (P::MAG) W[8] = W[8] * a.src_fac;
     prim<P>(W, a.gam_1, q);
     lds_put<NV>(A, t, q);
@@ -271,7 +269,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3))) void k
         lds_get<NV>(A, tm, fl);
 #pragma unroll
         for (int k = 0; k < NV; k++) {
-            const int v = uplane(DIR, k);
+            const int v = plane_of<DIR>(k);
             T[v] = T[v] + coef * (fl[k] - f[k]);
         }
         if (last) {
